@@ -160,13 +160,12 @@ __global__ void __launch_bounds__(256) qk_norm_rope_kernel(const T* q, const T* 
   }
 }
 
-// The fast path for whole-chunk heads with every value turning: one wave per
+// The fast path for whole-chunk heads: one wave per
 // (token, group of 64 / G heads), each in a one-wave block, G lanes per head,
 // each lane holding two chunks of its head (NeoX: a chunk and its partner;
 // otherwise chunks i and i + G). The waves are independent: no block barrier.
 // A wave issues its loads first; while they land it makes its token's cos and
 // sin (a pair a lane, the double sin and cos of sincos.hpp) in its own LDS.
-// Heads with mRoPE sections (a position per section) take the general kernel.
 //
 // Measured on MI355X at Q [4096,32,128], K [4096,8,128] bf16 (kernel-trace
 // medians), against the designs it replaced: a block of five waves per token
@@ -204,7 +203,10 @@ __device__ __forceinline__ int qk_pair_slot(int pair) {
 // nothing and sets *bad_page.
 //
 // Key heads per value tile: as many as keep the staged tile within 4 KiB of
-// values (one head of 128).
+// values (one head of 128). A head of more is tiled as whole parts of 128 (the
+// values and the cache both hold a head's parts as they would hold heads of
+// 128): a whole head of 256 staged 9 KiB, which held 17 one-wave blocks a CU.
+constexpr int kTileWidth(int dim) { return dim > 128 ? 128 : dim; }
 constexpr int kTileHeads(int dim) { return dim * 32 >= 4096 ? 1 : 4096 / (dim * 32); }
 
 __device__ __forceinline__ int tile_dword(int value, int position) { return value * 8 + (value / 8) * 8 + position / 2; }
@@ -297,6 +299,21 @@ __device__ __attribute__((noinline)) double2 sincos_far(float angle) {
   return make_double2(cn, sn);
 }
 
+// MIXED: heads of which only the first `rotary` values turn, or whose pairs
+// turn by sections (mRoPE, axes), or both. With R chunk pairs turning, NeoX
+// lane i0 < R holds chunks i0 and i0 + R, and lane i0 >= R two of the tail's
+// (i0 + R and i0 + G), so a head's chunks still lie on all G lanes and every
+// load covers whole lines; interleaved lanes hold i0 and i0 + G as ever. Tail
+// chunks are normed and not turned (a turn by cos 1, sin 0 would make an
+// infinite partner NaN). A pair's position comes from its section's row.
+// Memory sets its pace: a gated query of 16 heads of 256 with 2 key heads, 64
+// values turning by interleaved sections, 4,096 tokens with the cache (150 MB)
+// takes 28.9 us, 5.2 TB/s, in graph replays; the general kernel, which reads
+// values one by one and holds a block's barriers twice for every four heads,
+// took 137. The gate leaves by non-temporal stores (28 heads of 128 24.9 ->
+// 24.2 us, 16 of 64 25.3 -> 24.4, 16 of 256 even); storing it before the norm
+// to free its registers (74 -> 66) was even or slower.
+//
 // FAST: every wave's heads are all queries or all keys (so the choice of
 // tensor, and its addresses' base, is the wave's, not each lane's) and the
 // weight offset is 0 (the identity addition is left out: the two forms of
@@ -307,7 +324,7 @@ __device__ __attribute__((noinline)) double2 sincos_far(float angle) {
 // 2% faster than one group a wave, at 95 registers against 64; a pass loop
 // loading one group ahead was 5% slower, four groups a wave 30% slower, and
 // with the cache two groups were slower than one.
-template <typename T, int G, bool NEOX, bool EXTRAS, bool GATE, bool FAST, int P>
+template <typename T, int G, bool NEOX, bool EXTRAS, bool GATE, bool FAST, int P, bool MIXED>
 __device__ __forceinline__ void qk_wave_heads(const T* q, const T* k, T* q_out, T* k_out, const float* q_weight,
                                               const float* k_weight, const int32_t* positions, const QkArgs& a,
                                               const Extras<T>& e, int64_t t, int group, double2* cs) {
@@ -315,12 +332,22 @@ __device__ __forceinline__ void qk_wave_heads(const T* q, const T* k, T* q_out, 
   constexpr int N = Chunk<T>::N;
   using Raw = typename Chunk<T>::Raw;
   constexpr int kHeadsPerPass = kWave / G;
-  constexpr int dim = 2 * N * G, half = N * G;  // a head's pairs: half (rotary == dim)
+  constexpr int dim = 2 * N * G, kHalf = N * G;  // a head's pairs: kHalf where every value turns
   const RopeArgs& p = a.rope;
+  const int half = MIXED ? p.rotary / 2 : kHalf;
   const int lane = threadIdx.x;
   const int rows = a.q_heads + a.kv_heads;
   const int i0 = lane % G;
-  const int d0 = i0 * N, d1 = (NEOX ? half : G * N) + i0 * N;
+  int d0 = i0 * N, d1 = kHalf + i0 * N;
+  bool turns0 = true, turns1 = true;  // the chunks turn
+  if constexpr (MIXED && NEOX) {
+    turns0 = turns1 = d0 < half;
+    d1 = turns0 ? d0 + half : d1;
+    d0 = turns0 ? d0 : d0 + half;
+  } else if constexpr (MIXED) {
+    turns0 = d0 < p.rotary;
+    turns1 = d1 < p.rotary;
+  }
   const int first = group * kHeadsPerPass * P;  // the wave's first head
   const int h = first + lane / G;
   const bool live = h < rows;
@@ -332,11 +359,16 @@ __device__ __forceinline__ void qk_wave_heads(const T* q, const T* k, T* q_out, 
   // it (loads are never branched around). Measured at the C3 shape, against
   // weights staged as doubles in LDS, a position read per lane and a branch
   // for irregular sums: each of those cost about 1 us.
-  constexpr int kPairsPerLane = (half + kWave - 1) / kWave;
-  const int32_t position = positions[t];  // single-section rope: one position a token
+  constexpr int kPairsPerLane = (kHalf + kWave - 1) / kWave;
+  int32_t position[MIXED ? kPairsPerLane : 1];
+  if constexpr (!MIXED) position[0] = positions[t];  // single-section rope: one position a token
   float inverse[kPairsPerLane];
 #pragma unroll
-  for (int u = 0; u < kPairsPerLane; ++u) inverse[u] = p.inverse[min(lane + u * kWave, half - 1)];
+  for (int u = 0; u < kPairsPerLane; ++u) {
+    const int j = min(lane + u * kWave, half - 1);
+    inverse[u] = p.inverse[j];
+    if constexpr (MIXED) position[u] = positions[(int64_t)rope_section(j, p) * p.tokens + t];
+  }
   const int hc = min(h, rows - 1);
   const bool query_c = FAST ? query : hc < a.q_heads;
   const float* ws = query_c ? q_weight : k_weight;
@@ -386,7 +418,7 @@ __device__ __forceinline__ void qk_wave_heads(const T* q, const T* k, T* q_out, 
   for (int u = 0; u < kPairsPerLane; ++u) {
     const int j = lane + u * kWave;
     if (j < half) {
-      const float angle = (float)position * inverse[u];
+      const float angle = (float)position[MIXED ? u : 0] * inverse[u];
       double sn, cn;
       if (!sincos_reduced(angle, &sn, &cn)) {
         const double2 far = sincos_far(angle);
@@ -431,17 +463,27 @@ __device__ __forceinline__ void qk_wave_heads(const T* q, const T* k, T* q_out, 
       }
     }
     if constexpr (NEOX) {
+      if (turns0) {
 #pragma unroll
-      for (int i = 0; i < N; ++i) {
-        const double2 c = cs[qk_pair_slot<NEOX, G, N>(d0 + i)];
-        turn_fused(v0[i], v1[i], c.x, c.y, v0[i], v1[i]);
+        for (int i = 0; i < N; ++i) {
+          const double2 c = cs[qk_pair_slot<NEOX, G, N>(d0 + i)];
+          turn_fused(v0[i], v1[i], c.x, c.y, v0[i], v1[i]);
+        }
       }
     } else {
+      if (turns0) {
 #pragma unroll
-      for (int i = 0; i < N; i += 2) {
-        const double2 c0 = cs[(d0 + i) / 2], c1 = cs[(d1 + i) / 2];
-        turn_fused(v0[i], v0[i + 1], c0.x, c0.y, v0[i], v0[i + 1]);
-        turn_fused(v1[i], v1[i + 1], c1.x, c1.y, v1[i], v1[i + 1]);
+        for (int i = 0; i < N; i += 2) {
+          const double2 c = cs[(d0 + i) / 2];
+          turn_fused(v0[i], v0[i + 1], c.x, c.y, v0[i], v0[i + 1]);
+        }
+      }
+      if (turns1) {
+#pragma unroll
+        for (int i = 0; i < N; i += 2) {
+          const double2 c = cs[(d1 + i) / 2];
+          turn_fused(v1[i], v1[i + 1], c.x, c.y, v1[i], v1[i + 1]);
+        }
       }
     }
     if (!EXTRAS || query || !e.keys) {
@@ -452,8 +494,8 @@ __device__ __forceinline__ void qk_wave_heads(const T* q, const T* k, T* q_out, 
     if constexpr (EXTRAS) {
       if (GATE && query) {
         T* gh = e.gate + (t * a.q_heads + hh) * dim;
-        *reinterpret_cast<uint4*>(gh + d0) = g0;
-        *reinterpret_cast<uint4*>(gh + d1) = g1;
+        __builtin_nontemporal_store(u32x4{g0.x, g0.y, g0.z, g0.w}, reinterpret_cast<u32x4*>(gh + d0));
+        __builtin_nontemporal_store(u32x4{g1.x, g1.y, g1.z, g1.w}, reinterpret_cast<u32x4*>(gh + d1));
       }
       int64_t key;
       if (!query && e.keys && key_place(e, page, in_page, a.kv_heads, dim, hh - a.q_heads, key)) {
@@ -473,7 +515,7 @@ __device__ __forceinline__ void qk_wave_heads(const T* q, const T* k, T* q_out, 
   }
 }
 
-template <typename T, int G, bool NEOX, bool EXTRAS, bool GATE, bool FAST, int P>
+template <typename T, int G, bool NEOX, bool EXTRAS, bool GATE, bool FAST, int P, bool MIXED>
 __global__ void __launch_bounds__(kWave) qk_norm_rope_wave(const T* q, const T* k, T* q_out, T* k_out,
                                                           const float* q_weight, const float* k_weight,
                                                           const int32_t* positions, QkArgs a, Extras<T> e,
@@ -484,7 +526,8 @@ __global__ void __launch_bounds__(kWave) qk_norm_rope_wave(const T* q, const T* 
   // one LDS buffer for the token's angles or, in a tile block, the staged
   // tile (a block uses one of them; two buffers would hold fewer blocks)
   constexpr int kAngleWords = N * G * 4;  // double2 per pair
-  constexpr int kWords = EXTRAS && kTileWords(dim) > kAngleWords ? kTileWords(dim) : kAngleWords;
+  constexpr int kTileDim = kTileWidth(dim);
+  constexpr int kWords = EXTRAS && kTileWords(kTileDim) > kAngleWords ? kTileWords(kTileDim) : kAngleWords;
   __shared__ __align__(16) uint32_t lds[kWords];
   int64_t item = blockIdx.x;
   if constexpr (EXTRAS) {
@@ -492,7 +535,7 @@ __global__ void __launch_bounds__(kWave) qk_norm_rope_wave(const T* q, const T* 
     // Measured at the C3 shape with the cache (4,096 tokens, 2,048 tiles):
     // tiles first 20.6 us, interleaved evenly 21.8 us, last 21.6 us.
     if (item < e.tiles) {
-      cache_values_tile<T, dim>(e, p.tokens, a.kv_heads, item, lds);
+      cache_values_tile<T, kTileDim>(e, p.tokens, a.kv_heads * (dim / kTileDim), item, lds);
       return;
     }
     item -= e.tiles;
@@ -519,8 +562,8 @@ __global__ void __launch_bounds__(kWave) qk_norm_rope_wave(const T* q, const T* 
   }
   const int64_t t = token;
   const int group = (int)group_u;
-  qk_wave_heads<T, G, NEOX, EXTRAS, GATE, FAST, P>(q, k, q_out, k_out, q_weight, k_weight, positions, a, e, t, group,
-                                                reinterpret_cast<double2*>(lds));
+  qk_wave_heads<T, G, NEOX, EXTRAS, GATE, FAST, P, MIXED>(q, k, q_out, k_out, q_weight, k_weight, positions, a, e, t, group,
+                                                       reinterpret_cast<double2*>(lds));
 }
 
 // ------------------------------------------------------------------ cache write, split halves
@@ -607,8 +650,12 @@ int qk_launch(const char* entry, const T* q, const T* k, T* q_out, T* k_out, con
   constexpr int N = Chunk<T>::N;
   const int dim = p.dim;
   const int lanes_per_head = dim / (2 * N);
-  const bool whole = p.rotary == dim && dim % (2 * N) == 0 && (lanes_per_head & (lanes_per_head - 1)) == 0 &&
-                     lanes_per_head <= kWave / 2 && aligned && p.sections == DRIFT_SECTIONS_SINGLE;
+  // partial rotary and sections take the MIXED body, where whole chunks turn
+  // (F32 rotary of a multiple of 8, BF16 of 16, NeoX; half that interleaved);
+  // the general kernel keeps the rest
+  const bool mixed = p.rotary != dim || p.sections != DRIFT_SECTIONS_SINGLE;
+  const bool whole = p.rotary > 0 && p.rotary % (p.layout == DRIFT_ROPE_NEOX ? 2 * N : N) == 0 && dim % (2 * N) == 0 &&
+                     (lanes_per_head & (lanes_per_head - 1)) == 0 && lanes_per_head <= kWave / 2 && aligned;
   if (!whole) {
     hipLaunchKernelGGL((qk_norm_rope_kernel<T, EXTRAS>), dim3(grid_for(p.tokens, 1, 1 << 16)), dim3(256), 0, st, q,
                        k, q_out, k_out, q_weight, k_weight, positions, a, e);
@@ -619,7 +666,7 @@ int qk_launch(const char* entry, const T* q, const T* k, T* q_out, T* k_out, con
   const int heads_per_wave = kWave / lanes_per_head;
   // the fast body: query heads fill whole waves and the weight offset is 0;
   // two passes a wave where the query heads fill whole pairs of waves
-  const bool fast = a.q_heads % heads_per_wave == 0 && a.offset == 0.0f;
+  const bool fast = a.q_heads % heads_per_wave == 0 && a.offset == 0.0f && !mixed;
   const int passes = fast && !EXTRAS && a.q_heads % (2 * heads_per_wave) == 0 ? 2 : 1;
   const int waves_per_token = (int)ceil_div(a.q_heads + a.kv_heads, heads_per_wave * passes);
   // with the fast body a wave's heads are all queries or all keys, and the
@@ -628,23 +675,26 @@ int qk_launch(const char* entry, const T* q, const T* k, T* q_out, T* k_out, con
   const int query_waves = fast && a.kv_heads > 0 ? a.q_heads / (heads_per_wave * passes) : waves_per_token;
   const bool keys_first = EXTRAS && e.keys != nullptr;
   Extras<T> ex = e;
-  const int tile_heads = kTileHeads(dim);
+  const int tile_heads = kTileHeads(kTileWidth(dim));
   ex.tiles = EXTRAS && e.keys ? ((int64_t)(e.start + p.tokens - 1) / 16 - e.start / 16 + 1) *
-                                    ((a.kv_heads + tile_heads - 1) / tile_heads)
+                                    ceil_div((int64_t)a.kv_heads * (dim / kTileWidth(dim)), tile_heads)
                               : 0;
   const int64_t blocks = (int64_t)p.tokens * waves_per_token + ex.tiles;
   if (blocks > INT32_MAX) return refuse("%s: %d tokens of %d heads", entry, p.tokens, a.q_heads + a.kv_heads);
   const dim3 grid((unsigned)blocks), block(kWave);
   switch (lanes_per_head) {
 #define DRIFT_QK_LAUNCH(G, NEOX, GATE)                                                                               \
-  if (passes == 2)                                                                                                   \
-    hipLaunchKernelGGL((qk_norm_rope_wave<T, G, NEOX, EXTRAS, GATE, true, EXTRAS ? 1 : 2>), grid, block, 0, st, q,  \
+  if (mixed)                                                                                                         \
+    hipLaunchKernelGGL((qk_norm_rope_wave<T, G, NEOX, EXTRAS, GATE, false, 1, true>), grid, block, 0, st, q, k,     \
+                       q_out, k_out, q_weight, k_weight, positions, a, ex, waves_per_token, query_waves, keys_first);\
+  else if (passes == 2)                                                                                              \
+    hipLaunchKernelGGL((qk_norm_rope_wave<T, G, NEOX, EXTRAS, GATE, true, EXTRAS ? 1 : 2, false>), grid, block, 0, st, q, \
                        k, q_out, k_out, q_weight, k_weight, positions, a, ex, waves_per_token, query_waves, keys_first);\
   else if (fast)                                                                                                     \
-    hipLaunchKernelGGL((qk_norm_rope_wave<T, G, NEOX, EXTRAS, GATE, true, 1>), grid, block, 0, st, q, k, q_out,     \
+    hipLaunchKernelGGL((qk_norm_rope_wave<T, G, NEOX, EXTRAS, GATE, true, 1, false>), grid, block, 0, st, q, k, q_out, \
                        k_out, q_weight, k_weight, positions, a, ex, waves_per_token, query_waves, keys_first);      \
   else                                                                                                               \
-    hipLaunchKernelGGL((qk_norm_rope_wave<T, G, NEOX, EXTRAS, GATE, false, 1>), grid, block, 0, st, q, k, q_out,    \
+    hipLaunchKernelGGL((qk_norm_rope_wave<T, G, NEOX, EXTRAS, GATE, false, 1, false>), grid, block, 0, st, q, k, q_out, \
                        k_out, q_weight, k_weight, positions, a, ex, waves_per_token, query_waves, keys_first)
 #define DRIFT_QK_CASE(G)                                                                                             \
   case G:                                                                                                            \

@@ -252,3 +252,32 @@ def test_attention_inputs_with_weights_off_a_16_byte_boundary(hip, dtype, gated)
     pages = -(-(start + t) // PAGE) + 1
     table = np.random.default_rng(9).permutation(pages).astype(np.int32)
     run_attention_inputs(hip, dtype, t, 32, 8, 128, QWEN3_ROPE, start, table, pages, gated, 170, weight_shift=1)
+
+
+# partial rotary and sections: (heads, kv, dim, rotary, layout, sections,
+# gated); a tail of no, one and most chunks, a rotary of
+# whole 4-value chunks only (F32's chunks, not BF16's), heads of two value
+# tiles and of four, a last wave part full, key heads alone in it
+MIXED = [
+    (16, 2, 256, 64, 0, d.RopeSections.Interleaved(11, 11, 10), True),
+    (24, 4, 256, 64, 0, d.RopeSections.Single(), True),
+    (28, 4, 128, 128, 0, d.RopeSections.Contiguous(16, 24, 24), False),
+    (32, 3, 128, 64, 0, d.RopeSections.Axes((8, 12, 12)), False),
+    (5, 1, 64, 16, 0, d.RopeSections.Single(), True),
+    (3, 2, 512, 496, 0, d.RopeSections.Interleaved(90, 80, 78), False),
+    (6, 2, 128, 16, 0, d.RopeSections.Single(), True),
+    (7, 3, 32, 8, 0, d.RopeSections.Contiguous(2, 1, 1), False),
+    (9, 2, 128, 40, 1, d.RopeSections.Interleaved(8, 6, 6), True),
+    (4, 4, 64, 12, 1, d.RopeSections.Single(), False),
+]
+
+
+@pytest.mark.parametrize("dtype", ["f32", "bf16"])
+@pytest.mark.parametrize("heads,kv,dim,rotary,layout,sections,gated", MIXED)
+def test_attention_inputs_partial_rotary_and_sections(hip, dtype, heads, kv, dim, rotary, layout, sections, gated):
+    t, start = 35, 6
+    step(f"attentionInputs {dtype} heads {heads}/{kv} of {dim}, rotary {rotary}, layout {layout}, {sections}")
+    pages = -(-(start + t) // PAGE) + 1
+    table = np.random.default_rng(heads).permutation(pages).astype(np.int32)
+    rope = d.Rope(1e6, rotary, d.RopeLayout(layout), sections)
+    run_attention_inputs(hip, dtype, t, heads, kv, dim, rope, start, table, pages, gated, 200 + heads, offset=1.0)
