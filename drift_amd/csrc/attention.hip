@@ -640,8 +640,8 @@ __global__ void __launch_bounds__(256) split_halves_values(const T* x, T* first,
 // ------------------------------------------------------------------ launch layer
 
 // Picks the kernel for a checked call: the per-lane-chunk one where heads
-// are whole 16-byte chunks with every value turning (and the tensors allow
-// 16-byte access), else the LDS one.
+// are whole 16-byte chunks that turn whole or not at all (and the tensors
+// allow 16-byte access), else the LDS one.
 template <typename T, bool EXTRAS>
 int qk_launch(const char* entry, const T* q, const T* k, T* q_out, T* k_out, const float* q_weight,
               const float* k_weight, const int32_t* positions, const QkArgs& a, const Extras<T>& e, bool aligned,
@@ -650,37 +650,37 @@ int qk_launch(const char* entry, const T* q, const T* k, T* q_out, T* k_out, con
   constexpr int N = Chunk<T>::N;
   const int dim = p.dim;
   const int lanes_per_head = dim / (2 * N);
+  const int heads_per_wave = lanes_per_head > 0 ? kWave / lanes_per_head : 1;
   // partial rotary and sections take the MIXED body, where whole chunks turn
-  // (F32 rotary of a multiple of 8, BF16 of 16, NeoX; half that interleaved);
-  // the general kernel keeps the rest
+  // (F32 rotary of a multiple of 8, BF16 of 16, NeoX; half that interleaved)
   const bool mixed = p.rotary != dim || p.sections != DRIFT_SECTIONS_SINGLE;
-  const bool whole = p.rotary > 0 && p.rotary % (p.layout == DRIFT_ROPE_NEOX ? 2 * N : N) == 0 && dim % (2 * N) == 0 &&
-                     (lanes_per_head & (lanes_per_head - 1)) == 0 && lanes_per_head <= kWave / 2 && aligned;
-  if (!whole) {
-    hipLaunchKernelGGL((qk_norm_rope_kernel<T, EXTRAS>), dim3(grid_for(p.tokens, 1, 1 << 16)), dim3(256), 0, st, q,
-                       k, q_out, k_out, q_weight, k_weight, positions, a, e);
-    return launched(entry);
-  }
-  // a one-wave block per (token, group of 64 / G heads); with the cache,
-  // blocks before those write the values by tiles of 16 positions
-  const int heads_per_wave = kWave / lanes_per_head;
   // the fast body: query heads fill whole waves and the weight offset is 0;
   // two passes a wave where the query heads fill whole pairs of waves
   const bool fast = a.q_heads % heads_per_wave == 0 && a.offset == 0.0f && !mixed;
   const int passes = fast && !EXTRAS && a.q_heads % (2 * heads_per_wave) == 0 ? 2 : 1;
   const int waves_per_token = (int)ceil_div(a.q_heads + a.kv_heads, heads_per_wave * passes);
-  // with the fast body a wave's heads are all queries or all keys, and the
-  // grid runs the query waves and the key waves apart (the key waves first
-  // when they write the cache, last otherwise); else token by token
-  const int query_waves = fast && a.kv_heads > 0 ? a.q_heads / (heads_per_wave * passes) : waves_per_token;
-  const bool keys_first = EXTRAS && e.keys != nullptr;
   Extras<T> ex = e;
   const int tile_heads = kTileHeads(kTileWidth(dim));
   ex.tiles = EXTRAS && e.keys ? ((int64_t)(e.start + p.tokens - 1) / 16 - e.start / 16 + 1) *
                                     ceil_div((int64_t)a.kv_heads * (dim / kTileWidth(dim)), tile_heads)
                               : 0;
   const int64_t blocks = (int64_t)p.tokens * waves_per_token + ex.tiles;
+  const bool whole = p.rotary > 0 && p.rotary % (p.layout == DRIFT_ROPE_NEOX ? 2 * N : N) == 0 && dim % (2 * N) == 0 &&
+                     (lanes_per_head & (lanes_per_head - 1)) == 0 && lanes_per_head <= kWave / 2 && aligned;
+  // the general kernel takes any number of tokens
+  if (!whole || (mixed && blocks > INT32_MAX)) {
+    hipLaunchKernelGGL((qk_norm_rope_kernel<T, EXTRAS>), dim3(grid_for(p.tokens, 1, 1 << 16)), dim3(256), 0, st, q,
+                       k, q_out, k_out, q_weight, k_weight, positions, a, e);
+    return launched(entry);
+  }
   if (blocks > INT32_MAX) return refuse("%s: %d tokens of %d heads", entry, p.tokens, a.q_heads + a.kv_heads);
+  // a one-wave block per (token, group of 64 / G heads); with the cache,
+  // blocks before those write the values by tiles of 16 positions. With the
+  // fast body a wave's heads are all queries or all keys, and the grid runs
+  // the query waves and the key waves apart (the key waves first when they
+  // write the cache, last otherwise); else token by token
+  const int query_waves = fast && a.kv_heads > 0 ? a.q_heads / (heads_per_wave * passes) : waves_per_token;
+  const bool keys_first = EXTRAS && e.keys != nullptr;
   const dim3 grid((unsigned)blocks), block(kWave);
   switch (lanes_per_head) {
 #define DRIFT_QK_LAUNCH(G, NEOX, GATE)                                                                               \

@@ -129,6 +129,82 @@ __global__ void __launch_bounds__(256) rope_table_kernel(const T* x, const float
   }
 }
 
+// Heads and rotating parts of whole 16-byte chunks: one-wave blocks, a wave
+// per run of K * 64 items of a token, an item a chunk (interleaved: its pairs
+// sit inside it) or a chunk and its partner (halves), as turn_chunks' items.
+// The loads are all issued before any turn and never branched around. The
+// products a*c of floats are exact in double, so the one fma is the
+// reference's a*c - b*s rounded once.
+//
+// Memory sets its pace: in place over [14040, 24, 128] bf16 with a table row a
+// token (172 MB, written just before by a norm) it takes 24.5 us, 7 TB/s; the
+// kernel above, two values a thread, took 68. An RMSNorm and this for
+// queries and keys there took 146.1, 136.7, 138.2 and 153.1 us with K = 1, 2,
+// 3 and 4; over 72 tokens (432 waves at K = 1) 10.4, 12.0, 13.6 and 14.6.
+template <typename T, int K, bool HALVES, bool PER_HEAD>
+__global__ void __launch_bounds__(kWave) rope_table_chunks(const T* x, const float* cosines, const float* sines,
+                                                           T* out, uint32_t runs, int heads, int dim, int pairs) {
+  constexpr int N = Chunk<T>::N;
+  constexpr int P = HALVES ? N : N / 2;  // pairs of an item
+  using Raw = typename Chunk<T>::Raw;
+  const uint32_t token = blockIdx.x / runs, run = blockIdx.x - token * runs;
+  const int rotating = HALVES ? pairs / N : 2 * pairs / N;  // a head's items that turn
+  const int slots = HALVES ? rotating + (dim - 2 * pairs) / N : dim / N;
+  const int items = heads * slots;
+  const T* xt = x + (int64_t)token * heads * dim;
+  T* ot = out + (int64_t)token * heads * dim;
+  Raw r0[K], r1[HALVES ? K : 1];
+  float c[K][P], s[K][P];
+  int at[K];
+  bool turns[K];
+#pragma unroll
+  for (int k = 0; k < K; ++k) {
+    const int item = min((int)(run * K + k) * kWave + (int)threadIdx.x, items - 1);
+    const int h = item / slots, j = item - h * slots;
+    turns[k] = j < rotating;
+    at[k] = h * dim + (HALVES && !turns[k] ? 2 * pairs + (j - rotating) * N : j * N);
+    r0[k] = Chunk<T>::load_raw(xt + at[k]);
+    if constexpr (HALVES) r1[k] = Chunk<T>::load_raw(xt + at[k] + (turns[k] ? pairs : 0));
+    const int64_t row = PER_HEAD ? (int64_t)token * heads + h : (int64_t)token;
+    const int64_t q = row * pairs + (turns[k] ? j * P : 0);
+    if (pairs > 0) {
+#pragma unroll
+      for (int i = 0; i < P; i += P >= 4 ? 4 : 2) {
+        if constexpr (P >= 4) {
+          const float4 a = *reinterpret_cast<const float4*>(cosines + q + i);
+          const float4 b = *reinterpret_cast<const float4*>(sines + q + i);
+          c[k][i] = a.x, c[k][i + 1] = a.y, c[k][i + 2] = a.z, c[k][i + 3] = a.w;
+          s[k][i] = b.x, s[k][i + 1] = b.y, s[k][i + 2] = b.z, s[k][i + 3] = b.w;
+        } else {
+          const float2 a = *reinterpret_cast<const float2*>(cosines + q + i);
+          const float2 b = *reinterpret_cast<const float2*>(sines + q + i);
+          c[k][i] = a.x, c[k][i + 1] = a.y;
+          s[k][i] = b.x, s[k][i + 1] = b.y;
+        }
+      }
+    }
+  }
+#pragma unroll
+  for (int k = 0; k < K; ++k) {
+    if ((int)(run * K + k) * kWave + (int)threadIdx.x >= items) return;
+    float a[N], b[N];
+    Chunk<T>::unpack(r0[k], a);
+    if constexpr (HALVES) Chunk<T>::unpack(r1[k], b);
+    if (turns[k]) {
+#pragma unroll
+      for (int i = 0; i < P; ++i) {
+        if constexpr (HALVES)
+          turn_fused(a[i], b[i], c[k][i], s[k][i], a[i], b[i]);
+        else
+          turn_fused(a[2 * i], a[2 * i + 1], c[k][i], s[k][i], a[2 * i], a[2 * i + 1]);
+      }
+    }
+    Chunk<T>::store(ot + at[k], a);
+    if constexpr (HALVES)
+      if (turns[k]) Chunk<T>::store(ot + at[k] + pairs, b);
+  }
+}
+
 // ------------------------------------------------------------------ Wan 3-D rope
 
 struct Rope3dArgs {
@@ -284,9 +360,38 @@ int rope_table(const char* entry, const T* x, const float* cosines, const float*
   if (pairs < 0 || 2 * pairs > dim) return refuse("%s: %d pairs in heads of %d", entry, pairs, dim);
   if ((int64_t)tokens * heads == 0) return 0;
   if (!x || !cosines || !sines || !out) return refuse("%s: null x, cosines, sines or out", entry);
-  const int64_t items = (int64_t)tokens * heads * ((dim + 1) / 2);
-  hipLaunchKernelGGL(rope_table_kernel<T>, dim3(grid_for(items, 256, 1 << 16)), dim3(256), 0, (hipStream_t)stream,
-                     x, cosines, sines, out, tokens, heads, dim, pairs, per_head ? 1 : 0, halves ? 1 : 0);
+  constexpr int N = Chunk<T>::N;
+  const hipStream_t st = (hipStream_t)stream;
+  const bool chunked = aligned16(x) && aligned16(out) && aligned16(cosines) && aligned16(sines) && dim % N == 0 &&
+                       (halves ? pairs % N == 0 : 2 * pairs % N == 0) && (int64_t)heads * dim <= INT32_MAX;
+  const int64_t items = heads * (halves ? (dim - pairs) / N : dim / N);
+  // a lane's items: one where they are chunk pairs, and in launches of at most
+  // 16 waves a CU of one; else two (rope_table_chunks' comment)
+  const int per_lane = halves || tokens * ceil_div(items, kWave) <= 4096 ? 1 : 2;
+  const int64_t runs = ceil_div(items, per_lane * kWave);
+  if (chunked && tokens * runs <= kOneShotBlocks) {
+    const dim3 grid((unsigned)(tokens * runs)), block(kWave);
+#define DRIFT_TABLE_LAUNCH(K, HALVES, PER_HEAD)                                                               \
+  hipLaunchKernelGGL((rope_table_chunks<T, K, HALVES, PER_HEAD>), grid, block, 0, st, x, cosines, sines, out, \
+                     (uint32_t)runs, heads, dim, pairs)
+    if (halves && per_head)
+      DRIFT_TABLE_LAUNCH(1, true, true);
+    else if (halves)
+      DRIFT_TABLE_LAUNCH(1, true, false);
+    else if (per_head && per_lane == 2)
+      DRIFT_TABLE_LAUNCH(2, false, true);
+    else if (per_head)
+      DRIFT_TABLE_LAUNCH(1, false, true);
+    else if (per_lane == 2)
+      DRIFT_TABLE_LAUNCH(2, false, false);
+    else
+      DRIFT_TABLE_LAUNCH(1, false, false);
+#undef DRIFT_TABLE_LAUNCH
+    return launched(entry);
+  }
+  const int64_t threads = (int64_t)tokens * heads * ((dim + 1) / 2);
+  hipLaunchKernelGGL(rope_table_kernel<T>, dim3(grid_for(threads, 256, 1 << 16)), dim3(256), 0, st, x, cosines, sines,
+                     out, tokens, heads, dim, pairs, per_head ? 1 : 0, halves ? 1 : 0);
   return launched(entry);
 }
 

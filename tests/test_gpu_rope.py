@@ -135,6 +135,32 @@ def test_rope_table(hip, halves, per_head, shape, pairs):
     assert_bf16(o.to_bf16(o.rope_table(o.from_bf16(xb), cos, sin, halves)), host_bits(outb), what="ropeTable bf16")
 
 
+@pytest.mark.parametrize("halves", [False, True])
+@pytest.mark.parametrize("per_head", [False, True])
+@pytest.mark.parametrize("shape,pairs,dtype", [
+    # whole chunks turning: part of a wave's items, a token's last wave part
+    # full, a copied tail, no tail, nothing turning but four pairs; enough
+    # tokens that a lane takes two items
+    ((3, 3, 72), 36, "bf16"), ((5, 9, 128), 48, "bf16"), ((4, 2, 64), 8, "bf16"), ((300, 24, 128), 64, "bf16"),
+    ((701, 13, 128), 32, "bf16"), ((7, 5, 8), 4, "f32"), ((300, 24, 72), 32, "f32"), ((1, 1, 256), 128, "f32"),
+])
+def test_rope_table_chunks(hip, halves, per_head, shape, pairs, dtype):
+    tokens, heads, dim = shape
+    step(f"ropeTable {dtype} {shape}, {pairs} pairs, per head {per_head}, halves {halves}")
+    x = gaussian(11, shape)
+    angles = gaussian(12, (tokens, heads, pairs) if per_head else (tokens, pairs), 3.0)
+    c, s = np.cos(angles), np.sin(angles)
+    if dtype == "bf16":
+        x = o.from_bf16(bf16_input(x))
+    dev = dev_f32(x) if dtype == "f32" else dev_bf16(o.to_bf16(x))
+    hip.ropeTable(dev, dev_f32(c), dev_f32(s), dev, halves)  # in place
+    want = o.rope_table(x, c, s, halves)
+    if dtype == "f32":
+        assert_f32(want, host_f32(dev), what="table")
+    else:
+        assert_bf16(o.to_bf16(want), host_bits(dev), what="table bf16")
+
+
 # tokens of 1 to 18 chunks a lane (bf16: 1 to 72 heads of 128), each
 # wave-per-token variant, and heads of 126 (not whole chunks)
 @pytest.mark.parametrize("grid,heads,dim,samples", [((3, 4, 5), 2, 128, 2), ((1, 1, 9), 3, 128, 1),
