@@ -62,8 +62,14 @@ template <int N>
 __device__ __forceinline__ double chunk_squares(const float (&v)[N]) {
   double p = 0.0;
 #pragma unroll
-  for (int j = 0; j < N; ++j) p += (double)v[j] * (double)v[j];
+  for (int j = 0; j < N; ++j) p = fma((double)v[j], (double)v[j], p);  // the square is exact
   return p;
+}
+
+// 1 / sqrt(squares / cols + eps), the same in every kernel here.
+__device__ __forceinline__ double rms_factor(double squares, int cols, float eps) {
+  const double mean = squares / (double)cols + (double)eps;
+  return eps > 0.0f ? inverse_sqrt<true>(mean) : inverse_sqrt(mean);
 }
 
 // With q.xq, out is quantized too as it is written (quantize_chunk; cols a
@@ -110,7 +116,7 @@ __global__ void __launch_bounds__(256) rms_norm_rows(T* x, const T* y, const flo
       }
     }
     squares = row_sum<W>(squares, partial);
-    const double factor = 1.0 / sqrt(squares / (double)cols + (double)eps);
+    const double factor = rms_factor(squares, cols, eps);
 #pragma unroll
     for (int k = 0; k < K; ++k) {
       const int c = (k * W + sub) * kWave + lane;
@@ -132,6 +138,149 @@ __global__ void __launch_bounds__(256) rms_norm_rows(T* x, const T* y, const flo
         }
       }
     }
+  }
+}
+
+// Many long rows, no side output and one weight row: a wave per row, in
+// one-wave blocks, so a row waits on no barrier; its sum is taken in the
+// four-wave group's order (chunk_squares): four sums over the wave, chunk k's
+// squares in sum k % 4. Loads are never branched around (chunks past the row
+// are clamped to its last and left out).
+//
+// Once a row a wave (RESIDENT false) the weights are read after the sum, from
+// the L1 (at 5120 values they are 20 KiB of it, and more registers hold fewer
+// waves); RESIDENT keeps them in registers over the rows a wave takes, with
+// the next row's loads in flight. Memory bounds it. Measured, us a launch in
+// graph replays, four-wave group / once a row / RESIDENT at a wave a SIMD:
+//   bf16 [4093, 4096] 15.8 / 12.6 / 13.5, with the residual 26.4 / 22.6 / 25.3
+//   F32 [2000, 2560] 11.8 / 7.6 / 8.3, with the residual 16.7 / 13.6 / 14.2
+//   F32 [2500, 5120] 22.9 / 17.9 / 20.1, with the residual 37.2 / 40.8 / 53.6
+//   bf16 [6000, 4096] 21.5 / 17.6 / 18.7, with the residual 36.4 / 39.0 / 36.4
+//   bf16 [14040, 3072] 39.0 / 33.2 / 31.4 (172 MB), with the residual 64.3 / 61.8 / 59.9
+//   bf16 [8000, 5120] 36.1 / 36.6 / 30.3, with the residual 61.1 / 60.9 / 59.3
+//   F32 [7800, 3072] 37.4 / 37.5 / 33.5, with the residual 65.2 / 70.8 / 67.8
+//   bf16 [1000, 4096] 5.3 / 5.4 / 4.8; F32 [509, 2560] 4.8 / 4.7 / 3.9; bf16 [300, 4096] 3.8 / 4.4 / 3.9,
+//   with the residual 5.0 / 6.1 / 6.0
+// Two waves a SIMD in the resident grid were 1 to 4% slower on the larger of
+// these, three and four up to 15%.
+template <typename T, int K, bool ADD, bool RESIDENT>
+__global__ void __launch_bounds__(kWave) rms_norm_waves(T* x, const T* y, const float* weight, T* out, int64_t rows,
+                                                        int cols, float eps, float offset) {
+  constexpr int N = Chunk<T>::N;
+  using Raw = typename Chunk<T>::Raw;
+  const int lane = threadIdx.x;
+  const int chunks = cols / N;
+  auto load_row = [&](int64_t r, Raw(&into)[K], Raw(&also)[ADD ? K : 1]) {
+#pragma unroll
+    for (int k = 0; k < K; ++k) {
+      const int c = min(k * kWave + lane, chunks - 1);
+      into[k] = Chunk<T>::load_raw(x + r * cols + c * N);
+      if constexpr (ADD) also[k] = Chunk<T>::load_raw(y + r * cols + c * N);
+    }
+  };
+  int64_t row = blockIdx.x;
+  Raw raw[K], add[ADD ? K : 1];
+  load_row(row, raw, add);
+  float w[RESIDENT ? K : 1][N];
+  if constexpr (RESIDENT) {
+#pragma unroll
+    for (int k = 0; k < K; ++k) load_f32<N>(weight + min(k * kWave + lane, chunks - 1) * N, w[k]);
+  }
+  // chunk k's values, with the residual the F32 sum as add() rounds it
+  auto values = [&](int k, float(&v)[N]) {
+    Chunk<T>::unpack(raw[k], v);
+    if constexpr (ADD) {
+      float u[N];
+      Chunk<T>::unpack(add[k], u);
+#pragma unroll
+      for (int j = 0; j < N; ++j) v[j] += u[j];
+    }
+  };
+  while (true) {
+    const int64_t following = row + gridDim.x;
+    Raw next[K], next_add[ADD ? K : 1];
+    if constexpr (RESIDENT)
+      if (following < rows) load_row(following, next, next_add);
+    constexpr int kSums = K < 4 ? K : 4;
+    double sums[4] = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+    for (int k = 0; k < K; ++k) {
+      float v[N];
+      values(k, v);
+      const double squares = chunk_squares(v);
+      sums[k % 4] += k * kWave + lane < chunks ? squares : 0.0;
+    }
+#pragma unroll
+    for (int i = 0; i < kSums; ++i) sums[i] = group_sum<64>(sums[i]);
+    const double factor = rms_factor(((sums[0] + sums[1]) + sums[2]) + sums[3], cols, eps);
+#pragma unroll
+    for (int k = 0; k < K; ++k) {
+      const int c = k * kWave + lane;
+      if (c < chunks) {
+        opaque(raw[k]);
+        if constexpr (ADD) opaque(add[k]);
+        float v[N], wk[N], o[N];
+        values(k, v);
+        if constexpr (ADD) Chunk<T>::store(x + row * cols + c * N, v);  // before out (which may be x)
+        if constexpr (RESIDENT) {
+#pragma unroll
+          for (int j = 0; j < N; ++j) wk[j] = w[k][j];
+        } else {
+          load_f32<N>(weight + c * N, wk);
+        }
+#pragma unroll
+        for (int j = 0; j < N; ++j) o[j] = (float)((double)v[j] * factor * ((double)wk[j] + (double)offset));
+        Chunk<T>::store(out + row * cols + c * N, o);
+      }
+    }
+    if constexpr (!RESIDENT) return;
+    if (following >= rows) return;
+    row = following;
+#pragma unroll
+    for (int k = 0; k < K; ++k) {
+      raw[k] = next[k];
+      if constexpr (ADD) add[k] = next_add[k];
+    }
+  }
+}
+
+// Rows of at most 64 chunks (attention heads): G lanes a row, G the power of
+// two at or above its chunks, a wave taking U passes of 64 / G rows, every
+// load issued before the first sum and the lane's weights read once for all
+// its rows. The sum over G lanes is the wave's with zeros beyond
+// (rms_norm_rows), the same to the last bit. Memory bounds it from about 10
+// MB. Measured, us a launch in graph replays, rms_norm_rows (a row a wave,
+// half its lanes or more idle) / U = 1 / 2 / 4 / 8:
+//   F32 [65248, 128] 22.3 / 12.1 / 12.6 / 12.7 / 12.8
+//   bf16 [157104, 256] (161 MB) 60.4 / 29.5 / 28.1 / 27.8 / 29.4
+//   bf16 [100000, 128] 38.2 / 10.8 / 10.8 / 10.8 / 11.5
+//   F32 [70000, 72] 21.8 / 10.8 / 9.4 / 9.7 / 10.2
+//   bf16 [4192, 256] 3.5 / 2.5 / - / 3.1 / -; F32 [32, 128] 1.95 / 1.75 / - / 2.2 / -
+template <typename T, int G, int U>
+__global__ void __launch_bounds__(kWave) rms_norm_groups(const T* x, const float* weight, T* out, int64_t rows,
+                                                         int cols, float eps, float offset) {
+  constexpr int N = Chunk<T>::N;
+  constexpr int kRows = kWave / G;
+  const int lane = threadIdx.x;
+  const bool inside = lane % G < cols / N;
+  const int c = min(lane % G, cols / N - 1) * N;
+  const int64_t first = (int64_t)blockIdx.x * (kRows * U) + lane / G;
+  typename Chunk<T>::Raw raw[U];
+#pragma unroll
+  for (int u = 0; u < U; ++u) raw[u] = Chunk<T>::load_raw(x + min(first + u * kRows, rows - 1) * cols + c);
+  float w[N];
+  load_f32<N>(weight + c, w);
+#pragma unroll
+  for (int u = 0; u < U; ++u) {
+    float v[N], o[N];
+    Chunk<T>::unpack(raw[u], v);
+    double squares = chunk_squares(v);
+    if (!inside) squares = 0.0;
+    const double factor = rms_factor(group_sum<G>(squares), cols, eps);
+    const int64_t row = first + u * kRows;
+#pragma unroll
+    for (int j = 0; j < N; ++j) o[j] = (float)((double)v[j] * factor * ((double)w[j] + (double)offset));
+    if (inside && row < rows) Chunk<T>::store(out + row * cols + c, o);
   }
 }
 
@@ -188,7 +337,7 @@ __global__ void __launch_bounds__(64 * W) rms_norm_wide(T* x, const T* y, const 
     }
     __syncthreads();
     const double total = ((partial[0] + partial[1]) + partial[2]) + partial[3];
-    const double factor = 1.0 / sqrt(total / (double)cols + (double)eps);
+    const double factor = rms_factor(total, cols, eps);
 #pragma unroll
     for (int k = 0; k < K; ++k) {
       const int c = (k * W + wave) * kWave + lane;
@@ -224,7 +373,7 @@ __global__ void __launch_bounds__(256) rms_norm_rows_scalar(T* x, const T* y, co
       squares += (double)v * (double)v;
     }
     squares = row_sum<4>(squares, partial);
-    const double factor = 1.0 / sqrt(squares / (double)cols + (double)eps);
+    const double factor = rms_factor(squares, cols, eps);
     const float* w = weight + (row % weight_rows) * cols;
     for (int c = threadIdx.x; c < cols; c += 256) {
       float v = load_one(xr + c);
@@ -260,7 +409,7 @@ __global__ void __launch_bounds__(256) rms_norm_narrow(T* x, const T* y, const f
         squares += (double)v[c] * (double)v[c];
       }
     }
-    const double factor = 1.0 / sqrt(squares / (double)cols + (double)eps);
+    const double factor = rms_factor(squares, cols, eps);
     const float* w = weight + (row % weight_rows) * cols;
 #pragma unroll
     for (int c = 0; c < kNarrowCols; ++c) {
@@ -643,6 +792,63 @@ int wide_waves(int64_t rows, int cols, const RowPlan& plan) {
   return 0;
 }
 
+// rms_norm_waves for rows of four waves' chunks, where it measured faster than
+// the four-wave group (its comment's figures): alone, from 384 rows; with the
+// residual, from 1025 to 4096 rows of at most 12 chunks a lane, and BF16 rows
+// past the resident line. RESIDENT up to a row a wave (1024 waves: one a SIMD)
+// and from 7 on. Returns false for the others.
+constexpr int64_t kSimds = 1024;
+constexpr int64_t kWaveRowsMax = INT32_MAX;
+
+template <typename T>
+bool rms_waves_launch(T* x, const T* y, const float* weight, T* out, int64_t rows, int cols, float eps, float offset,
+                      hipStream_t s) {
+  const int per_lane = (int)ceil_div(cols / Chunk<T>::N, kWave);
+  const bool resident = rows <= kSimds || rows >= 7 * kSimds;
+  if (rows < 384 || rows > kWaveRowsMax || per_lane > 20) return false;
+  if (y && (per_lane > 12 || rows <= kSimds || (rows > 4 * kSimds && !(sizeof(T) == 2 && resident)))) return false;
+  const dim3 grid((unsigned)(resident ? std::min(rows, kSimds) : rows)), block(kWave);
+#define DRIFT_RMS_WAVES(K)                                                                                          \
+  if (per_lane <= K) {                                                                                              \
+    if (y && resident)                                                                                              \
+      hipLaunchKernelGGL((rms_norm_waves<T, K, true, true>), grid, block, 0, s, x, y, weight, out, rows, cols, eps, \
+                         offset);                                                                                   \
+    else if (y)                                                                                                     \
+      hipLaunchKernelGGL((rms_norm_waves<T, K, true, false>), grid, block, 0, s, x, y, weight, out, rows, cols,     \
+                         eps, offset);                                                                              \
+    else if (resident)                                                                                              \
+      hipLaunchKernelGGL((rms_norm_waves<T, K, false, true>), grid, block, 0, s, x, y, weight, out, rows, cols,     \
+                         eps, offset);                                                                              \
+    else                                                                                                            \
+      hipLaunchKernelGGL((rms_norm_waves<T, K, false, false>), grid, block, 0, s, x, y, weight, out, rows, cols,    \
+                         eps, offset);                                                                              \
+    return true;                                                                                                    \
+  }
+  DRIFT_RMS_WAVES(4)
+  DRIFT_RMS_WAVES(6)
+  DRIFT_RMS_WAVES(8)
+  DRIFT_RMS_WAVES(10)
+  DRIFT_RMS_WAVES(12)
+  DRIFT_RMS_WAVES(16)
+  DRIFT_RMS_WAVES(20)
+#undef DRIFT_RMS_WAVES
+  return false;
+}
+
+// rms_norm_groups: two passes a wave past 16 waves a CU, else one.
+template <typename T, int G>
+void rms_groups_launch(const T* x, const float* weight, T* out, int64_t rows, int cols, float eps, float offset,
+                       hipStream_t s) {
+  constexpr int kRows = kWave / G;
+  const int64_t waves = ceil_div(rows, kRows);
+  if (waves <= 4 * kSimds)
+    hipLaunchKernelGGL((rms_norm_groups<T, G, 1>), dim3((unsigned)waves), dim3(kWave), 0, s, x, weight, out, rows,
+                       cols, eps, offset);
+  else
+    hipLaunchKernelGGL((rms_norm_groups<T, G, 2>), dim3((unsigned)ceil_div(waves, 2)), dim3(kWave), 0, s, x, weight,
+                       out, rows, cols, eps, offset);
+}
+
 template <typename T>
 int rms_norm(const char* entry, T* x, const T* y, const float* weight, T* out, int64_t rows, int32_t cols, float eps,
              float offset, int32_t weight_rows, Quantized q, void* stream) {
@@ -667,6 +873,19 @@ int rms_norm(const char* entry, T* x, const T* y, const float* weight, T* out, i
   } else if (plan.per_lane == 0) {
     hipLaunchKernelGGL(rms_norm_rows_scalar<T>, dim3(grid_for(rows, 1)), dim3(256), 0, s, x, y, weight, out, rows,
                        (int)cols, eps, offset, (int)weight_rows);
+  } else if (weight_rows == 1 && !y && !q.xq && cols / Chunk<T>::N <= kWave && rows <= kWaveRowsMax) {
+    const int chunks = cols / Chunk<T>::N;
+    if (chunks <= 8)
+      rms_groups_launch<T, 8>(x, weight, out, rows, cols, eps, offset, s);
+    else if (chunks <= 16)
+      rms_groups_launch<T, 16>(x, weight, out, rows, cols, eps, offset, s);
+    else if (chunks <= 32)
+      rms_groups_launch<T, 32>(x, weight, out, rows, cols, eps, offset, s);
+    else
+      rms_groups_launch<T, 64>(x, weight, out, rows, cols, eps, offset, s);
+  } else if (weight_rows == 1 && !q.xq && plan.waves == 4 &&
+             rms_waves_launch(x, y, weight, out, rows, cols, eps, offset, s)) {
+    return launched(entry);
   } else if (const int wide = wide_waves<T>(rows, cols, plan)) {
     const int per_lane = (int)ceil_div(cols / Chunk<T>::N, kWave * wide);
     const dim3 grid((unsigned)rows), block(kWave * wide);

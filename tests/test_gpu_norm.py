@@ -120,6 +120,39 @@ def test_rms_norm_does_not_depend_on_the_batch(hip, dtype, cols):
     assert np.array_equal(host(few).view(np.uint8), host(batch)[100:107].view(np.uint8)), "rows 100-106"
 
 
+# rows on both sides of each line between a row's splits (384, 1,024, 4,096
+# and 7,168 rows of four waves' chunks; a last wave's rows part full), lanes
+# past the row's chunks, the most chunks a lane, and rows of at most 64 chunks
+# of one, two and many passes
+@pytest.mark.parametrize("rows,cols,dtype,add", [
+    (383, 1024, "f32", False), (384, 1028, "f32", False), (1024, 5120, "f32", False), (1025, 1024, "f32", True),
+    (1500, 3076, "f32", True), (4097, 1024, "f32", True), (7169, 1024, "f32", False), (400, 5124, "f32", False),
+    (1024, 2056, "bf16", False), (1025, 4104, "bf16", False), (4096, 2048, "bf16", True), (4097, 2048, "bf16", True),
+    (7168, 2056, "bf16", True), (8193, 2048, "bf16", False), (1100, 10240, "bf16", False),
+    (1, 36, "f32", False), (1001, 72, "f32", False), (9001, 256, "f32", False), (70001, 40, "bf16", False),
+    (20003, 128, "bf16", False), (9999, 264, "bf16", False), (8193, 512, "bf16", False),
+])
+def test_rms_norm_row_splits(hip, rows, cols, dtype, add):
+    step(f"rmsNorm {dtype} [{rows}, {cols}], residual {add}")
+    x, y = gaussian(51, (rows, cols), 2.0), gaussian(52, (rows, cols))
+    w = (1 + 0.1 * gaussian(53, cols)).astype(np.float32)
+    if dtype == "f32":
+        to, host, want = dev_f32, host_f32, o.rms_norm(x, w, 1e-6, 0.0, y=y if add else None)
+    else:
+        x, y = bf16_input(x), bf16_input(y)
+        to, host, want = dev_bf16, host_bits, o.rms_norm_bf16(x, w, 1e-6, y_bits=y if add else None)
+    xd = to(x)
+    if add:
+        out = torch.empty_like(xd)
+        hip.addRmsNorm(xd, to(y), d.RowNorm(dev_f32(w), 1e-6, 0.0, out))
+        summed, want = want
+        assert np.array_equal(host(xd), summed), "x += y"
+    else:
+        out = xd  # in place
+        hip.rmsNorm(xd, dev_f32(w), 1e-6, 0.0, out)
+    (assert_f32 if dtype == "f32" else assert_bf16)(want, host(out), what=f"rmsNorm [{rows}, {cols}]")
+
+
 # (rows, groups, width) of the group norm, one case for each way the library
 # splits a row: a thread per narrow row (<= 32 values), the scalar path
 # (widths not whole 16-byte chunks), a wave or a 4-wave group per row in a
