@@ -15,7 +15,6 @@
 // 89-146, as rope.hpp), and F32 -> F16 rounding to nearest even for the
 // cache (Float.floatToFloat16 in ops/CpuAttention.scala:181-210).
 #include "rope.hpp"
-#include "sincos.hpp"
 
 #include <algorithm>
 #include <climits>
@@ -212,7 +211,8 @@ constexpr int kTileHeads(int dim) { return dim * 32 >= 4096 ? 1 : 4096 / (dim * 
 __device__ __forceinline__ int tile_dword(int value, int position) { return value * 8 + (value / 8) * 8 + position / 2; }
 
 // LDS words the staged tile takes
-constexpr int kTileWords(int dim) { return kTileHeads(dim) * dim * 9; }
+constexpr int kTileWords(int dim, int heads) { return heads * dim * 9; }
+constexpr int kTileWords(int dim) { return kTileWords(dim, kTileHeads(dim)); }
 
 template <typename T, int DIM, int H = kTileHeads(DIM)>
 __device__ __forceinline__ void cache_values_tile(const Extras<T>& e, int64_t tokens, int kv_heads, int64_t tile,
@@ -283,20 +283,12 @@ __device__ __forceinline__ void cache_values_tile(const Extras<T>& e, int64_t to
     }
   } else {
     const uint16_t* halves = reinterpret_cast<const uint16_t*>(staged);
-    for (int c = lane; c < heads * DIM * kTile; c += kWave) {
-      const int value = c / kTile, i = c % kTile;
-      if (first + i >= lo && first + i < hi)
-        row0[(int64_t)value * e.page_size + i] = halves[2 * tile_dword(value, i) + (i & 1)];
+    const int width = (int)(hi - lo), skip = (int)(lo - first);  // a decode step's is 1
+    for (int c = lane; c < heads * DIM * width; c += kWave) {
+      const int value = c / width, i = skip + c - value * width;
+      row0[(int64_t)value * e.page_size + i] = halves[2 * tile_dword(value, i) + (i & 1)];
     }
   }
-}
-
-// cos and sin of an angle of 2^20 or more by the library, out of line: its
-// registers are not the kernel's while the heads and weights wait in theirs
-__device__ __attribute__((noinline)) double2 sincos_far(float angle) {
-  double sn, cn;
-  sincos((double)angle, &sn, &cn);
-  return make_double2(cn, sn);
 }
 
 // MIXED: heads of which only the first `rotary` values turn, or whose pairs
@@ -419,13 +411,7 @@ __device__ __forceinline__ void qk_wave_heads(const T* q, const T* k, T* q_out, 
     const int j = lane + u * kWave;
     if (j < half) {
       const float angle = (float)position[MIXED ? u : 0] * inverse[u];
-      double sn, cn;
-      if (!sincos_reduced(angle, &sn, &cn)) {
-        const double2 far = sincos_far(angle);
-        cn = far.x;
-        sn = far.y;
-      }
-      cs[qk_pair_slot<NEOX, G, N>(j)] = make_double2(cn, sn);
+      cs[qk_pair_slot<NEOX, G, N>(j)] = cos_sin(angle);
     }
   }
   wave_sync();
@@ -591,6 +577,44 @@ __global__ void __launch_bounds__(256) cache_write_chunks(const T* k, Extras<T> 
 #pragma unroll
     for (int j = 0; j < N; ++j) e.values[value + (int64_t)(c * N + j) * e.page_size] = (uint16_t)f16_bits(vx[j]);
   }
+}
+
+// The same for heads of whole runs of 8 values, in one-wave blocks: the first
+// `tiles` of them write the values by tiles of 16 positions (a token's values
+// are kv_heads * dim / 8 runs of 8 in the input and in a page alike, so the
+// tiles take them as heads of 8), the others 64 runs of 8 key values each.
+// The thread per chunk above stores its values 2 bytes at a time, page_size
+// apart; it stays for small writes, where the tiles are few waves with a
+// longer chain each. Measured, us a launch in graph replays, chunks / tiles:
+// F32 [2039, 8, 128] 18.1 / 7.0, bf16 [6546, 4, 256] 48.7 / 11.2, [600, 8,
+// 128] 7.6 / 4.7; bf16 [262, 2, 256] 3.3 / 3.9, F32 [64, 8, 128] 2.8 / 2.9,
+// one token of 8 heads 2.3 / 2.4.
+// More runs of 8 than these go by tiles (both kernels measure about 3.5 us
+// there).
+constexpr int64_t kTiledRuns = 20480;
+
+// Runs of 8 values a tile: what its wave loads with four chunks a lane.
+template <typename T>
+constexpr int kTileRuns = 2 * Chunk<T>::N;
+
+template <typename T>
+__global__ void __launch_bounds__(kWave) cache_write_tiles(const T* k, Extras<T> e, int64_t tokens, int runs,
+                                                           double runs_inverse) {
+  constexpr int kRun = 8;
+  constexpr int N = Chunk<T>::N;
+  __shared__ __align__(16) uint32_t staged[kTileWords(kRun, kTileRuns<T>)];
+  if (blockIdx.x < e.tiles) {
+    cache_values_tile<T, kRun, kTileRuns<T>>(e, tokens, runs, blockIdx.x, staged);
+    return;
+  }
+  const int64_t i = ((int64_t)blockIdx.x - e.tiles) * kWave + threadIdx.x;
+  const int64_t t = quotient(i, runs, runs_inverse);
+  if (t >= tokens) return;
+  float v[kRun];
+#pragma unroll
+  for (int j = 0; j < kRun; j += N) Chunk<T>::load(k + i * kRun + j, *reinterpret_cast<float(*)[N]>(v + j));
+  int64_t key, value;
+  if (cache_place(e, t, 1, runs * kRun, 0, key, value)) store_f16<kRun>(e.keys + key + (i - t * runs) * kRun, v);
 }
 
 template <typename T>
@@ -805,10 +829,18 @@ int cache_write(const char* entry, const T* k, const T* v, uint16_t* keys, uint1
   if ((int64_t)tokens * kv_heads == 0) return 0;
   if (!k || !v || !keys || !values || !page_table) return refuse("%s: null tensor", entry);
   const Extras<T> e{nullptr, v, keys, values, page_table, cache_pages, page_size, start, bad_page, 0};
-  constexpr int N = Chunk<T>::N;
   const hipStream_t st = (hipStream_t)stream;
   const int64_t values_count = (int64_t)tokens * kv_heads * dim;
-  if (dim % N == 0 && aligned16(k) && aligned16(v) && aligned16(keys))
+  const int64_t runs = (int64_t)kv_heads * dim / 8;
+  Extras<T> et = e;
+  et.tiles = (((int64_t)start + tokens - 1) / 16 - start / 16 + 1) * ceil_div(runs, kTileRuns<T>);
+  const int64_t blocks = et.tiles + ceil_div(tokens * runs, kWave);
+  constexpr int N = Chunk<T>::N;
+  if (dim % 8 == 0 && tokens * runs > kTiledRuns && aligned16(k) && aligned16(v) && aligned16(keys) &&
+      aligned16(values) && runs * 8 <= INT32_MAX && blocks <= kOneShotBlocks)
+    hipLaunchKernelGGL(cache_write_tiles<T>, dim3((unsigned)blocks), dim3(kWave), 0, st, k, et, (int64_t)tokens,
+                       (int)runs, 1.0 / (double)runs);
+  else if (dim % N == 0 && aligned16(k) && aligned16(v) && aligned16(keys))
     hipLaunchKernelGGL(cache_write_chunks<T>, dim3(grid_for(values_count / N, 256, kOneShotBlocks)), dim3(256), 0, st,
                        k, e, (int64_t)tokens, kv_heads, dim);
   else

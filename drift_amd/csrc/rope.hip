@@ -2,10 +2,10 @@
 // sections, per-axis), rope from cos/sin tables, Wan's 3-D rope with its
 // angles made in the kernel, and per-head query/key RMSNorm fused with rope.
 //
-// Layout: x, out [tokens, heads, head_dim], row-major. One workgroup takes a
-// token at a time: it first makes the token's cos/sin for every pair (once,
-// shared by all its heads: the reference recomputes them per value), then
-// turns every head's pairs. Where a head is whole 16-byte chunks, each lane
+// Layout: x, out [tokens, heads, head_dim], row-major. A wave (or, for the
+// awkward shapes, a block) first makes its tokens' cos/sin for every pair
+// (shared by the heads it takes: the reference recomputes them per value),
+// then turns the heads' pairs. Where a head is whole 16-byte chunks, each lane
 // reads a pair's two chunks (NeoX: a chunk and its partner half a rotary
 // away; interleaved: pairs sit inside a chunk), turns them in registers and
 // writes them back, so out may be x.
@@ -20,6 +20,7 @@
 
 #include <algorithm>
 #include <climits>
+#include <initializer_list>
 
 namespace drift {
 namespace {
@@ -67,31 +68,124 @@ __device__ __forceinline__ void turn_chunks(const T* xh, T* oh, int item, int ro
   }
 }
 
+// Any width and alignment: a block a token, a value or pair at a time.
 template <typename T>
-__device__ __forceinline__ int chunk_items(int dim, int rotary, int layout) {
-  constexpr int N = Chunk<T>::N;
-  return layout == DRIFT_ROPE_NEOX ? rotary / 2 / N + (dim - rotary) / N : dim / N;
-}
-
-template <typename T, bool CHUNKED>
 __global__ void __launch_bounds__(256) rope_kernel(const T* x, const int32_t* positions, T* out, RopeArgs p) {
   __shared__ double2 cs[kMaxPairs];
-  const int slots = CHUNKED ? chunk_items<T>(p.dim, p.rotary, p.layout) : (p.dim + 1) / 2;
+  const int slots = (p.dim + 1) / 2;
   for (int64_t t = blockIdx.x; t < p.tokens; t += gridDim.x) {
     token_angles(p, positions, t, cs);
     __syncthreads();
     const T* xt = x + t * p.heads * p.dim;
     T* ot = out + t * p.heads * p.dim;
-    for (int i = threadIdx.x; i < p.heads * slots; i += blockDim.x) {
-      const int h = i / slots, j = i % slots;
-      const T* xh = xt + (int64_t)h * p.dim;
-      T* oh = ot + (int64_t)h * p.dim;
-      if constexpr (CHUNKED)
-        turn_chunks<T>(xh, oh, j, p.rotary, p.layout, cs);
-      else
-        turn_slot<T>(j, p.dim, p.rotary, p.layout, cs, [&](int d) { return (double)load_one(xh + d); }, oh);
+    for (int64_t i = threadIdx.x; i < (int64_t)p.heads * slots; i += blockDim.x) {
+      const int64_t h = i / slots;
+      const T* xh = xt + h * p.dim;
+      turn_slot<T>((int)(i - h * slots), p.dim, p.rotary, p.layout, cs, [&](int d) { return (double)load_one(xh + d); },
+                   ot + h * p.dim);
     }
     __syncthreads();  // cs is remade for the next token
+  }
+}
+
+// Heads and rotating parts of whole 16-byte chunks, in one-wave blocks with no
+// barrier. An item is turn_chunks' (NeoX: a chunk and its partner;
+// interleaved: a chunk), a head has `rotating` of them and then its tail's
+// chunks (none in place: they stay as they are). A wave takes K * 64 items of
+// one token (`runs` waves a token) or, where a token has fewer, of `per_wave`
+// tokens. It issues its loads, makes its tokens' cos and sin while they land
+// (a pair a lane, into its LDS), and turns its items from there.
+//
+// Memory bounds the large launches. Measured, us a launch in graph replays, a
+// 256-thread block a token with two barriers and the library's sincos / this:
+// F32 in place [2039, 32, 128] (67 MB) 12.8 / 12.5, [2039, 8, 128] 5.8 / 4.3;
+// bf16 [6546, 24, 256] with 64 values turning, in place 43.5 / 10.9 (its tail
+// copied onto itself before), out of place (161 MB) 44.0 / 31.7, [6546, 4,
+// 256] in place 17.1 / 3.6; bf16 interleaved [4096, 32, 128] 15.8 / 12.1; F32
+// over two axes [4087, 16, 72] 10.4 / 9.9; one token of 32 heads 2.2 / 1.9.
+// K = 1, 2, 4 there: [2039, 32, 128] 12.1, 11.9, 12.5; out of place [6546, 24,
+// 256] 30.6, 32.5, 31.7; [4087, 16, 72] 9.7, 13.1 (its second wave nearly
+// empty), 9.8; [262, 16, 256] in place 2.4, 2.9, 3.9.
+//
+// Pair m of an item j sits in LDS at m * rotating + j, so that lanes on
+// consecutive items read consecutive entries.
+// Row i / slots comes from a product with slots_inverse = ceil(2^32 / slots)
+// (exact where i * slots < 2^32: the launcher's bound on a token; 0 where
+// slots is 1). TOKENS: a wave's items are of several tokens.
+template <typename T, bool NEOX, int K, bool TOKENS>
+__global__ void __launch_bounds__(kWave) rope_waves(const T* x, const int32_t* positions, T* out, RopeArgs p, int slots,
+                                                    uint32_t slots_inverse, uint32_t runs, int per_wave) {
+  constexpr int N = Chunk<T>::N;
+  constexpr int P = NEOX ? N : N / 2;  // pairs of an item
+  using Raw = typename Chunk<T>::Raw;
+  constexpr int kPairsPerLane = kMaxPairs / kWave;
+  __shared__ double2 cs[kMaxPairs];
+  const int lane = threadIdx.x;
+  const int half = p.rotary / 2, rotating = half / P;
+  const int items = p.heads * slots;  // a token's
+  const uint32_t group = blockIdx.x / runs, run = blockIdx.x - group * runs;
+  const int64_t t0 = TOKENS ? (int64_t)group * per_wave : (int64_t)group;
+  const int tokens = TOKENS ? (int)min((int64_t)per_wave, p.tokens - t0) : 1;
+  // the small operands load first (a pair's position and frequency), and are
+  // used only once the items' loads are issued
+  const int pairs = tokens * half;
+  int32_t position[kPairsPerLane];
+  float inverse[kPairsPerLane];
+#pragma unroll
+  for (int u = 0; u < kPairsPerLane; ++u) {
+    if (u * kWave < pairs) {
+      const int i = min(u * kWave + lane, pairs - 1);
+      const int tt = TOKENS ? i / half : 0, j = i - tt * half;
+      position[u] = positions[(int64_t)rope_section(j, p) * p.tokens + t0 + tt];
+      inverse[u] = p.inverse[j];
+    }
+  }
+  const T* xt = x + t0 * p.heads * p.dim;
+  T* ot = out + t0 * p.heads * p.dim;
+  const int last = tokens * items - 1;
+  Raw r0[K], r1[NEOX ? K : 1];
+  int at[K], slot[K];
+  bool turns[K];
+#pragma unroll
+  for (int k = 0; k < K; ++k) {
+    const int i = min((int)(run * K + k) * kWave + lane, last);
+    const int row = slots_inverse ? (int)__umulhi((uint32_t)i, slots_inverse) : i;  // (token, head) of the wave's
+    const int j = i - row * slots;
+    turns[k] = j < rotating;
+    at[k] = row * p.dim + (NEOX && !turns[k] ? p.rotary + (j - rotating) * N : j * N);
+    slot[k] = (TOKENS ? row / p.heads * half : 0) + j;
+    r0[k] = Chunk<T>::load_raw(xt + at[k]);
+    if constexpr (NEOX) r1[k] = Chunk<T>::load_raw(xt + at[k] + (turns[k] ? half : 0));
+  }
+#pragma unroll
+  for (int u = 0; u < kPairsPerLane; ++u) {
+    const int i = u * kWave + lane;
+    if (i < pairs) {
+      const int tt = TOKENS ? i / half : 0, j = i - tt * half;
+      asm volatile("" : "+v"(position[u]));  // converted here, not (waiting) before the items' loads
+      cs[tt * half + j % P * rotating + j / P] = cos_sin((float)position[u] * inverse[u]);
+    }
+  }
+  wave_sync();
+#pragma unroll
+  for (int k = 0; k < K; ++k) {
+    if ((int)(run * K + k) * kWave + lane > last) return;
+    float a[N], b[N];
+    Chunk<T>::unpack(r0[k], a);
+    if constexpr (NEOX) Chunk<T>::unpack(r1[k], b);
+    if (turns[k]) {
+#pragma unroll
+      for (int i = 0; i < P; ++i) {
+        const double2 q = cs[slot[k] + i * rotating];
+        if constexpr (NEOX)
+          turn_fused(a[i], b[i], q.x, q.y, a[i], b[i]);
+        else
+          turn_fused(a[2 * i], a[2 * i + 1], q.x, q.y, a[2 * i], a[2 * i + 1]);
+      }
+    }
+    Chunk<T>::store(ot + at[k], a);
+    if constexpr (NEOX)
+      if (turns[k]) Chunk<T>::store(ot + at[k] + half, b);
   }
 }
 
@@ -341,14 +435,57 @@ int rope(const char* entry, const T* x, const int32_t* positions, T* out, int32_
   RopeArgs p;
   fill_rope(p, tokens, heads, dim, rotary, theta, layout, sections, s);
   constexpr int N = Chunk<T>::N;
-  const bool chunked = aligned16(x) && aligned16(out) && dim % N == 0 &&
-                       rotary % (layout == DRIFT_ROPE_NEOX ? 2 * N : N) == 0;
-  const dim3 grid(grid_for(tokens, 1, 1 << 16));
+  const bool neox = layout == DRIFT_ROPE_NEOX;
+  const bool chunked = aligned16(x) && aligned16(out) && dim % N == 0 && rotary % (neox ? 2 * N : N) == 0 &&
+                       (int64_t)heads * dim <= (1 << 24);
   const hipStream_t st = (hipStream_t)stream;
-  if (chunked)
-    hipLaunchKernelGGL((rope_kernel<T, true>), grid, dim3(256), 0, st, x, positions, out, p);
-  else
-    hipLaunchKernelGGL((rope_kernel<T, false>), grid, dim3(256), 0, st, x, positions, out, p);
+  const int rotating = neox ? rotary / 2 / N : rotary / N;
+  const int slots = x == out ? rotating : rotating + (dim - rotary) / N;
+  if (chunked && slots == 0) return 0;  // in place with nothing to turn
+  const int64_t items = (int64_t)heads * std::max(slots, 1);
+  // items a lane: one in launches of up to 8 waves a CU of one; else the count
+  // of 4, 3 or 2 whose waves hold a token's items with the fewest idle lanes
+  int per_lane = 1;
+  if (tokens * items > 2048 * kWave) {
+    per_lane = 4;
+    for (int k : {3, 2})
+      if (ceil_div(items, k * kWave) * k < ceil_div(items, per_lane * kWave) * per_lane &&
+          items > per_lane * kWave / 2)
+        per_lane = k;
+  }
+  const int64_t runs = ceil_div(items, per_lane * kWave);
+  // whole tokens of a wave: as many as its items and its LDS's pairs hold
+  const int64_t fit = std::min<int64_t>(per_lane * kWave / items, rotary > 0 ? kMaxPairs / (rotary / 2) : kMaxPairs);
+  const int64_t per_wave = std::max<int64_t>(1, std::min<int64_t>(fit, tokens));
+  const int64_t blocks = ceil_div(tokens, per_wave) * runs;
+  if (chunked && blocks <= kOneShotBlocks) {
+    const dim3 grid((unsigned)blocks), block(kWave);
+    const uint32_t slots_inverse = slots == 1 ? 0 : (uint32_t)ceil_div((int64_t)1 << 32, slots);
+#define DRIFT_ROPE_LAUNCH(NEOX, K, TOKENS)                                                                       \
+  hipLaunchKernelGGL((rope_waves<T, NEOX, K, TOKENS>), grid, block, 0, st, x, positions, out, p, slots,          \
+                     slots_inverse, (uint32_t)runs, (int)per_wave)
+#define DRIFT_ROPE_CASE(K)                \
+  case K:                                 \
+    if (neox && per_wave > 1)             \
+      DRIFT_ROPE_LAUNCH(true, K, true);   \
+    else if (neox)                        \
+      DRIFT_ROPE_LAUNCH(true, K, false);  \
+    else if (per_wave > 1)                \
+      DRIFT_ROPE_LAUNCH(false, K, true);  \
+    else                                  \
+      DRIFT_ROPE_LAUNCH(false, K, false); \
+    break;
+    switch (per_lane) {
+      DRIFT_ROPE_CASE(1)
+      DRIFT_ROPE_CASE(2)
+      DRIFT_ROPE_CASE(3)
+      DRIFT_ROPE_CASE(4)
+    }
+#undef DRIFT_ROPE_CASE
+#undef DRIFT_ROPE_LAUNCH
+  } else {
+    hipLaunchKernelGGL(rope_kernel<T>, dim3(grid_for(tokens, 1, 1 << 16)), dim3(256), 0, st, x, positions, out, p);
+  }
   return launched(entry);
 }
 

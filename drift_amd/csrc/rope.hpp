@@ -8,6 +8,7 @@
 #include <cstring>
 
 #include "common.hpp"
+#include "sincos.hpp"
 
 namespace drift {
 namespace {
@@ -45,6 +46,21 @@ __device__ __forceinline__ void token_angles(const RopeArgs& p, const int32_t* p
     sincos((double)angle, &sn, &cn);
     cs[j] = make_double2(cn, sn);
   }
+}
+
+// cos and sin of an angle of 2^20 or more by the library, out of line: its
+// registers are not the kernel's while the heads and weights wait in theirs
+__device__ __attribute__((noinline)) double2 sincos_far(float angle) {
+  double sn, cn;
+  sincos((double)angle, &sn, &cn);
+  return make_double2(cn, sn);
+}
+
+// (cos, sin) of an angle in double, as sincos.hpp makes them.
+__device__ __forceinline__ double2 cos_sin(float angle) {
+  double sn, cn;
+  if (!sincos_reduced(angle, &sn, &cn)) return sincos_far(angle);
+  return make_double2(cn, sn);
 }
 
 // The turn of one pair (a first, b second) in double, as the CPU does it.

@@ -49,7 +49,11 @@ def cache(pages, kv, dim, fill_seed):
 
 
 @pytest.mark.parametrize("dtype", ["f32", "bf16"])
-@pytest.mark.parametrize("tokens,kv,dim,start", [(1, 8, 128, 14), (37, 2, 128, 5), (5, 3, 72, 30), (1, 1, 8, 0)])
+@pytest.mark.parametrize("tokens,kv,dim,start", [(1, 8, 128, 14), (37, 2, 128, 5), (5, 3, 72, 30), (1, 1, 8, 0),
+                                                    # past the line to the value tiles: runs that fill no whole
+                                                    # tile, first and last pages cut, one run a token
+                                                    (431, 3, 136, 7), (700, 8, 128, 16), (1200, 1, 152, 33),
+                                                    (20501, 1, 8, 3), (650, 5, 56, 15)])
 def test_cache_write(hip, dtype, tokens, kv, dim, start):
     step(f"cacheWrite {dtype} {tokens} tokens, {kv} heads of {dim}, start {start}")
     pages = -(-(start + tokens) // PAGE) + 1

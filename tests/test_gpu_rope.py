@@ -96,6 +96,36 @@ def test_rope_odd_shapes_and_in_place(hip, shape, rotary, layout):
     assert_f32(oracle_rope(x, p, rope), host_f32(xd), what="rope in place")
 
 
+# whole chunks: several tokens a wave (the last group part full), a token over
+# several waves, one to four items a lane, tails copied and left in place,
+# nothing turning, angles past 2^20
+@pytest.mark.parametrize("in_place", [True, False])
+@pytest.mark.parametrize("dtype", ["f32", "bf16"])
+@pytest.mark.parametrize("shape,rotary,layout,sections,scale", [
+    ((1001, 4, 256), 64, 0, R.Single(), 1), ((700, 16, 72), 72, 0, R.Axes((18, 18)), 1),
+    ((300, 28, 128), 128, 0, R.Contiguous(16, 24, 24), 1), ((515, 24, 256), 64, 0, R.Interleaved(11, 11, 10), 1),
+    ((1203, 9, 64), 48, 1, R.Single(), 1), ((37, 1, 16), 16, 0, R.Single(), 1), ((5, 3, 512), 512, 0, R.Single(), 1),
+    ((4100, 1, 32), 16, 0, R.Single(), 977), ((3, 2, 128), 128, 1, R.Axes((16, 24, 24)), 99991),
+])
+def test_rope_chunks(hip, shape, rotary, layout, sections, scale, dtype, in_place):
+    step(f"rope {dtype} {shape} rotary {rotary} layout {layout} {sections}, in place {in_place}")
+    count = sections.positionsPerToken
+    p = ((np.arange(count * shape[0]) * 131) % 4096 * scale).astype(np.int32)
+    p = p if count == 1 else p.reshape(count, shape[0])
+    rope = d.Rope(1e4, rotary, d.RopeLayout(layout), sections)
+    x = gaussian(21, shape, 3.0)
+    if dtype == "bf16":
+        x = o.from_bf16(bf16_input(x))
+    xd = dev_f32(x) if dtype == "f32" else dev_bf16(o.to_bf16(x))
+    out = xd if in_place else torch.full_like(xd, 7.0)
+    hip.rope(xd, dev_i32(p), rope, out)
+    want = oracle_rope(x, p, rope)
+    if dtype == "f32":
+        assert_f32(want, host_f32(out), what="rope")
+    else:
+        assert_bf16(o.to_bf16(want), host_bits(out), what="rope bf16")
+
+
 def test_c1_rms_norm_then_rope_seed_0(hip):
     # C1: RMSNorm (eps 1e-6) on x[8, 2048] ~ N(0,1), weight ~ N(1, 0.1); NeoX
     # RoPE (theta 1e4) on Q[8, 16, 128] at positions 0..7; inputs from
