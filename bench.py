@@ -683,7 +683,7 @@ def row_probes(k: Kernel, lib) -> list:
         probe.slices = slices
         for _, _, (table, ids, out, count, vocab, cols, _) in k.calls:
             row_bytes = cols // 32 * 34
-            if row_bytes % 16 or table.value % 16:
+            if row_bytes % 16 or table % 16:
                 return []
             if slices == 0:
                 probe.calls.append(("drift_row_probe", lib.drift_row_probe,

@@ -18,7 +18,6 @@ stream given to the constructor); nothing synchronizes.
 
 from __future__ import annotations
 
-import ctypes
 import enum
 from dataclasses import dataclass, replace
 from typing import Optional, Sequence, Tuple
@@ -115,12 +114,15 @@ class KvCache:
     pageSize: int
 
     def __post_init__(self):
-        _require(self.pageSize % 16 == 0, f"pages of {self.pageSize} tokens: not a multiple of 16")
-        _require(self.keys.dtype == F16 and self.values.dtype == F16, "the cache is F16")
-        _require(self.keys.dim() == 4 and self.values.dim() == 4, "the cache's keys and values are 4-dimensional")
+        if self.pageSize % 16 != 0:
+            raise ValueError(f"pages of {self.pageSize} tokens: not a multiple of 16")
+        if not (self.keys.dtype == F16 and self.values.dtype == F16):
+            raise ValueError("the cache is F16")
+        if not (self.keys.dim() == 4 and self.values.dim() == 4):
+            raise ValueError("the cache's keys and values are 4-dimensional")
         self.pages, _, self.kvHeads, self.headDimension = (int(d) for d in self.keys.shape)
-        _require(tuple(self.values.shape) == (self.pages, self.kvHeads, self.headDimension, self.pageSize),
-                 f"cache values {_shape(self.values)} for keys {_shape(self.keys)}")
+        if tuple(self.values.shape) != (self.pages, self.kvHeads, self.headDimension, self.pageSize):
+            raise ValueError(f"cache values {_shape(self.values)} for keys {_shape(self.keys)}")
 
     @staticmethod
     def allocate(pages: int, pageSize: int, kvHeads: int, headDimension: int, device="cuda") -> "KvCache":
@@ -141,7 +143,8 @@ class StorageType:
     align: int
 
     def rowBytes(self, cols: int) -> int:
-        _require(cols % self.values == 0, f"{cols} elements are not whole {self.name} blocks of {self.values}")
+        if cols % self.values != 0:
+            raise ValueError(f"{cols} elements are not whole {self.name} blocks of {self.values}")
         return cols // self.values * self.bytes
 
 
@@ -249,12 +252,9 @@ class QuantizedValues:
 
 
 # ------------------------------------------------------------------ checks
-# object Ops (ops/Ops.scala:36-93) and the groups' checks.
-
-def _require(condition: bool, message: str) -> None:
-    if not condition:
-        raise ValueError(message)
-
+# object Ops (ops/Ops.scala:36-93) and the groups' checks. A refusal's message
+# is made only when it is raised: made before each check, as `require`'s
+# argument, the messages were two thirds of a decode step's host time.
 
 def _name(dtype) -> str:
     return {F32: "F32", BF16: "BF16", F16: "F16", I32: "I32", torch.int8: "I8", torch.uint8: "U8",
@@ -273,30 +273,35 @@ def _shape(t) -> str:
 
 def requireF32(operation: str, *tensors) -> None:
     for t in tensors:
-        _require(t.dtype == F32, f"{operation} takes F32, not {_name(t.dtype)}")
+        if t.dtype != F32:
+            raise ValueError(f"{operation} takes F32, not {_name(t.dtype)}")
 
 
 def requireSameShape(operation: str, *tensors) -> None:
-    _require(len({tuple(t.shape) for t in tensors}) == 1,
-             f"{operation} needs equal shapes, got {', '.join(_shape(t) for t in tensors)}")
+    first = tensors[0].shape
+    if not all(t.shape == first for t in tensors[1:]):
+        raise ValueError(f"{operation} needs equal shapes, got {', '.join(_shape(t) for t in tensors)}")
 
 
 def checkElementwise(operation: str, *tensors) -> None:
     """Same-shape operands of one float type (F32, or BF16 here)."""
-    _require(tensors[0].dtype in _FLOAT_TYPES, f"{operation} takes F32 or BF16, not {_name(tensors[0].dtype)}")
+    if tensors[0].dtype not in _FLOAT_TYPES:
+        raise ValueError(f"{operation} takes F32 or BF16, not {_name(tensors[0].dtype)}")
     for t in tensors[1:]:
-        _require(t.dtype == tensors[0].dtype,
-                 f"{operation} takes one type, not {_name(tensors[0].dtype)} and {_name(t.dtype)}")
+        if t.dtype != tensors[0].dtype:
+            raise ValueError(f"{operation} takes one type, not {_name(tensors[0].dtype)} and {_name(t.dtype)}")
     requireSameShape(operation, *tensors)
 
 
 def checkRowWise(operation: str, x, out, *rowVectors) -> int:
     """Returns the row count (ops/Ops.scala:76-92)."""
     checkElementwise(operation, x, out)
-    _require(x.dim() >= 1, f"{operation} needs at least one dimension")
+    if x.dim() < 1:
+        raise ValueError(f"{operation} needs at least one dimension")
     for vector in rowVectors:
         requireF32(operation, vector)
-        _require(tuple(vector.shape) == (x.shape[-1],), f"{operation}: {_shape(vector)} for rows of {x.shape[-1]}")
+        if vector.shape != x.shape[-1:]:
+            raise ValueError(f"{operation}: {_shape(vector)} for rows of {x.shape[-1]}")
     return x.numel() // x.shape[-1] if x.shape[-1] else 0
 
 
@@ -305,12 +310,14 @@ def checkChunks(operation: str, x, table, out, *indices) -> tuple:
     [rows, chunks * C], every index a chunk (ops/ElementwiseOps.scala:55-76)."""
     checkElementwise(operation, x, out)
     requireF32(operation, table)
-    _require(x.dim() == 2, f"{operation} takes [rows, C], not {_shape(x)}")
+    if x.dim() != 2:
+        raise ValueError(f"{operation} takes [rows, C], not {_shape(x)}")
     rows, channels = x.shape
     width = table.shape[-1] if table.dim() else 0
-    _require(table.dim() == 2 and table.shape[0] == rows and channels > 0 and width % channels == 0
-             and all(0 <= i < width // channels for i in indices),
-             f"{operation}: table {_shape(table)} for {_shape(x)}, chunks ArraySeq({', '.join(map(str, indices))})")
+    if not (table.dim() == 2 and table.shape[0] == rows and channels > 0 and width % channels == 0
+            and all(0 <= i < width // channels for i in indices)):
+        raise ValueError(f"{operation}: table {_shape(table)} for {_shape(x)}, "
+                         f"chunks ArraySeq({', '.join(map(str, indices))})")
     return rows, channels, width // channels
 
 
@@ -318,28 +325,32 @@ def checkRowGatedAdd(x, y, gate) -> tuple:
     """Returns (rows, cols) (ops/ElementwiseOps.scala:79-92)."""
     checkElementwise("rowGatedAdd", x, y)
     requireF32("rowGatedAdd", gate)
-    _require(x.dim() == 2, f"rowGatedAdd takes [rows, cols], not {_shape(x)}")
+    if x.dim() != 2:
+        raise ValueError(f"rowGatedAdd takes [rows, cols], not {_shape(x)}")
     rows, cols = x.shape
-    _require(gate.numel() == rows, f"rowGatedAdd: gate {_shape(gate)} for {_shape(x)}")
+    if gate.numel() != rows:
+        raise ValueError(f"rowGatedAdd: gate {_shape(gate)} for {_shape(x)}")
     return rows, cols
 
 
 def checkRope(x, positions, rope: Rope, out) -> tuple:
     """ops/AttentionOps.scala:185-223; returns (tokens, heads, headDimension)."""
     checkElementwise("rope", x, out)
-    _require(x.dim() == 3, f"rope takes [tokens, heads, headDimension], got {_shape(x)}")
+    if x.dim() != 3:
+        raise ValueError(f"rope takes [tokens, heads, headDimension], got {_shape(x)}")
     tokens, heads, dimension = x.shape
-    _require(positions.dtype == I32, f"rope positions are I32, not {_name(positions.dtype)}")
+    if positions.dtype != I32:
+        raise ValueError(f"rope positions are I32, not {_name(positions.dtype)}")
     if rope.sections.code == 3:
         pairs = rope.sections.sizes
-        _require(len(pairs) <= 4 and all(p > 0 for p in pairs) and sum(pairs) * 2 == rope.rotaryDimensions,
-                 f"rope: axes of {list(pairs)} pairs for {rope.rotaryDimensions} rotary values")
+        if not (len(pairs) <= 4 and all(p > 0 for p in pairs) and sum(pairs) * 2 == rope.rotaryDimensions):
+            raise ValueError(f"rope: axes of {list(pairs)} pairs for {rope.rotaryDimensions} rotary values")
     count = rope.sections.positionsPerToken
     expected = (tokens,) if count == 1 else (count, tokens)
-    _require(tuple(positions.shape) == expected,
-             f"rope positions {_shape(positions)}, expected {_dims(expected)}")
-    _require(rope.rotaryDimensions % 2 == 0 and rope.rotaryDimensions <= dimension,
-             f"rope: {rope.rotaryDimensions} rotary dimensions in heads of {dimension}")
+    if tuple(positions.shape) != expected:
+        raise ValueError(f"rope positions {_shape(positions)}, expected {_dims(expected)}")
+    if not (rope.rotaryDimensions % 2 == 0 and rope.rotaryDimensions <= dimension):
+        raise ValueError(f"rope: {rope.rotaryDimensions} rotary dimensions in heads of {dimension}")
     return tokens, heads, dimension
 
 
@@ -347,63 +358,67 @@ def checkRopeTable(x, cosines, sines, out) -> tuple:
     """ops/AttentionOps.scala:129-151; returns (tokens, heads, D, pairs, perHead)."""
     checkElementwise("ropeTable", x, out)
     requireF32("ropeTable", cosines, sines)
-    _require(x.dim() == 3, f"ropeTable takes [tokens, heads, D], not {_shape(x)}")
+    if x.dim() != 3:
+        raise ValueError(f"ropeTable takes [tokens, heads, D], not {_shape(x)}")
     tokens, heads, d = x.shape
     pairs = cosines.shape[-1]
     per_head = cosines.dim() == 3
-    _require((tuple(cosines.shape) in ((tokens, pairs), (tokens, heads, pairs)))
-             and sines.shape == cosines.shape and 2 * pairs <= d,
-             f"ropeTable: tables {_shape(cosines)}, {_shape(sines)} for {_shape(x)}")
+    if not ((tuple(cosines.shape) in ((tokens, pairs), (tokens, heads, pairs)))
+            and sines.shape == cosines.shape and 2 * pairs <= d):
+        raise ValueError(f"ropeTable: tables {_shape(cosines)}, {_shape(sines)} for {_shape(x)}")
     return tokens, heads, d, pairs, per_head
 
 
 def checkEmbedding(table, ids, out) -> None:
     """ops/LinearOps.scala:92-106."""
     shape = table.shape
-    _require(len(shape) == 2, f"an embedding table is [vocabulary, D], not {list(shape)}")
-    _require(ids.dtype == I32 and ids.dim() == 1,
-             f"embedding ids are I32 [tokens], not {_name(ids.dtype)} {_shape(ids)}")
-    _require(out.dtype in _FLOAT_TYPES, f"embedding takes F32 or BF16, not {_name(out.dtype)}")
-    _require(tuple(out.shape) == (ids.shape[0], shape[-1]),
-             f"embedding: out {_shape(out)} for {ids.shape[0]} rows of {shape[-1]}")
+    if len(shape) != 2:
+        raise ValueError(f"an embedding table is [vocabulary, D], not {list(shape)}")
+    if not (ids.dtype == I32 and ids.dim() == 1):
+        raise ValueError(f"embedding ids are I32 [tokens], not {_name(ids.dtype)} {_shape(ids)}")
+    if out.dtype not in _FLOAT_TYPES:
+        raise ValueError(f"embedding takes F32 or BF16, not {_name(out.dtype)}")
+    if tuple(out.shape) != (ids.shape[0], shape[-1]):
+        raise ValueError(f"embedding: out {_shape(out)} for {ids.shape[0]} rows of {shape[-1]}")
 
 
 def checkRotated(codes, parts: ConvRotParts) -> RotatedTable:
     """Ops.checkRotated (ops/LinearOps.scala:121-157): the weight `codes`
     make with `parts`."""
-    _require(codes.dtype == torch.int8 and codes.dim() == 2,
-             f"rotated: {_name(codes.dtype)} codes {_shape(codes)}")
+    if not (codes.dtype == torch.int8 and codes.dim() == 2):
+        raise ValueError(f"rotated: {_name(codes.dtype)} codes {_shape(codes)}")
     n = codes.shape[0]
     k = codes.shape[1] * (1 if parts.levels is None else 2)
-    _require(k % CONVROT_GROUP == 0, f"rotated: rows of {k} columns")
+    if k % CONVROT_GROUP != 0:
+        raise ValueError(f"rotated: rows of {k} columns")
     scaleCount = parts.scales.numel()
-    _require(parts.scales.dtype == F32 and (scaleCount == n or scaleCount == 1 and parts.levels is None),
-             f"rotated: {scaleCount} {_name(parts.scales.dtype)} scales for {n} rows")
+    if not (parts.scales.dtype == F32 and (scaleCount == n or scaleCount == 1 and parts.levels is None)):
+        raise ValueError(f"rotated: {scaleCount} {_name(parts.scales.dtype)} scales for {n} rows")
     l = parts.levels
     if l is not None:
-        _require(l.groupSize > 0 and l.groupSize % 16 == 0 and k % l.groupSize == 0,
-                 f"rotated: {k} columns in groups of {l.groupSize}")
-        _require(l.codebook.dtype == F32 and l.codebook.numel() == 16,
-                 f"rotated: a codebook {_name(l.codebook.dtype)} {_shape(l.codebook)}")
-        _require(l.relative.dtype in (torch.uint8, torch.float8_e4m3fn) and
-                 tuple(l.relative.shape) == (n, k // l.groupSize),
-                 f"rotated: relative scales {_name(l.relative.dtype)} {_shape(l.relative)}")
+        if not (l.groupSize > 0 and l.groupSize % 16 == 0 and k % l.groupSize == 0):
+            raise ValueError(f"rotated: {k} columns in groups of {l.groupSize}")
+        if not (l.codebook.dtype == F32 and l.codebook.numel() == 16):
+            raise ValueError(f"rotated: a codebook {_name(l.codebook.dtype)} {_shape(l.codebook)}")
+        if not (l.relative.dtype in (torch.uint8, torch.float8_e4m3fn)
+                and tuple(l.relative.shape) == (n, k // l.groupSize)):
+            raise ValueError(f"rotated: relative scales {_name(l.relative.dtype)} {_shape(l.relative)}")
     return RotatedTable(codes, parts, k)
 
 
 def checkPageTable(pageTable, cache: KvCache, positions: int) -> None:
     """ops/AttentionOps.scala:243-256."""
-    _require(pageTable.dtype == I32 and pageTable.dim() == 1,
-             f"a page table is I32 [pages], not {_name(pageTable.dtype)} {_shape(pageTable)}")
-    _require(pageTable.numel() * cache.pageSize >= positions,
-             f"a page table of {pageTable.numel()} pages for {positions} positions")
+    if not (pageTable.dtype == I32 and pageTable.dim() == 1):
+        raise ValueError(f"a page table is I32 [pages], not {_name(pageTable.dtype)} {_shape(pageTable)}")
+    if pageTable.numel() * cache.pageSize < positions:
+        raise ValueError(f"a page table of {pageTable.numel()} pages for {positions} positions")
 
 
 def checkCacheWrite(k, v, cache: KvCache, pageTable, start: int) -> int:
     """ops/AttentionOps.scala:225-241; returns the token count."""
     checkElementwise("cacheWrite", k, v)
-    _require(k.dim() == 3 and tuple(k.shape[1:]) == (cache.kvHeads, cache.headDimension),
-             f"cacheWrite: {_shape(k)} into a cache of {cache.kvHeads} heads of {cache.headDimension}")
+    if not (k.dim() == 3 and tuple(k.shape[1:]) == (cache.kvHeads, cache.headDimension)):
+        raise ValueError(f"cacheWrite: {_shape(k)} into a cache of {cache.kvHeads} heads of {cache.headDimension}")
     tokens = int(k.shape[0])
     checkPageTable(pageTable, cache, start + tokens)
     return tokens
@@ -413,9 +428,10 @@ def checkSplitHalves(x, first, second) -> None:
     """ops/LayoutOps.scala:73-80 (F32, or BF16 here)."""
     checkElementwise("splitHalves", x)
     checkElementwise("splitHalves", first, second)
-    _require(x.dtype == first.dtype, f"splitHalves takes one type, not {_name(x.dtype)} and {_name(first.dtype)}")
-    _require(x.numel() == 2 * first.numel() and first.dim() >= 1 and x.shape[-1] == 2 * first.shape[-1],
-             f"splitHalves: {_shape(x)} into {_shape(first)}")
+    if x.dtype != first.dtype:
+        raise ValueError(f"splitHalves takes one type, not {_name(x.dtype)} and {_name(first.dtype)}")
+    if not (x.numel() == 2 * first.numel() and first.dim() >= 1 and x.shape[-1] == 2 * first.shape[-1]):
+        raise ValueError(f"splitHalves: {_shape(x)} into {_shape(first)}")
 
 
 # ops/HipBase.scala:268-274's codes (fp8 E4M3 bytes as uint8 or float8_e4m3fn)
@@ -428,18 +444,22 @@ def checkConvert(x, out) -> int:
     E4M3 to F32."""
     requireSameShape("convert", x, out)
     kind = _CONVERSIONS.get((x.dtype, out.dtype))
-    _require(kind is not None, f"convert: no conversion from {_name(x.dtype)} to {_name(out.dtype)}")
+    if kind is None:
+        raise ValueError(f"convert: no conversion from {_name(x.dtype)} to {_name(out.dtype)}")
     return kind
 
 
 def _on_device(operation: str, *tensors) -> None:
     for t in tensors:
-        _require(t.is_cuda, f"{operation}: tensors live in device memory")
-        _require(t.is_contiguous(), f"{operation}: tensors are dense row-major")
+        if not t.is_cuda:
+            raise ValueError(f"{operation}: tensors live in device memory")
+        if not t.is_contiguous():
+            raise ValueError(f"{operation}: tensors are dense row-major")
 
 
-def _ptr(t: Optional[torch.Tensor]):
-    return None if t is None else ctypes.c_void_p(t.data_ptr())
+def _ptr(t: Optional[torch.Tensor]) -> Optional[int]:
+    """t's device address, as a c_void_p argument takes it."""
+    return None if t is None else t.data_ptr()
 
 
 def _suffix(dtype) -> str:
@@ -471,9 +491,11 @@ class HipOps:
         self._quantizedBuffer: Optional[torch.Tensor] = None
         self._scratch: Optional[torch.Tensor] = None
 
-    def _stream(self):
-        s = self.stream if self.stream is not None else torch.cuda.current_stream()
-        return ctypes.c_void_p(s.cuda_stream)
+    def _stream(self) -> int:
+        if self.stream is not None:
+            return self.stream.cuda_stream
+        # torch.cuda.current_stream().cuda_stream without making the Stream (2.7 -> 0.6 us)
+        return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device())
 
     def _launch(self, entry: str, *args) -> None:
         self.deviceWrites += 1
@@ -529,8 +551,8 @@ class HipOps:
         run, so the norms quantize as they write from now on
         (ops/HipLinear.scala:366-386)."""
         self.quantizesX = True
-        _require(x.dtype in (F32, BF16) and (m * k) % 32 == 0 and x.numel() >= m * k,
-                 f"quantize: {m} rows of {k} from {_shape(x)}")
+        if not (x.dtype in (F32, BF16) and (m * k) % 32 == 0 and x.numel() >= m * k):
+            raise ValueError(f"quantize: {m} rows of {k} from {_shape(x)}")
         _on_device("quantize", x)
         blocks = m * k // 32
         size = m * k + 8 * blocks
@@ -583,7 +605,8 @@ class HipOps:
         of width values, row r weighted by weight row r % groups, with no
         int8 side output (ops/HipNormalisation.scala:133-158)."""
         rows = checkRowWise("groupRmsNorm", x, out, weight)
-        _require(groups > 0 and x.shape[-1] % groups == 0, f"{_shape(x)} in {groups} groups")
+        if not (groups > 0 and x.shape[-1] % groups == 0):
+            raise ValueError(f"{_shape(x)} in {groups} groups")
         _on_device("groupRmsNorm", x, weight, out)
         self._launch(f"drift_rms_norm_{_suffix(x.dtype)}", _ptr(x), None, _ptr(weight), _ptr(out), rows * groups,
                      x.shape[-1] // groups, epsilon, weightOffset, groups, None, None, None)
@@ -619,10 +642,11 @@ class HipOps:
             requireF32("gatedAdd", gate)
             cols = x.shape[-1]
             rows = x.numel() // cols if cols else 0
-            _require(rowsPerSample is not None and rowsPerSample > 0, "gatedAdd: per-sample gates need rowsPerSample")
+            if not (rowsPerSample is not None and rowsPerSample > 0):
+                raise ValueError("gatedAdd: per-sample gates need rowsPerSample")
             samples = -(-rows // rowsPerSample)
-            _require(gate.dim() == 2 and tuple(gate.shape) == (samples, cols),
-                     f"gatedAdd: {_shape(gate)} for {samples} samples of rows of {cols}")
+            if not (gate.dim() == 2 and tuple(gate.shape) == (samples, cols)):
+                raise ValueError(f"gatedAdd: {_shape(gate)} for {samples} samples of rows of {cols}")
             per = rowsPerSample
         _on_device("gatedAdd", x, y, gate)
         self._launch(f"drift_gated_add_{_suffix(x.dtype)}", _ptr(x), _ptr(y), _ptr(gate), rows, x.shape[-1], per)
@@ -656,15 +680,16 @@ class HipOps:
         over that sample's rows (models/Wan.scala:431-432). x, out [rows, C]."""
         checkElementwise("layerNormModulate", x, out)
         requireF32("layerNormModulate", scale, shift)
-        _require(x.dim() == 2, f"layerNormModulate takes [rows, C], not {_shape(x)}")
+        if x.dim() != 2:
+            raise ValueError(f"layerNormModulate takes [rows, C], not {_shape(x)}")
         rows, cols = x.shape
         scale2 = scale.reshape(-1, cols) if scale.dim() == 1 else scale
-        _require(scale2.dim() == 2 and scale2.shape[1] == cols and tuple(shift.shape) == tuple(scale.shape),
-                 f"layerNormModulate: scale {_shape(scale)}, shift {_shape(shift)} for rows of {cols}")
+        if not (scale2.dim() == 2 and scale2.shape[1] == cols and tuple(shift.shape) == tuple(scale.shape)):
+            raise ValueError(f"layerNormModulate: scale {_shape(scale)}, shift {_shape(shift)} for rows of {cols}")
         samples = scale2.shape[0]
         per = rowsPerSample if rowsPerSample is not None else -(-rows // samples)
-        _require(per > 0 and samples * per >= rows,
-                 f"layerNormModulate: {samples} samples of {per} rows for {rows} rows")
+        if not (per > 0 and samples * per >= rows):
+            raise ValueError(f"layerNormModulate: {samples} samples of {per} rows for {rows} rows")
         _on_device("layerNormModulate", x, scale, shift, out)
         self._launch(f"drift_layer_norm_modulate_{_suffix(x.dtype)}", _ptr(x), _ptr(scale), _ptr(shift), _ptr(out),
                      rows, cols, per, epsilon)
@@ -713,7 +738,8 @@ class HipOps:
         `frames x rows x columns` grid; token i of x is grid token
         (tokenOffset + i) mod (frames * rows * columns)."""
         checkElementwise("rope3d", x, out)
-        _require(x.dim() == 3, f"rope3d takes [tokens, heads, D], not {_shape(x)}")
+        if x.dim() != 3:
+            raise ValueError(f"rope3d takes [tokens, heads, D], not {_shape(x)}")
         _on_device("rope3d", x, out)
         tokens, heads, d = x.shape
         self._launch(f"drift_rope_3d_{_suffix(x.dtype)}", _ptr(x), _ptr(out), tokens, heads, d, frames, rows,
@@ -725,15 +751,17 @@ class HipOps:
         rmsNorm, rmsNorm, rope, rope. q [t, heads, D], k [t, kvHeads, D]."""
         checkElementwise("queryKeyNormRope", q, rotatedQueries)
         checkElementwise("queryKeyNormRope", k, rotatedKeys)
-        _require(q.dtype == k.dtype, "queryKeyNormRope takes one type for queries and keys")
-        _require(q.dim() == 3 and k.dim() == 3 and q.shape[0] == k.shape[0] and q.shape[2] == k.shape[2],
-                 f"queryKeyNormRope: queries {_shape(q)}, keys {_shape(k)}")
+        if q.dtype != k.dtype:
+            raise ValueError("queryKeyNormRope takes one type for queries and keys")
+        if not (q.dim() == 3 and k.dim() == 3 and q.shape[0] == k.shape[0] and q.shape[2] == k.shape[2]):
+            raise ValueError(f"queryKeyNormRope: queries {_shape(q)}, keys {_shape(k)}")
         tokens, heads, d = q.shape
         kv = k.shape[1]
         checkRope(q, positions, norms.rope, rotatedQueries)
         for name, w in (("queryNorm", norms.queryNorm), ("keyNorm", norms.keyNorm)):
             requireF32("queryKeyNormRope", w)
-            _require(tuple(w.shape) == (d,), f"queryKeyNormRope: {name} {_shape(w)} for heads of {d}")
+            if tuple(w.shape) != (d,):
+                raise ValueError(f"queryKeyNormRope: {name} {_shape(w)} for heads of {d}")
         _on_device("queryKeyNormRope", q, k, rotatedQueries, rotatedKeys, norms.queryNorm, norms.keyNorm, positions)
         r = norms.rope
         self._launch(f"drift_qk_norm_rope_{_suffix(q.dtype)}", _ptr(q), _ptr(k), _ptr(rotatedQueries),
@@ -776,8 +804,8 @@ class HipOps:
         `rotatedKeys` are the unfused steps' scratch, checked and not written,
         as the reference's fused launch leaves them."""
         t, heads, d = (int(n) for n in queries.shape) if queries.dim() == 3 else (0, 0, 0)
-        _require(d <= self.AttentionInputDimension,
-                 f"attentionInputs: heads of {d} values (at most {self.AttentionInputDimension} fused)")
+        if d > self.AttentionInputDimension:
+            raise ValueError(f"attentionInputs: heads of {d} values (at most {self.AttentionInputDimension} fused)")
         checkSplitHalves(queryAndGate, queries, gate)
         checkRope(queries, positions, norms.rope, rotatedQueries)
         checkRope(keys, positions, norms.rope, rotatedKeys)
@@ -792,8 +820,8 @@ class HipOps:
         queries into `rotatedQueries` and the keys, with the values v, into
         the cache at `start` (models/DenseDecoder.scala:834-863 runs rmsNorm,
         rmsNorm, rope, rope, cacheWrite)."""
-        _require(q.dim() == 3 and q.shape[2] <= self.AttentionInputDimension,
-                 f"queryKeyNormRopeCache: queries {_shape(q)}")
+        if not (q.dim() == 3 and q.shape[2] <= self.AttentionInputDimension):
+            raise ValueError(f"queryKeyNormRopeCache: queries {_shape(q)}")
         checkRope(q, positions, norms.rope, rotatedQueries)
         checkRope(k, positions, norms.rope, k)
         checkCacheWrite(k, v, cache, pageTable, start)
@@ -802,14 +830,15 @@ class HipOps:
     def _attentionInputs(self, queryAndGate, keys, values, norms, positions, cache, pageTable, start, gate,
                          rotatedQueries, badPage) -> None:
         tokens, heads, d = (int(n) for n in rotatedQueries.shape)
-        _require(tuple(keys.shape) == (tokens, cache.kvHeads, d),
-                 f"attentionInputs: keys {_shape(keys)} for {tokens} tokens of heads of {d}")
-        _require(queryAndGate.dtype == keys.dtype == values.dtype == rotatedQueries.dtype and
-                 (gate is None or gate.dtype == keys.dtype),
-                 "attentionInputs takes one type for queries, gate, keys and values")
+        if tuple(keys.shape) != (tokens, cache.kvHeads, d):
+            raise ValueError(f"attentionInputs: keys {_shape(keys)} for {tokens} tokens of heads of {d}")
+        if not (queryAndGate.dtype == keys.dtype == values.dtype == rotatedQueries.dtype and (gate is None
+                or gate.dtype == keys.dtype)):
+            raise ValueError("attentionInputs takes one type for queries, gate, keys and values")
         for name, w in (("queryNorm", norms.queryNorm), ("keyNorm", norms.keyNorm)):
             requireF32("attentionInputs", w)
-            _require(tuple(w.shape) == (d,), f"attentionInputs: {name} {_shape(w)} for heads of {d}")
+            if tuple(w.shape) != (d,):
+                raise ValueError(f"attentionInputs: {name} {_shape(w)} for heads of {d}")
         tensors = [queryAndGate, keys, values, norms.queryNorm, norms.keyNorm, positions, cache.keys, cache.values,
                    pageTable, rotatedQueries] + ([] if gate is None else [gate])
         _on_device("attentionInputs", *tensors)
@@ -834,8 +863,8 @@ class HipOps:
             self._rotated(f"drift_rotated_embedding_{_suffix(out.dtype)}", table, out, ids, badId)
             return
         t = self._checkStored("embedding", table)
-        _require(table.cols % 8 == 0 or t.values == 1,
-                 f"embedding: rows of {table.cols} values (quant kernels take multiples of 8)")
+        if not (table.cols % 8 == 0 or t.values == 1):
+            raise ValueError(f"embedding: rows of {table.cols} values (quant kernels take multiples of 8)")
         _on_device("embedding", table.data, ids, out)
         vocab, cols = table.shape
         if t.name == "Q8_0":
@@ -855,9 +884,9 @@ class HipOps:
     def _rotated(self, entry: str, table: RotatedTable, out, ids=None, badId=None) -> None:
         table = checkRotated(table.codes, table.parts)
         p, l = table.parts, table.parts.levels
-        _require(table.codes.is_contiguous() and p.scales.is_contiguous() and
-                 (l is None or l.codebook.is_contiguous() and l.relative.is_contiguous()),
-                 f"{entry}: codes, scales and levels must be contiguous")
+        if not (table.codes.is_contiguous() and p.scales.is_contiguous() and (l is None
+                or l.codebook.is_contiguous() and l.relative.is_contiguous())):
+            raise ValueError(f"{entry}: codes, scales and levels must be contiguous")
         tensors = [table.codes, p.scales, out] + ([] if l is None else [l.codebook, l.relative]) + \
             ([] if ids is None else [ids])
         _on_device(entry, *tensors)
@@ -874,28 +903,35 @@ class HipOps:
         the GEMM path (kernels/matvec.hip:801-827 dequantize, dequantize_bf16);
         a RotatedTable to BF16 (ops/HipBase.scala:276-311)."""
         if isinstance(table, RotatedTable):
-            _require(out.dtype == BF16, f"convert: no conversion from {table.dtype} to {_name(out.dtype)}")
-            _require(tuple(out.shape) == table.shape, f"convert: out {_shape(out)} for {_dims(table.shape)}")
+            if out.dtype != BF16:
+                raise ValueError(f"convert: no conversion from {table.dtype} to {_name(out.dtype)}")
+            if tuple(out.shape) != table.shape:
+                raise ValueError(f"convert: out {_shape(out)} for {_dims(table.shape)}")
             self._rotated("drift_rotated_dequantize_bf16", table, out)
             return
         t = self._checkStored("dequantize", table)
-        _require(out.dtype in (BF16, F16), f"dequantize writes BF16 or F16, not {_name(out.dtype)}")
-        _require(tuple(out.shape) == table.shape, f"dequantize: out {_shape(out)} for a table {_dims(table.shape)}")
-        _require(table.cols % 8 == 0 or t.values == 1,
-                 f"dequantize: rows of {table.cols} values (quant kernels take multiples of 8)")
+        if out.dtype not in (BF16, F16):
+            raise ValueError(f"dequantize writes BF16 or F16, not {_name(out.dtype)}")
+        if tuple(out.shape) != table.shape:
+            raise ValueError(f"dequantize: out {_shape(out)} for a table {_dims(table.shape)}")
+        if not (table.cols % 8 == 0 or t.values == 1):
+            raise ValueError(f"dequantize: rows of {table.cols} values (quant kernels take multiples of 8)")
         _on_device("dequantize", table.data, out)
         entry = "drift_dequantize_bf16" if out.dtype == BF16 else "drift_dequantize_f16"
         self._launch(entry, _ptr(table.data), t.ggmlId, _ptr(out), table.shape[0], table.cols)
 
     @staticmethod
     def _checkStored(operation: str, table: StoredTable) -> StorageType:
-        _require(isinstance(table, StoredTable), f"{operation}: a table of stored bytes")
+        if not isinstance(table, StoredTable):
+            raise ValueError(f"{operation}: a table of stored bytes")
         t = table.dtype
         vocab, cols = table.shape
-        _require(cols % t.values == 0, f"{cols} elements are not whole {t.name} blocks of {t.values}")
-        _require(table.data.dtype == torch.uint8 and tuple(table.data.shape) == (vocab, t.rowBytes(cols)),
-                 f"{operation}: {t.name} bytes {_shape(table.data)} for rows of {cols}")
-        _require(table.data.is_contiguous(), f"{operation}: {t.name} bytes must be contiguous rows")
+        if cols % t.values != 0:
+            raise ValueError(f"{cols} elements are not whole {t.name} blocks of {t.values}")
+        if not (table.data.dtype == torch.uint8 and tuple(table.data.shape) == (vocab, t.rowBytes(cols))):
+            raise ValueError(f"{operation}: {t.name} bytes {_shape(table.data)} for rows of {cols}")
+        if not table.data.is_contiguous():
+            raise ValueError(f"{operation}: {t.name} bytes must be contiguous rows")
         return t
 
     def convert(self, x, out) -> None:
