@@ -692,7 +692,7 @@ int qk_launch(const char* entry, const T* q, const T* k, T* q_out, T* k_out, con
   const bool whole = p.rotary > 0 && p.rotary % (p.layout == DRIFT_ROPE_NEOX ? 2 * N : N) == 0 && dim % (2 * N) == 0 &&
                      (lanes_per_head & (lanes_per_head - 1)) == 0 && lanes_per_head <= kWave / 2 && aligned;
   // the general kernel takes any number of tokens
-  if (!whole || (mixed && blocks > INT32_MAX)) {
+  if (!whole || (mixed && blocks > kOneWaveBlocks)) {
     hipLaunchKernelGGL((qk_norm_rope_kernel<T, EXTRAS>), dim3(grid_for(p.tokens, 1, 1 << 16)), dim3(256), 0, st, q,
                        k, q_out, k_out, q_weight, k_weight, positions, a, e);
     return launched(entry);
@@ -837,7 +837,7 @@ int cache_write(const char* entry, const T* k, const T* v, uint16_t* keys, uint1
   const int64_t blocks = et.tiles + ceil_div(tokens * runs, kWave);
   constexpr int N = Chunk<T>::N;
   if (dim % 8 == 0 && tokens * runs > kTiledRuns && aligned16(k) && aligned16(v) && aligned16(keys) &&
-      aligned16(values) && runs * 8 <= INT32_MAX && blocks <= kOneShotBlocks)
+      aligned16(values) && runs * 8 <= INT32_MAX && blocks <= kOneWaveBlocks)
     hipLaunchKernelGGL(cache_write_tiles<T>, dim3((unsigned)blocks), dim3(kWave), 0, st, k, et, (int64_t)tokens,
                        (int)runs, 1.0 / (double)runs);
   else if (dim % N == 0 && aligned16(k) && aligned16(v) && aligned16(keys))

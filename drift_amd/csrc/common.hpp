@@ -295,6 +295,10 @@ inline int64_t ceil_div(int64_t a, int64_t b) { return (a + b - 1) / b; }
 // grid-stride loop that runs once below this many blocks.
 constexpr int64_t kOneShotBlocks = (int64_t)1 << 30;
 
+// One-wave blocks a launch can have (less one wave): a dimension's threads
+// number below 2^32.
+constexpr int64_t kOneWaveBlocks = ((int64_t)1 << 26) - 1;
+
 // Workgroups for a grid-stride launch: enough to fill the chip many times
 // over, never more than the grid allows.
 inline unsigned grid_for(int64_t items, int per_block, int64_t cap = 1 << 20) {

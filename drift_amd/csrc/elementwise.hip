@@ -245,20 +245,59 @@ __global__ void __launch_bounds__(256) convert_kernel(const void* x, void* out, 
   }
 }
 
-// 8 values per thread for the F32 <-> BF16 pairs.
-__global__ void __launch_bounds__(256) convert_bf16_chunks(const void* x, void* out, int64_t chunks, int kind) {
-  const int64_t stride = (int64_t)gridDim.x * blockDim.x;
-  for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < chunks; i += stride) {
-    float v[8];
-    if (kind == DRIFT_F32_TO_BF16) {
-      Chunk<float>::load(static_cast<const float*>(x) + i * 8, *reinterpret_cast<float(*)[4]>(v));
-      Chunk<float>::load(static_cast<const float*>(x) + i * 8 + 4, *reinterpret_cast<float(*)[4]>(v + 4));
-      Chunk<uint16_t>::store(static_cast<uint16_t*>(out) + i * 8, v);
-    } else {
-      Chunk<uint16_t>::load(static_cast<const uint16_t*>(x) + i * 8, v);
-      Chunk<float>::store(static_cast<float*>(out) + i * 8, *reinterpret_cast<float(*)[4]>(v));
-      Chunk<float>::store(static_cast<float*>(out) + i * 8 + 4, *reinterpret_cast<float(*)[4]>(v + 4));
+// F32 <-> BF16 in one-wave blocks, 64 chunks of 8 values each, every load and
+// store instruction covering whole consecutive lines: the F32 side moves as
+// two runs of 64 16-byte quarters, the BF16 side as 16-byte chunks of which
+// even lanes hold the first 32 and odd lanes the other 32, and the lanes of a
+// pair trade the halves the other needs by DPP. A lane moving its own 32
+// bytes of F32 reads or writes half of each line an instruction. Memory bounds
+// it: [65520, 3072] to BF16 (1.2 GB) 217.8 -> 177.6 us (6.8 TB/s), [7800,
+// 3072] to F32 29.0 -> 23.6, against 8 values a lane in a resident grid; that
+// in one pass took 192.3 and 30.0, in one-wave blocks 193.3 and 27.6.
+template <bool TO_BF16>
+__global__ void __launch_bounds__(kWave) convert_bf16_waves(const void* x, void* out, int64_t chunks) {
+  const int lane = threadIdx.x;
+  const int64_t first = (int64_t)blockIdx.x * kWave;
+  const float* xf = static_cast<const float*>(x) + first * 8;
+  const uint16_t* xb = static_cast<const uint16_t*>(x) + first * 8;
+  float* of = static_cast<float*>(out) + first * 8;
+  uint16_t* ob = static_cast<uint16_t*>(out) + first * 8;
+  if (first + kWave > chunks) {  // the last wave, part full
+    if (first + lane < chunks) {
+      float v[8];
+      if constexpr (TO_BF16) {
+        Chunk<float>::load(xf + lane * 8, *reinterpret_cast<float(*)[4]>(v));
+        Chunk<float>::load(xf + lane * 8 + 4, *reinterpret_cast<float(*)[4]>(v + 4));
+        Chunk<uint16_t>::store(ob + lane * 8, v);
+      } else {
+        Chunk<uint16_t>::load(xb + lane * 8, v);
+        Chunk<float>::store(of + lane * 8, *reinterpret_cast<float(*)[4]>(v));
+        Chunk<float>::store(of + lane * 8 + 4, *reinterpret_cast<float(*)[4]>(v + 4));
+      }
     }
+    return;
+  }
+  const bool odd = lane & 1;
+  const int chunk = lane / 2 + (odd ? kWave / 2 : 0);  // the lane's BF16 chunk
+  if constexpr (TO_BF16) {
+    float lo[4], hi[4];  // quarter `lane` of each run: half of chunk lane / 2, and of chunk 32 + lane / 2
+    Chunk<float>::load(xf + lane * 4, lo);
+    Chunk<float>::load(xf + 4 * kWave + lane * 4, hi);
+    const uint32_t a0 = pack_bf16(lo[0], lo[1]), a1 = pack_bf16(lo[2], lo[3]);
+    const uint32_t b0 = pack_bf16(hi[0], hi[1]), b1 = pack_bf16(hi[2], hi[3]);
+    const uint32_t r0 = (uint32_t)dpp_move32<0xb1>((int)(odd ? a0 : b0));
+    const uint32_t r1 = (uint32_t)dpp_move32<0xb1>((int)(odd ? a1 : b1));
+    const u32x4 q = odd ? u32x4{r0, r1, b0, b1} : u32x4{a0, a1, r0, r1};
+    __builtin_nontemporal_store(q, reinterpret_cast<u32x4*>(ob + chunk * 8));
+  } else {
+    const uint4 q = stream_load(xb + chunk * 8);
+    const uint32_t r0 = (uint32_t)dpp_move32<0xb1>((int)(odd ? q.x : q.z));
+    const uint32_t r1 = (uint32_t)dpp_move32<0xb1>((int)(odd ? q.y : q.w));
+    const uint32_t a0 = odd ? r0 : q.x, a1 = odd ? r1 : q.y, b0 = odd ? q.z : r0, b1 = odd ? q.w : r1;
+    const float lo[4] = {bf16_lo(a0), bf16_hi(a0), bf16_lo(a1), bf16_hi(a1)};
+    const float hi[4] = {bf16_lo(b0), bf16_hi(b0), bf16_lo(b1), bf16_hi(b1)};
+    Chunk<float>::store(of + lane * 4, lo);
+    Chunk<float>::store(of + 4 * kWave + lane * 4, hi);
   }
 }
 
@@ -281,6 +320,10 @@ int activation(const char* entry, const T* x, T* out, int64_t n, int32_t kind, f
         break;
       case DRIFT_GELU_TANH:
         hipLaunchKernelGGL((activation_kernel<T, DRIFT_GELU_TANH>), dim3(grid), dim3(kWave), 0, s, x, out, n, kind,
+                           scale);
+        break;
+      case DRIFT_GELU_ERF:  // F32 [4830, 5120] 39.1 us with the kind an argument, 37.6 so
+        hipLaunchKernelGGL((activation_kernel<T, DRIFT_GELU_ERF>), dim3(grid), dim3(kWave), 0, s, x, out, n, kind,
                            scale);
         break;
       default:
@@ -361,9 +404,14 @@ extern "C" int drift_convert(const void* x, void* out, int64_t n, int32_t kind, 
   if (x == out) return refuse("%s: x and out are the same buffer of different types", entry);
   const hipStream_t s = (hipStream_t)stream;
   const bool bf16 = kind == DRIFT_F32_TO_BF16 || kind == DRIFT_BF16_TO_F32;
-  if (bf16 && n % 8 == 0 && aligned16(x) && aligned16(out))
-    hipLaunchKernelGGL(convert_bf16_chunks, dim3(grid_for(n / 8, 256, 8192)), dim3(256), 0, s, x, out, n / 8, kind);
-  else
+  if (bf16 && n % 8 == 0 && aligned16(x) && aligned16(out) && ceil_div(n / 8, kWave) <= kOneWaveBlocks) {
+    const dim3 grid((unsigned)ceil_div(n / 8, kWave)), block(kWave);
+    if (kind == DRIFT_F32_TO_BF16)
+      hipLaunchKernelGGL(convert_bf16_waves<true>, grid, block, 0, s, x, out, n / 8);
+    else
+      hipLaunchKernelGGL(convert_bf16_waves<false>, grid, block, 0, s, x, out, n / 8);
+  } else {
     hipLaunchKernelGGL(convert_kernel, dim3(grid_for(n, 256, 8192)), dim3(256), 0, s, x, out, n, kind);
+  }
   return launched(entry);
 }

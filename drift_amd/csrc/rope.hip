@@ -458,7 +458,7 @@ int rope(const char* entry, const T* x, const int32_t* positions, T* out, int32_
   const int64_t fit = std::min<int64_t>(per_lane * kWave / items, rotary > 0 ? kMaxPairs / (rotary / 2) : kMaxPairs);
   const int64_t per_wave = std::max<int64_t>(1, std::min<int64_t>(fit, tokens));
   const int64_t blocks = ceil_div(tokens, per_wave) * runs;
-  if (chunked && blocks <= kOneShotBlocks) {
+  if (chunked && blocks <= kOneWaveBlocks) {
     const dim3 grid((unsigned)blocks), block(kWave);
     const uint32_t slots_inverse = slots == 1 ? 0 : (uint32_t)ceil_div((int64_t)1 << 32, slots);
 #define DRIFT_ROPE_LAUNCH(NEOX, K, TOKENS)                                                                       \
@@ -506,7 +506,7 @@ int rope_table(const char* entry, const T* x, const float* cosines, const float*
   // 16 waves a CU of one; else two (rope_table_chunks' comment)
   const int per_lane = halves || tokens * ceil_div(items, kWave) <= 4096 ? 1 : 2;
   const int64_t runs = ceil_div(items, per_lane * kWave);
-  if (chunked && tokens * runs <= kOneShotBlocks) {
+  if (chunked && tokens * runs <= kOneWaveBlocks) {
     const dim3 grid((unsigned)(tokens * runs)), block(kWave);
 #define DRIFT_TABLE_LAUNCH(K, HALVES, PER_HEAD)                                                               \
   hipLaunchKernelGGL((rope_table_chunks<T, K, HALVES, PER_HEAD>), grid, block, 0, st, x, cosines, sines, out, \

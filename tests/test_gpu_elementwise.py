@@ -138,6 +138,23 @@ def test_convert_round_trips(hip):
     assert_bits(o.to_bf16(odd), host_bits(bo), what="odd length")
 
 
+@pytest.mark.parametrize("n", [8, 504, 512, 520, 1016, 65536, 3 * 512 + 256])
+def test_convert_waves(hip, n):
+    # a wave takes 512 values: less than one, whole ones, a part-full last one
+    step(f"convert {n} values")
+    f = gaussian(61, n, 5.0)
+    f[:4] = [np.inf, -np.inf, 0.0, -0.0]
+    f[4] = np.nan
+    padded = torch.full((n + 8,), -3, dtype=torch.bfloat16, device=DEV)
+    hip.convert(dev_f32(f), padded[:n])
+    assert_bits(o.to_bf16(f), host_bits(padded[:n]), what="to bf16")
+    assert bool((padded[n:] == -3).all()), "nothing past the end"
+    back = torch.full((n + 8,), -3, dtype=torch.float32, device=DEV)
+    hip.convert(dev_bf16(o.to_bf16(f)), back[:n])
+    assert np.array_equal(o.from_bf16(o.to_bf16(f)).view(np.uint32), host_f32(back[:n]).view(np.uint32)), "to F32"
+    assert bool((back[n:] == -3).all()), "nothing past the end"
+
+
 def test_convert_fp8_e4m3_to_f32(hip):
     # the reference's conversion code 4 (ops/HipBase.scala:268-274): every
     # E4M3 "fn" byte, as uint8 or torch's float8_e4m3fn, against the
