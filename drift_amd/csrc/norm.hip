@@ -67,7 +67,7 @@ __device__ __forceinline__ double chunk_squares(const float (&v)[N]) {
 }
 
 // 1 / sqrt(squares / cols + eps), the same in every kernel here.
-__device__ __forceinline__ double rms_factor(double squares, int cols, float eps) {
+__device__ __forceinline__ double row_factor(double squares, int cols, float eps) {
   const double mean = squares / (double)cols + (double)eps;
   return eps > 0.0f ? inverse_sqrt<true>(mean) : inverse_sqrt(mean);
 }
@@ -116,7 +116,7 @@ __global__ void __launch_bounds__(256) rms_norm_rows(T* x, const T* y, const flo
       }
     }
     squares = row_sum<W>(squares, partial);
-    const double factor = rms_factor(squares, cols, eps);
+    const double factor = row_factor(squares, cols, eps);
 #pragma unroll
     for (int k = 0; k < K; ++k) {
       const int c = (k * W + sub) * kWave + lane;
@@ -212,7 +212,7 @@ __global__ void __launch_bounds__(kWave) rms_norm_waves(T* x, const T* y, const 
     }
 #pragma unroll
     for (int i = 0; i < kSums; ++i) sums[i] = group_sum<64>(sums[i]);
-    const double factor = rms_factor(((sums[0] + sums[1]) + sums[2]) + sums[3], cols, eps);
+    const double factor = row_factor(((sums[0] + sums[1]) + sums[2]) + sums[3], cols, eps);
 #pragma unroll
     for (int k = 0; k < K; ++k) {
       const int c = k * kWave + lane;
@@ -276,7 +276,7 @@ __global__ void __launch_bounds__(kWave) rms_norm_groups(const T* x, const float
     Chunk<T>::unpack(raw[u], v);
     double squares = chunk_squares(v);
     if (!inside) squares = 0.0;
-    const double factor = rms_factor(group_sum<G>(squares), cols, eps);
+    const double factor = row_factor(group_sum<G>(squares), cols, eps);
     const int64_t row = first + u * kRows;
 #pragma unroll
     for (int j = 0; j < N; ++j) o[j] = (float)((double)v[j] * factor * ((double)w[j] + (double)offset));
@@ -337,7 +337,7 @@ __global__ void __launch_bounds__(64 * W) rms_norm_wide(T* x, const T* y, const 
     }
     __syncthreads();
     const double total = ((partial[0] + partial[1]) + partial[2]) + partial[3];
-    const double factor = rms_factor(total, cols, eps);
+    const double factor = row_factor(total, cols, eps);
 #pragma unroll
     for (int k = 0; k < K; ++k) {
       const int c = (k * W + wave) * kWave + lane;
@@ -373,7 +373,7 @@ __global__ void __launch_bounds__(256) rms_norm_rows_scalar(T* x, const T* y, co
       squares += (double)v * (double)v;
     }
     squares = row_sum<4>(squares, partial);
-    const double factor = rms_factor(squares, cols, eps);
+    const double factor = row_factor(squares, cols, eps);
     const float* w = weight + (row % weight_rows) * cols;
     for (int c = threadIdx.x; c < cols; c += 256) {
       float v = load_one(xr + c);
@@ -409,7 +409,7 @@ __global__ void __launch_bounds__(256) rms_norm_narrow(T* x, const T* y, const f
         squares += (double)v[c] * (double)v[c];
       }
     }
-    const double factor = rms_factor(squares, cols, eps);
+    const double factor = row_factor(squares, cols, eps);
     const float* w = weight + (row % weight_rows) * cols;
 #pragma unroll
     for (int c = 0; c < kNarrowCols; ++c) {
@@ -457,11 +457,11 @@ __global__ void __launch_bounds__(256) layer_norm_rows(const T* x, const float* 
 #pragma unroll
         for (int j = 0; j < N; ++j) {
           const double d = (double)v[k][j] - mean;
-          squares += d * d;
+          squares = fma(d, d, squares);
         }
       }
     }
-    const double factor = 1.0 / sqrt(row_sum<W>(squares, partial) / (double)cols + (double)eps);
+    const double factor = row_factor(row_sum<W>(squares, partial), cols, eps);
     const float* s0 = weight;  // MODULATE: the sample's scale row
     const float* s1 = bias;    // MODULATE: the sample's shift row
     if constexpr (MODULATE) {
@@ -499,6 +499,75 @@ __global__ void __launch_bounds__(256) layer_norm_rows(const T* x, const float* 
   }
 }
 
+// LayerNorm of many rows of four waves' chunks: a wave a row in one-wave
+// blocks, so a row waits on no barrier (the four-wave group has four). Its
+// sums are taken in the four-wave group's order, chunk k's in sum k % 4. The
+// weights and biases are read after the sums: read first, their registers (as
+// doubles) held half as many waves. Measured, us a launch in graph replays,
+// four-wave group / weights first / this: [4087, 1152] (38 MB) 12.6 / 8.9 /
+// 8.4, [4830, 1280] 14.9 / 12.7 / 9.8, [9000, 1024] 19.1 / 18.1 / 15.5; [600,
+// 1152] 4.2 / 4.4 / 4.5, so up to 1,024 rows keep the group.
+template <int K>
+__global__ void __launch_bounds__(kWave) layer_norm_waves(const float* x, const float* weight, const float* bias,
+                                                          float* out, int64_t rows, int cols, float eps) {
+  constexpr int N = 4;
+  const int lane = threadIdx.x;
+  const int chunks = cols / N;
+  const int64_t row = blockIdx.x;
+  uint4 raw[K];
+#pragma unroll
+  for (int k = 0; k < K; ++k) raw[k] = stream_load(x + row * cols + min(k * kWave + lane, chunks - 1) * N);
+  constexpr int kSums = K < 4 ? K : 4;
+  double sums[4] = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+  for (int k = 0; k < K; ++k) {
+    float v[N];
+    Chunk<float>::unpack(raw[k], v);
+    if (k * kWave + lane < chunks) {
+#pragma unroll
+      for (int j = 0; j < N; ++j) sums[k % 4] += (double)v[j];
+    }
+  }
+#pragma unroll
+  for (int i = 0; i < kSums; ++i) sums[i] = group_sum<64>(sums[i]);
+  const double mean = (((sums[0] + sums[1]) + sums[2]) + sums[3]) / (double)cols;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) sums[i] = 0.0;
+#pragma unroll
+  for (int k = 0; k < K; ++k) {
+    opaque(raw[k]);
+    float v[N];
+    Chunk<float>::unpack(raw[k], v);
+    if (k * kWave + lane < chunks) {
+#pragma unroll
+      for (int j = 0; j < N; ++j) {
+        const double d = (double)v[j] - mean;
+        sums[k % 4] = fma(d, d, sums[k % 4]);
+      }
+    }
+  }
+#pragma unroll
+  for (int i = 0; i < kSums; ++i) sums[i] = group_sum<64>(sums[i]);
+  const double factor = row_factor(((sums[0] + sums[1]) + sums[2]) + sums[3], cols, eps);
+#pragma unroll
+  for (int k = 0; k < K; ++k) {
+    const int c = k * kWave + lane;
+    if (c < chunks) {
+      opaque(raw[k]);
+      float v[N], w[N], b[N], o[N];
+      Chunk<float>::unpack(raw[k], v);
+      if (weight) load_f32<N>(weight + c * N, w);
+      if (bias) load_f32<N>(bias + c * N, b);
+#pragma unroll
+      for (int j = 0; j < N; ++j) {
+        const double normal = ((double)v[j] - mean) * factor;
+        o[j] = (float)(normal * (weight ? (double)w[j] : 1.0) + (bias ? (double)b[j] : 0.0));
+      }
+      Chunk<float>::store(out + row * cols + c * N, o);
+    }
+  }
+}
+
 template <typename T, bool MODULATE>
 __global__ void __launch_bounds__(256) layer_norm_rows_scalar(const T* x, const float* weight, const float* bias,
                                                               T* out, int64_t rows, int cols,
@@ -512,9 +581,9 @@ __global__ void __launch_bounds__(256) layer_norm_rows_scalar(const T* x, const 
     double squares = 0.0;
     for (int c = threadIdx.x; c < cols; c += 256) {
       const double d = (double)load_one(xr + c) - mean;
-      squares += d * d;
+      squares = fma(d, d, squares);
     }
-    const double factor = 1.0 / sqrt(row_sum<4>(squares, partial) / (double)cols + (double)eps);
+    const double factor = row_factor(row_sum<4>(squares, partial), cols, eps);
     const float* s0 = weight;
     const float* s1 = bias;
     if constexpr (MODULATE) {
@@ -536,8 +605,13 @@ __global__ void __launch_bounds__(256) layer_norm_rows_scalar(const T* x, const 
   }
 }
 
-// F32 AdaLN, one wave per row, four rows of one sample per block (grid.y =
-// sample), the grid covering the rows in one pass. Each lane reads its
+// AdaLN, one wave per row, B / 64 rows of one sample per block (grid.y =
+// sample), the grid covering the rows in one pass: F32 rows, in one-wave
+// blocks, and BF16 rows past adaln_resident's registers, in 256-thread blocks
+// ([16380, 5120] 73.7 us, one-wave blocks 77.4, layer_norm_rows 99.2). F32, us
+// a launch in graph replays, 256-thread / one-wave blocks: [1500, 3840] 14.4 /
+// 9.5, [7800, 3072] 36.9 / 37.6, [8190, 1536] 19.2 / 18.6; [4000, 5120] 44.0
+// in layer_norm_rows, 28.1. Each lane reads its
 // chunks' scale and shift from the sample's rows (cached: every row of the
 // sample reads them).
 //
@@ -547,17 +621,17 @@ __global__ void __launch_bounds__(256) layer_norm_rows_scalar(const T* x, const 
 // most. The arithmetic is the reference's, in double: n = float((x - mean) *
 // factor) is layerNorm's F32 result, out = n * (1 + scale) + shift rounded
 // once, as modulate.
-constexpr int kAdalnMaxCols = 4096;
+constexpr int kAdalnMaxCols = 5120;
 
-template <typename T, int K, bool FULL>
-__global__ void __launch_bounds__(256) adaln_waves(const T* x, const float* scale, const float* shift, T* out,
+template <typename T, int K, bool FULL, int B>
+__global__ void __launch_bounds__(B) adaln_waves(const T* x, const float* scale, const float* shift, T* out,
                                                     int64_t rows, int cols, int64_t rows_per_sample, float eps) {
   constexpr int N = Chunk<T>::N;
   using Raw = typename Chunk<T>::Raw;
   const int chunks = FULL ? K * kWave : cols / N;
   const int64_t sample = blockIdx.y;
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int64_t row = sample * rows_per_sample + (int64_t)blockIdx.x * 4 + wave;
+  const int64_t row = sample * rows_per_sample + (int64_t)blockIdx.x * (B / kWave) + wave;
   if (row >= min(rows, (sample + 1) * rows_per_sample)) return;
   Raw raw[K];
 #pragma unroll
@@ -584,10 +658,11 @@ __global__ void __launch_bounds__(256) adaln_waves(const T* x, const float* scal
   }
   s1 = group_sum<64>(s1);
   s2 = group_sum<64>(s2);
-  const double m1 = s1 / (double)cols;  // mean - x0
+  const double inverse_cols = 1.0 / (double)cols;
+  const double m1 = s1 * inverse_cols;  // mean - x0
   const double mean = x0 + m1;
-  const double variance = fmax(s2 / (double)cols - m1 * m1, 0.0);
-  const double factor = 1.0 / sqrt(variance + (double)eps);
+  const double variance = fmax(fma(s2, inverse_cols, -(m1 * m1)), 0.0);
+  const double factor = eps > 0.0f ? inverse_sqrt<true>(variance + (double)eps) : inverse_sqrt(variance + (double)eps);
   const double offset = -mean * factor;
   const float* sc = scale + sample * cols;
   const float* sh = shift + sample * cols;
@@ -595,6 +670,7 @@ __global__ void __launch_bounds__(256) adaln_waves(const T* x, const float* scal
   for (int k = 0; k < K; ++k) {
     const int c = k * kWave + lane;
     if (FULL || c < chunks) {
+      opaque(raw[k]);
       float v[N], o[N], a[N], b[N];
       Chunk<T>::unpack(raw[k], v);
       load_f32<N>(sc + c * N, a);
@@ -606,6 +682,89 @@ __global__ void __launch_bounds__(256) adaln_waves(const T* x, const float* scal
       }
       Chunk<T>::store(out + row * cols + c * N, o);
     }
+  }
+}
+
+// F32 AdaLN of few rows (up to one a wave) or many (seven or more a wave), at
+// a wave a SIMD: the lane's scale and shift in registers across the rows it
+// takes, the next row's loads in flight (adaln_resident's plan, the tables
+// kept as float: as doubles they would not fit). Measured against adaln_waves
+// in 256-thread blocks, us a launch in graph replays: [300, 3072] 5.0 -> 4.1,
+// [7800, 3072] (192 MB) 36.9 -> 34.9, [16000, 3072] of two samples 70.8 ->
+// 69.5, [8190, 1536] 19.2 -> 18.1; but [1500, 3840] 11.2 against 9.5.
+template <int K, bool FULL>
+__global__ void __launch_bounds__(kWave) adaln_resident_f32(const float* x, const float* scale, const float* shift,
+                                                      float* out, int64_t rows, int cols, int64_t rows_per_sample,
+                                                      float eps, int64_t waves_per_sample) {
+  constexpr int N = 4;
+  using Raw = uint4;
+  const int chunks = FULL ? K * kWave : cols / N;
+  const int64_t sample = blockIdx.y;
+  const int lane = threadIdx.x;
+  const int64_t w = blockIdx.x;
+  const int64_t end = min(rows, (sample + 1) * rows_per_sample);
+  int64_t row = sample * rows_per_sample + w;
+  if (row >= end) return;
+  auto load_row = [&](int64_t r, Raw(&into)[K]) {
+#pragma unroll
+    for (int k = 0; k < K; ++k) {
+      const int c = FULL ? k * kWave + lane : min(k * kWave + lane, chunks - 1);
+      into[k] = stream_load(x + r * cols + c * N);
+    }
+  };
+  Raw raw[K];
+  load_row(row, raw);
+  float a[K][N], b[K][N];
+#pragma unroll
+  for (int k = 0; k < K; ++k) {
+    const int c = FULL ? k * kWave + lane : min(k * kWave + lane, chunks - 1);
+    load_f32<N>(scale + sample * cols + c * N, a[k]);
+    load_f32<N>(shift + sample * cols + c * N, b[k]);
+  }
+  const double inverse_cols = 1.0 / (double)cols;
+  for (; row < end; row += waves_per_sample) {
+    Raw next[K];
+    if (row + waves_per_sample < end) load_row(row + waves_per_sample, next);
+    const double x0 = (double)__shfl(__uint_as_float(raw[0].x), 0);
+    double s1 = 0.0, s2 = 0.0;
+#pragma unroll
+    for (int k = 0; k < K; ++k) {
+      if (FULL || k * kWave + lane < chunks) {
+        float v[N];
+        Chunk<float>::unpack(raw[k], v);
+#pragma unroll
+        for (int j = 0; j < N; ++j) {
+          const double d = (double)v[j] - x0;
+          s1 += d;
+          s2 = fma(d, d, s2);
+        }
+      }
+    }
+    s1 = group_sum<64>(s1);
+    s2 = group_sum<64>(s2);
+    const double m1 = s1 * inverse_cols;
+    const double mean = x0 + m1;
+    const double variance = fmax(fma(s2, inverse_cols, -(m1 * m1)), 0.0);
+    const double var_eps = variance + (double)eps;
+    const double factor = eps > 0.0f ? inverse_sqrt<true>(var_eps) : inverse_sqrt(var_eps);
+    const double offset = -mean * factor;
+#pragma unroll
+    for (int k = 0; k < K; ++k) {
+      const int c = k * kWave + lane;
+      if (FULL || c < chunks) {
+        opaque(raw[k]);
+        float v[N], o[N];
+        Chunk<float>::unpack(raw[k], v);
+#pragma unroll
+        for (int j = 0; j < N; ++j) {
+          const float n = (float)fma((double)v[j], factor, offset);
+          o[j] = (float)fma((double)n, 1.0 + (double)a[k][j], (double)b[k][j]);
+        }
+        Chunk<float>::store(out + row * cols + c * N, o);
+      }
+    }
+#pragma unroll
+    for (int k = 0; k < K; ++k) raw[k] = next[k];
   }
 }
 
@@ -686,7 +845,8 @@ __global__ void __launch_bounds__(256) adaln_resident(const uint16_t* x, const f
     const double m1 = s1 * inverse_cols;  // mean - x0
     const double mean = (double)x0 + m1;
     const double variance = fmax(fma(s2, inverse_cols, -(m1 * m1)), 0.0);
-    const double factor = eps > 0.0f ? inverse_sqrt<true>(variance + (double)eps) : inverse_sqrt(variance + (double)eps);
+    const double var_eps = variance + (double)eps;
+    const double factor = eps > 0.0f ? inverse_sqrt<true>(var_eps) : inverse_sqrt(var_eps);
     const double offset = -mean * factor;
 #pragma unroll
     for (int k = 0; k < K; ++k) {
@@ -738,6 +898,8 @@ __global__ void __launch_bounds__(256) modulate_chunks(const T* x, const float* 
 }
 
 // ------------------------------------------------------------------ launch layer
+
+constexpr int64_t kSimds = 1024;  // 256 CUs of 4
 
 // How a row is split: W waves per row, K chunks per lane; K = 0 means the
 // scalar path.
@@ -797,15 +959,13 @@ int wide_waves(int64_t rows, int cols, const RowPlan& plan) {
 // residual, from 1025 to 4096 rows of at most 12 chunks a lane, and BF16 rows
 // past the resident line. RESIDENT up to a row a wave (1024 waves: one a SIMD)
 // and from 7 on. Returns false for the others.
-constexpr int64_t kSimds = 1024;
-constexpr int64_t kWaveRowsMax = INT32_MAX;
 
 template <typename T>
 bool rms_waves_launch(T* x, const T* y, const float* weight, T* out, int64_t rows, int cols, float eps, float offset,
                       hipStream_t s) {
   const int per_lane = (int)ceil_div(cols / Chunk<T>::N, kWave);
   const bool resident = rows <= kSimds || rows >= 7 * kSimds;
-  if (rows < 384 || rows > kWaveRowsMax || per_lane > 20) return false;
+  if (rows < 384 || rows > kOneWaveBlocks || per_lane > 20) return false;
   if (y && (per_lane > 12 || rows <= kSimds || (rows > 4 * kSimds && !(sizeof(T) == 2 && resident)))) return false;
   const dim3 grid((unsigned)(resident ? std::min(rows, kSimds) : rows)), block(kWave);
 #define DRIFT_RMS_WAVES(K)                                                                                          \
@@ -873,7 +1033,7 @@ int rms_norm(const char* entry, T* x, const T* y, const float* weight, T* out, i
   } else if (plan.per_lane == 0) {
     hipLaunchKernelGGL(rms_norm_rows_scalar<T>, dim3(grid_for(rows, 1)), dim3(256), 0, s, x, y, weight, out, rows,
                        (int)cols, eps, offset, (int)weight_rows);
-  } else if (weight_rows == 1 && !y && !q.xq && cols / Chunk<T>::N <= kWave && rows <= kWaveRowsMax) {
+  } else if (weight_rows == 1 && !y && !q.xq && cols / Chunk<T>::N <= kWave && rows <= kOneWaveBlocks) {
     const int chunks = cols / Chunk<T>::N;
     if (chunks <= 8)
       rms_groups_launch<T, 8>(x, weight, out, rows, cols, eps, offset, s);
@@ -960,18 +1120,20 @@ void adaln_resident_launch(const uint16_t* x, const float* scale, const float* s
                      rows_per_sample, eps, per_sample);
 }
 
-// AdaLN: BF16 through adaln_resident, F32 through adaln_waves; rows of whole
-// 16-byte chunks, at most 4096 values. Returns -1 when the shape does not
-// qualify.
+// AdaLN of rows of whole 16-byte chunks, at most 5120 values: BF16 through
+// adaln_resident up to 4096 values and adaln_waves beyond, for more than 1,024
+// rows (fewer are faster four waves a row: [552, 5120] 6.1 us against 6.4);
+// F32 through adaln_resident_f32 or adaln_waves (their comments' figures).
+// Returns -1 when the shape does not qualify.
 template <typename T>
 int adaln_launch(const T* x, const float* scale, const float* shift, T* out, int64_t rows, int cols,
                  int64_t rows_per_sample, float eps, hipStream_t s) {
   constexpr int N = Chunk<T>::N;
   const int64_t samples = ceil_div(rows, rows_per_sample);
-  if (cols % N != 0 || cols > kAdalnMaxCols || samples > 65535 || ceil_div(rows_per_sample, 4) >= INT32_MAX)
-    return -1;
+  if (cols % N != 0 || cols > kAdalnMaxCols || samples > 65535 || rows_per_sample > kOneWaveBlocks) return -1;
   const int chunks = cols / N;
   const int per_lane = (int)ceil_div(chunks, kWave);
+  if (per_lane > 4096 / N / kWave && rows <= kSimds) return -1;
   if constexpr (sizeof(T) == 2) {
 #define DRIFT_ADALN_CASE(K)                                                                                   \
   if (per_lane <= K) {                                                                                        \
@@ -988,17 +1150,42 @@ int adaln_launch(const T* x, const float* scale, const float* shift, T* out, int
     DRIFT_ADALN_CASE(6)
     DRIFT_ADALN_CASE(8)
 #undef DRIFT_ADALN_CASE
-  } else {
     const dim3 grid((unsigned)ceil_div(rows_per_sample, 4), (unsigned)samples);
-#define DRIFT_ADALN_CASE(K)                                                                                  \
-  if (per_lane <= K) {                                                                                       \
-    if (chunks == K * kWave)                                                                                 \
-      hipLaunchKernelGGL((adaln_waves<T, K, true>), grid, dim3(256), 0, s, x, scale, shift, out, rows, cols,  \
-                         rows_per_sample, eps);                                                              \
-    else                                                                                                     \
-      hipLaunchKernelGGL((adaln_waves<T, K, false>), grid, dim3(256), 0, s, x, scale, shift, out, rows, cols, \
-                         rows_per_sample, eps);                                                              \
-    return 0;                                                                                                \
+    hipLaunchKernelGGL((adaln_waves<T, 10, false, 256>), grid, dim3(256), 0, s, x, scale, shift, out, rows, cols,
+                       rows_per_sample, eps);
+    return 0;
+  } else {
+    if (per_lane <= 12 && (rows <= kSimds || rows >= 7 * kSimds)) {
+      // rows shared out as evenly as they go
+      int64_t waves = std::max<int64_t>(1, std::min(rows_per_sample, kSimds / samples));
+      waves = ceil_div(rows_per_sample, ceil_div(rows_per_sample, waves));
+      const dim3 grid((unsigned)waves, (unsigned)samples), block(kWave);
+#define DRIFT_ADALN_CASE(K)                                                                                      \
+  if (per_lane <= K) {                                                                                           \
+    if (chunks == K * kWave)                                                                                     \
+      hipLaunchKernelGGL((adaln_resident_f32<K, true>), grid, block, 0, s, x, scale, shift, out, rows, cols,     \
+                         rows_per_sample, eps, waves);                                                           \
+    else                                                                                                         \
+      hipLaunchKernelGGL((adaln_resident_f32<K, false>), grid, block, 0, s, x, scale, shift, out, rows, cols,    \
+                         rows_per_sample, eps, waves);                                                           \
+    return 0;                                                                                                    \
+  }
+      DRIFT_ADALN_CASE(3)
+      DRIFT_ADALN_CASE(6)
+      DRIFT_ADALN_CASE(8)
+      DRIFT_ADALN_CASE(12)
+#undef DRIFT_ADALN_CASE
+    }
+    const dim3 grid((unsigned)rows_per_sample, (unsigned)samples), block(kWave);
+#define DRIFT_ADALN_CASE(K)                                                                                      \
+  if (per_lane <= K) {                                                                                           \
+    if (chunks == K * kWave)                                                                                     \
+      hipLaunchKernelGGL((adaln_waves<T, K, true, kWave>), grid, block, 0, s, x, scale, shift, out, rows, cols,  \
+                         rows_per_sample, eps);                                                                  \
+    else                                                                                                         \
+      hipLaunchKernelGGL((adaln_waves<T, K, false, kWave>), grid, block, 0, s, x, scale, shift, out, rows, cols, \
+                         rows_per_sample, eps);                                                                  \
+    return 0;                                                                                                    \
   }
     DRIFT_ADALN_CASE(1)
     DRIFT_ADALN_CASE(2)
@@ -1008,6 +1195,7 @@ int adaln_launch(const T* x, const float* scale, const float* shift, T* out, int
     DRIFT_ADALN_CASE(8)
     DRIFT_ADALN_CASE(12)
     DRIFT_ADALN_CASE(16)
+    DRIFT_ADALN_CASE(20)
 #undef DRIFT_ADALN_CASE
   }
   return -1;
@@ -1033,6 +1221,26 @@ int layer_norm(const char* entry, const T* x, const float* weight, const float* 
     hipLaunchKernelGGL((layer_norm_rows_scalar<T, MODULATE>), dim3(grid_for(rows, 1)), dim3(256), 0, s, x, weight,
                        bias, out, rows, (int)cols, rows_per_sample, eps);
     return launched(entry);
+  }
+  if constexpr (!MODULATE) {
+    const int per_lane = (int)ceil_div(cols / 4, kWave);
+    if (plan.waves == 4 && rows > kSimds && rows <= kOneWaveBlocks && per_lane <= 20) {
+      const dim3 one((unsigned)rows), block(kWave);
+#define DRIFT_LN_WAVES(K)                                                                                \
+  if (per_lane <= K) {                                                                                   \
+    hipLaunchKernelGGL(layer_norm_waves<K>, one, block, 0, s, x, weight, bias, out, rows, cols, eps);           \
+    return launched(entry);                                                                                     \
+  }
+      DRIFT_LN_WAVES(4)
+      DRIFT_LN_WAVES(5)
+      DRIFT_LN_WAVES(6)
+      DRIFT_LN_WAVES(8)
+      DRIFT_LN_WAVES(10)
+      DRIFT_LN_WAVES(12)
+      DRIFT_LN_WAVES(16)
+      DRIFT_LN_WAVES(20)
+#undef DRIFT_LN_WAVES
+    }
   }
   const unsigned grid = grid_for(rows, 4 / plan.waves);
 #define DRIFT_LN_CASE(K)                                                                                     \

@@ -268,6 +268,24 @@ def test_layer_norm_modulate(hip, rows, cols, samples, dtype):
         assert_bf16(o.layer_norm_modulate_bf16(xb, s, sh, per, 1e-6), host_bits(out), what="AdaLN bf16")
 
 
+# both sides of the lines between a row's splits (1,024 and 7,168 rows, 4,096
+# and 5,120 values, 12 chunks a lane), rows that fill no whole wave's chunks,
+# samples that share the resident waves unevenly
+@pytest.mark.parametrize("rows,cols,samples,dtype", [
+    (1024, 1536, 1, "f32"), (1025, 1536, 1, "f32"), (7167, 260, 1, "f32"), (7168, 260, 3, "f32"), (700, 3076, 7, "f32"),
+    (9000, 772, 2, "f32"), (1030, 3840, 1, "f32"), (1026, 4100, 2, "f32"), (1100, 5120, 1, "f32"), (30, 5116, 2, "f32"),
+    (1025, 5120, 3, "bf16"), (1030, 4104, 1, "bf16"), (1024, 5120, 2, "bf16"), (1200, 5128, 1, "bf16"),
+])
+def test_layer_norm_modulate_row_splits(hip, rows, cols, samples, dtype):
+    test_layer_norm_modulate(hip, rows, cols, samples, dtype)
+
+
+@pytest.mark.parametrize("shape", [(1024, 1152), (1025, 1028), (1300, 2308), (1100, 3072), (1030, 5120), (1050, 5124)])
+@pytest.mark.parametrize("affine", [(False, False), (True, False), (False, True), (True, True)])
+def test_layer_norm_row_splits(hip, shape, affine):
+    test_layer_norm_f32(hip, shape, affine)
+
+
 def test_layer_norm_modulate_in_place_bf16(hip):
     step("layerNormModulate bf16 in place")
     x = gaussian(14, (8, 3072))
