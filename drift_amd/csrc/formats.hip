@@ -18,6 +18,8 @@
 // bit-exact, BF16 being the F32 result rounded to nearest even.
 #include "common.hpp"
 
+#include <climits>
+
 namespace drift {
 namespace {
 
@@ -440,28 +442,39 @@ constexpr int run_field_align() {
   return (F::kBytes & -F::kBytes) < 8 ? (F::kBytes & -F::kBytes) : 8;
 }
 
-// Whether a format's rows of whole runs take decode_runs rather than
-// decode_rows by row (its two-dimensional grid). Timed on a [14336, 4096]
-// weight decoded to bf16, the two decoders' graph replays alternating with
-// the format's stream probe, both orders (us, runs / by row): Q4_K 25.0 /
-// 28.1, Q5_K 26.4 / 32.9, IQ4_NL 25.3 / 25.7 and ROCmFP4 25.4 / 26.9 take
-// runs; Q5_1 26.6 / 25.7, Q6_K 30.8 / 29.7, IQ4_XS 27.3 / 26.3 and ROCmFP4
-// fast 27.4 / 27.0 decode by row, as do Q4_0, Q4_1, Q5_0 and Q8_0.
+// Whether a gather's rows of whole runs take decode_runs rather than
+// decode_rows by row (its two-dimensional grid), and from how many runs on a
+// whole table does. Gathers: timed on a [14336, 4096] weight decoded to bf16
+// row by row, the two decoders' graph replays alternating with the format's
+// stream probe, both orders (us, runs / by row): Q4_K 25.0 / 28.1, Q5_K 26.4 /
+// 32.9, IQ4_NL 25.3 / 25.7 and ROCmFP4 25.4 / 26.9 take runs; Q5_1 26.6 /
+// 25.7, Q6_K 30.8 / 29.7, IQ4_XS 27.3 / 26.3 and ROCmFP4 fast 27.4 / 27.0
+// decode by row, as do Q4_0, Q4_1, Q5_0 and Q8_0. Whole tables, as one row (us
+// a launch in graph replays, runs / by row): Q4_K [14336, 4096] 25.9 / 26.0,
+// [9001, 5120] 21.1 / 21.3, [5001, 4864] 12.2 / 11.9, [1025, 1024] 2.9 / 2.3;
+// Q5_K 27.5 / 29.9, 22.0 / 24.6, 12.6 / 13.9, 3.0 / 2.2, [3001, 4096] 7.8 /
+// 8.0, [1537, 2560] 4.0 / 3.7; IQ4_NL 26.1 / 22.4, 21.4 / 18.2, 12.6 / 10.4,
+// 3.0 / 2.0 and ROCmFP4 26.2 / 23.0, 21.4 / 18.8, 12.7 / 10.7, 2.8 / 2.0
+// never.
 template <typename F>
 struct TakesRuns {
   static constexpr bool value = false;
+  static constexpr int64_t kWholeFrom = INT64_MAX;
 };
 template <bool FIVE>
 struct TakesRuns<QK45<FIVE>> {
   static constexpr bool value = true;
+  static constexpr int64_t kWholeFrom = FIVE ? 4096 : 16384;
 };
 template <>
 struct TakesRuns<IQ4_NL> {
   static constexpr bool value = true;
+  static constexpr int64_t kWholeFrom = INT64_MAX;
 };
 template <>
 struct TakesRuns<RocmFp4<false>> {
   static constexpr bool value = true;
+  static constexpr int64_t kWholeFrom = INT64_MAX;
 };
 
 template <typename T, typename F>
@@ -479,7 +492,7 @@ __global__ void __launch_bounds__(kWave) decode_runs(const uint8_t* table, const
   if constexpr (F::kLut != 0) {
     if (lane < 16) lut[lane] = lut_entry(F::kLut, lane);
   }
-  const int runs_per_row = cols / kRunValues;
+  const int runs_per_row = cols / kRunValues + (cols % kRunValues != 0);
   const int64_t run = blockIdx.x;
   const int64_t t = run / runs_per_row;
   const int r = (int)(run - t * runs_per_row);
@@ -487,18 +500,22 @@ __global__ void __launch_bounds__(kWave) decode_runs(const uint8_t* table, const
   const bool bad = id < 0 || id >= vocab;
   const uint4* src = reinterpret_cast<const uint4*>(table + (bad ? 0 : id) * row_bytes +
                                                     (int64_t)r * (kRunValues / F::kValues) * F::kBytes);
+  // a row's last run may be part full (the launcher: of whole pieces)
+  const int run_chunks = min(kRunValues / 8, cols / 8 - r * (kRunValues / 8));
+  const int pieces = run_chunks / kBlockChunks * F::kBytes / 16;
   uint4 piece[kLoads];
 #pragma unroll
-  for (int k = 0; k < kLoads; ++k) piece[k] = stream_load(src + min(lane + k * kWave, kPieces - 1));
+  for (int k = 0; k < kLoads; ++k) piece[k] = stream_load(src + min(lane + k * kWave, pieces - 1));
 #pragma unroll
   for (int k = 0; k < kLoads; ++k)
-    if (lane + k * kWave < kPieces) reinterpret_cast<uint4*>(staged)[lane + k * kWave] = piece[k];
+    if (lane + k * kWave < pieces) reinterpret_cast<uint4*>(staged)[lane + k * kWave] = piece[k];
   wave_sync();
   if (bad && bad_id && lane == 0) *bad_id = 1;
   T* target = out + t * cols + (int64_t)r * kRunValues;
 #pragma unroll
   for (int k = 0; k < 4; ++k) {
     const int chunk = k * kWave + lane;
+    if (chunk >= run_chunks) return;
     float v[8];
     if (bad) {
 #pragma unroll
@@ -577,6 +594,18 @@ int decode_launch(const char* entry, const void* table, int32_t format, const in
   if (!aligned16(out)) return refuse("%s: out is not 16-byte aligned", entry);
   if (reinterpret_cast<uintptr_t>(table) % (uintptr_t)l.align != 0)
     return refuse("%s: the table is not %d-byte aligned", entry, l.align);
+  // A whole table (no ids) is its rows' blocks one after another, and so is its
+  // output: it decodes as one row, whose runs and blocks of 256 chunks ignore
+  // where the table's rows end. By the rows' own blocks of 256 chunks and runs,
+  // widths that fill none of them whole left lanes idle and took the slower
+  // decoder: Q4_K [14337, 2560] 23.4 -> 16.9 us a launch in graph replays,
+  // [14337, 5120] 34.8 -> 32.1, Q6_K [13825, 2560] 23.9 -> 17.4, F16 [13825,
+  // 2560] 27.2 -> 23.3, Q8_0 [8191, 4864] 18.1 -> 17.7; [14336, 4096] even.
+  const bool whole = !ids && count == vocab && count * cols <= INT32_MAX;
+  if (whole) {
+    cols = (int32_t)(count * cols);
+    count = vocab = 1;
+  }
   const int64_t row_bytes = (int64_t)cols / l.values * l.bytes;
   const int64_t chunks = count * (cols / 8);
   const dim3 grid(grid_for(chunks, 256, kOneShotBlocks));
@@ -585,8 +614,10 @@ int decode_launch(const char* entry, const void* table, int32_t format, const in
 #define DRIFT_DECODE(CODE, F)                                                                                     \
   case CODE:                                                                                                     \
     if constexpr (TakesRuns<F>::value) {                                                                        \
-      const int64_t runs = count * (cols / kRunValues);                                                          \
-      if (vocab > 0 && cols % kRunValues == 0 && aligned16(table) && runs <= kOneShotBlocks) {                   \
+      const int64_t runs = count * ceil_div(cols, kRunValues);                                                   \
+      const bool by_runs = whole ? runs >= TakesRuns<F>::kWholeFrom && row_bytes % 16 == 0                       \
+                                 : vocab > 0 && cols % kRunValues == 0 && runs <= kOneShotBlocks;                \
+      if (by_runs && aligned16(table)) {                                                                         \
         hipLaunchKernelGGL((decode_runs<T, F>), dim3((unsigned)runs), dim3(kWave), 0, s, bytes, ids, out, count,  \
                            vocab, cols, row_bytes, bad_id);                                                      \
         break;                                                                                                   \

@@ -109,6 +109,21 @@ def test_rows_of_whole_runs(hip, name, cols):
         assert_bits(expected, host_bits(out), what=f"{name} dequantize {dtype} rows of {cols}")
 
 
+# whole tables decode as one row: rows that fill no block of 256 chunks or run
+# of 2,048 values, a last run part full, enough runs for the run decoder where
+# the format takes it (16,384 for Q4_K, 4,096 for Q5_K), fewer than one
+@pytest.mark.parametrize("name,rows,cols", [(n, 3, 256) for n in NAMES] + [(n, 131, 1280) for n in NAMES] + [
+    ("Q5_K", 6555, 1280), ("Q4_K", 13109, 2560), ("IQ4_NL", 6555, 1312), ("Q5_K", 4096, 2048), ("Q4_K", 16383, 2048)])
+def test_whole_tables_as_one_row(hip, name, rows, cols):
+    raw, table = table_of(name, rows, cols, 101)
+    step(f"dequantize {name} -> bf16 [{rows}, {cols}]")
+    flat = torch.full((rows * cols + 64,), -3, dtype=torch.bfloat16, device=DEV)
+    hip.dequantize(table, flat[:rows * cols].view(rows, cols))
+    want = o.to_bf16(o.embedding(name, raw, rows, cols, np.arange(rows, dtype=np.int32)))
+    assert_bits(want, host_bits(flat[:rows * cols].view(rows, cols)), what=f"{name} [{rows}, {cols}]")
+    assert bool((flat[rows * cols:] == -3).all()), "nothing past the end"
+
+
 @pytest.mark.parametrize("name", RUN_FORMATS)
 def test_runs_off_a_16_byte_boundary(hip, name):
     # the same rows from a table 8 bytes past a 16-byte boundary: the
