@@ -300,7 +300,7 @@ __device__ __forceinline__ void cache_values_tile(const Extras<T>& e, int64_t to
 // infinite partner NaN). A pair's position comes from its section's row.
 // Memory sets its pace: a gated query of 16 heads of 256 with 2 key heads, 64
 // values turning by interleaved sections, 4,096 tokens with the cache (150 MB)
-// takes 28.9 us, 5.2 TB/s, in graph replays; the general kernel, which reads
+// takes 23.9 us, 6.3 TB/s, in graph replays; the general kernel, which reads
 // values one by one and holds a block's barriers twice for every four heads,
 // took 137. The gate leaves by non-temporal stores (28 heads of 128 24.9 ->
 // 24.2 us, 16 of 64 25.3 -> 24.4, 16 of 256 even); storing it before the norm
@@ -372,8 +372,18 @@ __device__ __forceinline__ void qk_wave_heads(const T* q, const T* k, T* q_out, 
     w1[i] = x1.x, w1[i + 1] = x1.y, w1[i + 2] = x1.z, w1[i + 3] = x1.w;
   }
   const T* xh = query_c ? q + (t * a.q_heads + hc) * a.q_stride : k + (t * a.kv_heads + (hc - a.q_heads)) * dim;
-  const Raw r0 = Chunk<T>::load_raw(xh + d0);
-  const Raw r1 = Chunk<T>::load_raw(xh + d1);
+  // with the cache (or the gate) the heads load through the L2 as usual, not
+  // non-temporally, us a launch in graph replays: 28 heads of 128 16.3 -> 15.0,
+  // C3's 18.8 -> 18.3; gated, 16 heads of 256 with 64 turning 29.0 -> 23.9
+  // (its gate so too: 28.3 with the heads alone), F32 25.3 -> 23.0, 28 of 128
+  // 24.2 -> 21.5. Without the cache C3 takes 15.3 non-temporally, 15.7 so; the
+  // value tiles' loads too stay non-temporal (C3 18.7 -> 19.0).
+  auto load = [](const T* from) {
+    if constexpr (EXTRAS) return *reinterpret_cast<const Raw*>(from);
+    else return Chunk<T>::load_raw(from);
+  };
+  const Raw r0 = load(xh + d0);
+  const Raw r1 = load(xh + d1);
   // the second group's heads (P = 2; FAST: the same tensor as the first's)
   Raw s0, s1;
   if constexpr (P == 2) {
@@ -387,8 +397,8 @@ __device__ __forceinline__ void qk_wave_heads(const T* q, const T* k, T* q_out, 
   if constexpr (GATE) {
     if (a.q_heads > 0) {
       const T* gh = q + (t * a.q_heads + min(hc, a.q_heads - 1)) * a.q_stride + dim;
-      g0 = Chunk<T>::load_raw(gh + d0);
-      g1 = Chunk<T>::load_raw(gh + d1);
+      g0 = load(gh + d0);
+      g1 = load(gh + d1);
     }
   }
   // with the cache, a key wave's page and the token's place in it, divided

@@ -161,8 +161,8 @@ __global__ void __launch_bounds__(256) rms_norm_rows(T* x, const T* y, const flo
 //   F32 [7800, 3072] 37.4 / 37.5 / 33.5, with the residual 65.2 / 70.8 / 67.8
 //   bf16 [1000, 4096] 5.3 / 5.4 / 4.8; F32 [509, 2560] 4.8 / 4.7 / 3.9; bf16 [300, 4096] 3.8 / 4.4 / 3.9,
 //   with the residual 5.0 / 6.1 / 6.0
-// Two waves a SIMD in the resident grid were 1 to 4% slower on the larger of
-// these, three and four up to 15%.
+// Alone, two waves a SIMD in the resident grid were 1 to 4% slower on the
+// larger of these, three and four up to 15%.
 template <typename T, int K, bool ADD, bool RESIDENT>
 __global__ void __launch_bounds__(kWave) rms_norm_waves(T* x, const T* y, const float* weight, T* out, int64_t rows,
                                                         int cols, float eps, float offset) {
@@ -967,7 +967,11 @@ bool rms_waves_launch(T* x, const T* y, const float* weight, T* out, int64_t row
   const bool resident = rows <= kSimds || rows >= 7 * kSimds;
   if (rows < 384 || rows > kOneWaveBlocks || per_lane > 20) return false;
   if (y && (per_lane > 12 || rows <= kSimds || (rows > 4 * kSimds && !(sizeof(T) == 2 && resident)))) return false;
-  const dim3 grid((unsigned)(resident ? std::min(rows, kSimds) : rows)), block(kWave);
+  // waves of the resident grid: two a SIMD for BF16 alone, whose output a rope
+  // reads next (with ropeTable over [14040, 24, 128] queries and keys 122.7 us
+  // against 130.3 at one a SIMD; F32 and the residual 1% faster at one)
+  const int64_t waves = sizeof(T) == 2 && !y ? 2 * kSimds : kSimds;
+  const dim3 grid((unsigned)(resident ? std::min(rows, waves) : rows)), block(kWave);
 #define DRIFT_RMS_WAVES(K)                                                                                          \
   if (per_lane <= K) {                                                                                              \
     if (y && resident)                                                                                              \

@@ -112,7 +112,14 @@ __global__ void __launch_bounds__(256) rope_kernel(const T* x, const int32_t* po
 // Row i / slots comes from a product with slots_inverse = ceil(2^32 / slots)
 // (exact where i * slots < 2^32: the launcher's bound on a token; 0 where
 // slots is 1). TOKENS: a wave's items are of several tokens.
-template <typename T, bool NEOX, int K, bool TOKENS>
+//
+// STREAM: the loads are non-temporal, for chunks rewritten where they were
+// read, whole lines at a time (plain loads there: F32 [2039, 32, 128] 12.5 ->
+// 15.1, bf16 interleaved [4096, 32, 128] 11.9 -> 14.5). Elsewhere plain loads
+// are faster: bf16 [6546, 24, 256] with 64 turning 31.9 -> 28.7, in place
+// (halves of a line) 10.9 -> 9.4, F32 [4087, 16, 72] 9.9 -> 8.0, [4830, 12,
+// 64] 6.6 -> 5.4, [2039, 32, 128] out of place 12.5 -> 11.9.
+template <typename T, bool NEOX, int K, bool TOKENS, bool STREAM>
 __global__ void __launch_bounds__(kWave) rope_waves(const T* x, const int32_t* positions, T* out, RopeArgs p, int slots,
                                                     uint32_t slots_inverse, uint32_t runs, int per_wave) {
   constexpr int N = Chunk<T>::N;
@@ -154,8 +161,12 @@ __global__ void __launch_bounds__(kWave) rope_waves(const T* x, const int32_t* p
     turns[k] = j < rotating;
     at[k] = row * p.dim + (NEOX && !turns[k] ? p.rotary + (j - rotating) * N : j * N);
     slot[k] = (TOKENS ? row / p.heads * half : 0) + j;
-    r0[k] = Chunk<T>::load_raw(xt + at[k]);
-    if constexpr (NEOX) r1[k] = Chunk<T>::load_raw(xt + at[k] + (turns[k] ? half : 0));
+    auto load = [](const T* from) {
+      if constexpr (STREAM) return Chunk<T>::load_raw(from);
+      else return *reinterpret_cast<const Raw*>(from);
+    };
+    r0[k] = load(xt + at[k]);
+    if constexpr (NEOX) r1[k] = load(xt + at[k] + (turns[k] ? half : 0));
   }
 #pragma unroll
   for (int u = 0; u < kPairsPerLane; ++u) {
@@ -461,19 +472,25 @@ int rope(const char* entry, const T* x, const int32_t* positions, T* out, int32_
   if (chunked && blocks <= kOneWaveBlocks) {
     const dim3 grid((unsigned)blocks), block(kWave);
     const uint32_t slots_inverse = slots == 1 ? 0 : (uint32_t)ceil_div((int64_t)1 << 32, slots);
-#define DRIFT_ROPE_LAUNCH(NEOX, K, TOKENS)                                                                       \
-  hipLaunchKernelGGL((rope_waves<T, NEOX, K, TOKENS>), grid, block, 0, st, x, positions, out, p, slots,          \
-                     slots_inverse, (uint32_t)runs, (int)per_wave)
-#define DRIFT_ROPE_CASE(K)                \
-  case K:                                 \
-    if (neox && per_wave > 1)             \
-      DRIFT_ROPE_LAUNCH(true, K, true);   \
-    else if (neox)                        \
-      DRIFT_ROPE_LAUNCH(true, K, false);  \
-    else if (per_wave > 1)                \
-      DRIFT_ROPE_LAUNCH(false, K, true);  \
-    else                                  \
-      DRIFT_ROPE_LAUNCH(false, K, false); \
+    const bool stream = x == out && (!neox || rotary / 2 * sizeof(T) % 128 == 0);
+#define DRIFT_ROPE_LAUNCH(NEOX, K, TOKENS)                                                                         \
+  if (stream)                                                                                                      \
+    hipLaunchKernelGGL((rope_waves<T, NEOX, K, TOKENS, true>), grid, block, 0, st, x, positions, out, p, slots,    \
+                       slots_inverse, (uint32_t)runs, (int)per_wave);                                              \
+  else                                                                                                             \
+    hipLaunchKernelGGL((rope_waves<T, NEOX, K, TOKENS, false>), grid, block, 0, st, x, positions, out, p, slots,   \
+                       slots_inverse, (uint32_t)runs, (int)per_wave)
+#define DRIFT_ROPE_CASE(K)                  \
+  case K:                                   \
+    if (neox && per_wave > 1) {             \
+      DRIFT_ROPE_LAUNCH(true, K, true);     \
+    } else if (neox) {                      \
+      DRIFT_ROPE_LAUNCH(true, K, false);    \
+    } else if (per_wave > 1) {              \
+      DRIFT_ROPE_LAUNCH(false, K, true);    \
+    } else {                                \
+      DRIFT_ROPE_LAUNCH(false, K, false);   \
+    }                                       \
     break;
     switch (per_lane) {
       DRIFT_ROPE_CASE(1)
