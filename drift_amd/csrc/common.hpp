@@ -48,6 +48,10 @@ __device__ __forceinline__ uint4 stream_load(const void* p) {
   return make_uint4(q.x, q.y, q.z, q.w);
 }
 
+// The same through the caches as usual, for lines that several waves or
+// instructions share.
+__device__ __forceinline__ uint4 cached_load(const void* p) { return *reinterpret_cast<const uint4*>(p); }
+
 // A 16-byte chunk of a row: 4 floats or 8 bf16, unpacked to float.
 template <typename T>
 struct Chunk;

@@ -290,7 +290,7 @@ __global__ void __launch_bounds__(kWave) convert_bf16_waves(const void* x, void*
     const u32x4 q = odd ? u32x4{r0, r1, b0, b1} : u32x4{a0, a1, r0, r1};
     __builtin_nontemporal_store(q, reinterpret_cast<u32x4*>(ob + chunk * 8));
   } else {
-    const uint4 q = stream_load(xb + chunk * 8);
+    const uint4 q = cached_load(xb + chunk * 8);  // 23.6 us non-temporally, 21.8 so ([7800, 3072])
     const uint32_t r0 = (uint32_t)dpp_move32<0xb1>((int)(odd ? q.x : q.z));
     const uint32_t r1 = (uint32_t)dpp_move32<0xb1>((int)(odd ? q.y : q.w));
     const uint32_t a0 = odd ? r0 : q.x, a1 = odd ? r1 : q.y, b0 = odd ? q.z : r0, b1 = odd ? q.w : r1;

@@ -420,8 +420,10 @@ __global__ void __launch_bounds__(256) decode_staged(const uint8_t* table, const
 
 // Block formats a run of 2048 values at a time (8 blocks of 256 or 64 of 32),
 // for rows of whole runs on 16-byte boundaries: a one-wave block copies the
-// run's bytes (1,152 to 1,408 for the formats that take it, a multiple of 16)
-// into LDS with 16-byte loads, all in flight together, then each lane decodes
+// run's bytes (1,088 to 1,680 for the formats that take it, a multiple of 16)
+// into LDS with 16-byte loads, all in flight together and plain (a run's first
+// and last lines are its neighbours' too: Q4_K [14336, 4096] 26.3 us
+// non-temporally, 23.1 so), then each lane decodes
 // 4 chunks (chunk k * 64 + lane of the run's 256) from there, so each store
 // instruction writes 64 consecutive 16-byte pieces and a block's scales are
 // read from LDS by the lanes that share them.
@@ -445,36 +447,47 @@ constexpr int run_field_align() {
 // Whether a gather's rows of whole runs take decode_runs rather than
 // decode_rows by row (its two-dimensional grid), and from how many runs on a
 // whole table does. Gathers: timed on a [14336, 4096] weight decoded to bf16
-// row by row, the two decoders' graph replays alternating with the format's
-// stream probe, both orders (us, runs / by row): Q4_K 25.0 / 28.1, Q5_K 26.4 /
-// 32.9, IQ4_NL 25.3 / 25.7 and ROCmFP4 25.4 / 26.9 take runs; Q5_1 26.6 /
-// 25.7, Q6_K 30.8 / 29.7, IQ4_XS 27.3 / 26.3 and ROCmFP4 fast 27.4 / 27.0
-// decode by row, as do Q4_0, Q4_1, Q5_0 and Q8_0. Whole tables, as one row (us
-// a launch in graph replays, runs / by row): Q4_K [14336, 4096] 25.9 / 26.0,
-// [9001, 5120] 21.1 / 21.3, [5001, 4864] 12.2 / 11.9, [1025, 1024] 2.9 / 2.3;
-// Q5_K 27.5 / 29.9, 22.0 / 24.6, 12.6 / 13.9, 3.0 / 2.2, [3001, 4096] 7.8 /
-// 8.0, [1537, 2560] 4.0 / 3.7; IQ4_NL 26.1 / 22.4, 21.4 / 18.2, 12.6 / 10.4,
-// 3.0 / 2.0 and ROCmFP4 26.2 / 23.0, 21.4 / 18.8, 12.7 / 10.7, 2.8 / 2.0
-// never.
+// row by row, the runs loaded non-temporally (us, runs / by row): Q4_K 25.0 /
+// 28.1, Q5_K 26.4 / 32.9, IQ4_NL 25.3 / 25.7 and ROCmFP4 25.4 / 26.9 take
+// runs; Q5_1 26.6 / 25.7, Q6_K 30.8 / 29.7, IQ4_XS 27.3 / 26.3 and ROCmFP4
+// fast 27.4 / 27.0 decode by row, as do Q4_0, Q4_1, Q5_0 and Q8_0.
+// Whole tables, as one row (us a launch in graph replays, runs / by row, at
+// [2001, 2048], [4096, 4096], [9000, 5120] and [14336, 4096]): Q4_K 3.2 / 3.3,
+// 7.7 / 8.8, 18.7 / 21.2, 22.7 / 26.0; Q5_K 3.7 / 3.8, 7.8 / 9.8, 19.5 / 24.6,
+// 23.5 / 30.3; Q6_K 3.9 / 3.6, 8.8 / 9.5, 20.5 / 21.8, 25.3 / 27.8; ROCmFP4
+// 3.6 / 2.9, 7.5 / 7.9, 18.1 / 18.2, 22.1 / 23.1; IQ4_XS 3.2 / 3.0, 8.1 / 7.8,
+// 18.4 / 18.5, 22.7 / 23.6; IQ4_NL 3.4 / 2.8, 7.5 / 7.6, 18.1 / 17.7, 22.2 /
+// 22.4. At [14336, 4096] Q4_0 22.6 / 21.5, Q5_0 29.1 / 23.7, Q5_1 24.6 / 22.8,
+// Q8_0 26.7 / 25.6.
 template <typename F>
 struct TakesRuns {
-  static constexpr bool value = false;
+  static constexpr bool kGather = false;
   static constexpr int64_t kWholeFrom = INT64_MAX;
 };
 template <bool FIVE>
 struct TakesRuns<QK45<FIVE>> {
-  static constexpr bool value = true;
-  static constexpr int64_t kWholeFrom = FIVE ? 4096 : 16384;
+  static constexpr bool kGather = true;
+  static constexpr int64_t kWholeFrom = 2048;
+};
+template <>
+struct TakesRuns<Q6_K> {
+  static constexpr bool kGather = false;
+  static constexpr int64_t kWholeFrom = 8192;
+};
+template <>
+struct TakesRuns<IQ4_XS> {
+  static constexpr bool kGather = false;
+  static constexpr int64_t kWholeFrom = 20480;
 };
 template <>
 struct TakesRuns<IQ4_NL> {
-  static constexpr bool value = true;
+  static constexpr bool kGather = true;
   static constexpr int64_t kWholeFrom = INT64_MAX;
 };
 template <>
 struct TakesRuns<RocmFp4<false>> {
-  static constexpr bool value = true;
-  static constexpr int64_t kWholeFrom = INT64_MAX;
+  static constexpr bool kGather = true;
+  static constexpr int64_t kWholeFrom = 8192;
 };
 
 template <typename T, typename F>
@@ -505,7 +518,7 @@ __global__ void __launch_bounds__(kWave) decode_runs(const uint8_t* table, const
   const int pieces = run_chunks / kBlockChunks * F::kBytes / 16;
   uint4 piece[kLoads];
 #pragma unroll
-  for (int k = 0; k < kLoads; ++k) piece[k] = stream_load(src + min(lane + k * kWave, pieces - 1));
+  for (int k = 0; k < kLoads; ++k) piece[k] = cached_load(src + min(lane + k * kWave, pieces - 1));
 #pragma unroll
   for (int k = 0; k < kLoads; ++k)
     if (lane + k * kWave < pieces) reinterpret_cast<uint4*>(staged)[lane + k * kWave] = piece[k];
@@ -598,9 +611,8 @@ int decode_launch(const char* entry, const void* table, int32_t format, const in
   // output: it decodes as one row, whose runs and blocks of 256 chunks ignore
   // where the table's rows end. By the rows' own blocks of 256 chunks and runs,
   // widths that fill none of them whole left lanes idle and took the slower
-  // decoder: Q4_K [14337, 2560] 23.4 -> 16.9 us a launch in graph replays,
-  // [14337, 5120] 34.8 -> 32.1, Q6_K [13825, 2560] 23.9 -> 17.4, F16 [13825,
-  // 2560] 27.2 -> 23.3, Q8_0 [8191, 4864] 18.1 -> 17.7; [14336, 4096] even.
+  // decoder: by row [13825, 2560] Q6_K 23.9 -> 17.4 us a launch in graph
+  // replays, F16 27.2 -> 23.3, Q8_0 [8191, 4864] 18.1 -> 17.7.
   const bool whole = !ids && count == vocab && count * cols <= INT32_MAX;
   if (whole) {
     cols = (int32_t)(count * cols);
@@ -613,10 +625,11 @@ int decode_launch(const char* entry, const void* table, int32_t format, const in
   switch (format) {
 #define DRIFT_DECODE(CODE, F)                                                                                     \
   case CODE:                                                                                                     \
-    if constexpr (TakesRuns<F>::value) {                                                                        \
+    if constexpr (TakesRuns<F>::kGather || TakesRuns<F>::kWholeFrom != INT64_MAX) {                              \
       const int64_t runs = count * ceil_div(cols, kRunValues);                                                   \
       const bool by_runs = whole ? runs >= TakesRuns<F>::kWholeFrom && row_bytes % 16 == 0                       \
-                                 : vocab > 0 && cols % kRunValues == 0 && runs <= kOneShotBlocks;                \
+                                 : TakesRuns<F>::kGather && vocab > 0 && cols % kRunValues == 0 &&               \
+                                       runs <= kOneShotBlocks;                                                   \
       if (by_runs && aligned16(table)) {                                                                         \
         hipLaunchKernelGGL((decode_runs<T, F>), dim3((unsigned)runs), dim3(kWave), 0, s, bytes, ids, out, count,  \
                            vocab, cols, row_bytes, bad_id);                                                      \
