@@ -505,8 +505,9 @@ __global__ void __launch_bounds__(256) layer_norm_rows(const T* x, const float* 
 // weights and biases are read after the sums: read first, their registers (as
 // doubles) held half as many waves. Measured, us a launch in graph replays,
 // four-wave group / weights first / this: [4087, 1152] (38 MB) 12.6 / 8.9 /
-// 8.4, [4830, 1280] 14.9 / 12.7 / 9.8, [9000, 1024] 19.1 / 18.1 / 15.5; [600,
-// 1152] 4.2 / 4.4 / 4.5, so up to 1,024 rows keep the group.
+// 8.4, [4830, 1280] 14.9 / 12.7 / 9.8, [9000, 1024] 19.1 / 18.1 / 15.5; group / this
+// [2000, 2048] 9.2 / 7.9, [1100, 4096] 11.6 / 11.1; but [1100, 1024] 4.0 / 4.7
+// and [600, 1152] 4.2 / 4.5: up to 1,024 rows or 2^19 chunks keep the group.
 template <int K>
 __global__ void __launch_bounds__(kWave) layer_norm_waves(const float* x, const float* weight, const float* bias,
                                                           float* out, int64_t rows, int cols, float eps) {
@@ -955,46 +956,54 @@ int wide_waves(int64_t rows, int cols, const RowPlan& plan) {
 }
 
 // rms_norm_waves for rows of four waves' chunks, where it measured faster than
-// the four-wave group (its comment's figures): alone, from 384 rows; with the
-// residual, from 1025 to 4096 rows of at most 12 chunks a lane, and BF16 rows
-// past the resident line. RESIDENT up to a row a wave (1024 waves: one a SIMD)
-// and from 7 on. Returns false for the others.
-
+// the four-wave group (its comment's figures): alone, from 384 rows (BF16 of
+// more than 8 chunks a lane, from 1025: [600, 6144] 5.5 us in the group, 5.9
+// so); with the residual, from 1025 to 4096 rows of at most 12 chunks a lane,
+// and BF16 rows of at most 10 past the resident line ([9000, 6144] 77.9 in the
+// group, 80.2 so). RESIDENT up to a row a wave (1024 waves: one a SIMD) and
+// from 7 on. Returns false for the others.
 template <typename T>
 bool rms_waves_launch(T* x, const T* y, const float* weight, T* out, int64_t rows, int cols, float eps, float offset,
                       hipStream_t s) {
   const int per_lane = (int)ceil_div(cols / Chunk<T>::N, kWave);
   const bool resident = rows <= kSimds || rows >= 7 * kSimds;
-  if (rows < 384 || rows > kOneWaveBlocks || per_lane > 20) return false;
-  if (y && (per_lane > 12 || rows <= kSimds || (rows > 4 * kSimds && !(sizeof(T) == 2 && resident)))) return false;
+  if (rows < 384 || rows > kOneWaveBlocks || per_lane > (sizeof(T) == 4 ? 20 : 16)) return false;
+  if (sizeof(T) == 2 && per_lane > 8 && rows <= kSimds) return false;
+  if (y && (per_lane > 12 || rows <= kSimds)) return false;
+  if (y && rows > 4 * kSimds && !(sizeof(T) == 2 && resident && per_lane <= 10)) return false;
   // waves of the resident grid: two a SIMD for BF16 alone, whose output a rope
   // reads next (with ropeTable over [14040, 24, 128] queries and keys 122.7 us
   // against 130.3 at one a SIMD; F32 and the residual 1% faster at one)
   const int64_t waves = sizeof(T) == 2 && !y ? 2 * kSimds : kSimds;
   const dim3 grid((unsigned)(resident ? std::min(rows, waves) : rows)), block(kWave);
-#define DRIFT_RMS_WAVES(K)                                                                                          \
+#define DRIFT_RMS_WAVES(K, ADD)                                                                                     \
   if (per_lane <= K) {                                                                                              \
-    if (y && resident)                                                                                              \
-      hipLaunchKernelGGL((rms_norm_waves<T, K, true, true>), grid, block, 0, s, x, y, weight, out, rows, cols, eps, \
-                         offset);                                                                                   \
-    else if (y)                                                                                                     \
-      hipLaunchKernelGGL((rms_norm_waves<T, K, true, false>), grid, block, 0, s, x, y, weight, out, rows, cols,     \
-                         eps, offset);                                                                              \
-    else if (resident)                                                                                              \
-      hipLaunchKernelGGL((rms_norm_waves<T, K, false, true>), grid, block, 0, s, x, y, weight, out, rows, cols,     \
-                         eps, offset);                                                                              \
-    else                                                                                                            \
-      hipLaunchKernelGGL((rms_norm_waves<T, K, false, false>), grid, block, 0, s, x, y, weight, out, rows, cols,    \
-                         eps, offset);                                                                              \
+    if constexpr (sizeof(T) == 2 || !ADD) { /* F32 with the residual is never resident */                           \
+      if (resident) {                                                                                               \
+        hipLaunchKernelGGL((rms_norm_waves<T, K, ADD, true>), grid, block, 0, s, x, y, weight, out, rows, cols,     \
+                           eps, offset);                                                                            \
+        return true;                                                                                                \
+      }                                                                                                             \
+    }                                                                                                               \
+    hipLaunchKernelGGL((rms_norm_waves<T, K, ADD, false>), grid, block, 0, s, x, y, weight, out, rows, cols, eps,   \
+                       offset);                                                                                     \
     return true;                                                                                                    \
   }
-  DRIFT_RMS_WAVES(4)
-  DRIFT_RMS_WAVES(6)
-  DRIFT_RMS_WAVES(8)
-  DRIFT_RMS_WAVES(10)
-  DRIFT_RMS_WAVES(12)
-  DRIFT_RMS_WAVES(16)
-  DRIFT_RMS_WAVES(20)
+  if (y) {
+    DRIFT_RMS_WAVES(4, true)
+    DRIFT_RMS_WAVES(6, true)
+    DRIFT_RMS_WAVES(8, true)
+    DRIFT_RMS_WAVES(10, true)
+    DRIFT_RMS_WAVES(12, true)
+  } else {
+    DRIFT_RMS_WAVES(4, false)
+    DRIFT_RMS_WAVES(6, false)
+    DRIFT_RMS_WAVES(8, false)
+    DRIFT_RMS_WAVES(10, false)
+    DRIFT_RMS_WAVES(12, false)
+    DRIFT_RMS_WAVES(16, false)
+    if constexpr (sizeof(T) == 4) DRIFT_RMS_WAVES(20, false)
+  }
 #undef DRIFT_RMS_WAVES
   return false;
 }
@@ -1228,7 +1237,8 @@ int layer_norm(const char* entry, const T* x, const float* weight, const float* 
   }
   if constexpr (!MODULATE) {
     const int per_lane = (int)ceil_div(cols / 4, kWave);
-    if (plan.waves == 4 && rows > kSimds && rows <= kOneWaveBlocks && per_lane <= 20) {
+    if (plan.waves == 4 && rows > kSimds && rows * (cols / 4) >= (1 << 19) && rows <= kOneWaveBlocks &&
+        per_lane <= 20) {
       const dim3 one((unsigned)rows), block(kWave);
 #define DRIFT_LN_WAVES(K)                                                                                \
   if (per_lane <= K) {                                                                                   \

@@ -448,7 +448,7 @@ int rope(const char* entry, const T* x, const int32_t* positions, T* out, int32_
   constexpr int N = Chunk<T>::N;
   const bool neox = layout == DRIFT_ROPE_NEOX;
   const bool chunked = aligned16(x) && aligned16(out) && dim % N == 0 && rotary % (neox ? 2 * N : N) == 0 &&
-                       (int64_t)heads * dim <= (1 << 24);
+                       (int64_t)heads * dim <= INT32_MAX;
   const hipStream_t st = (hipStream_t)stream;
   const int rotating = neox ? rotary / 2 / N : rotary / N;
   const int slots = x == out ? rotating : rotating + (dim - rotary) / N;
@@ -469,7 +469,7 @@ int rope(const char* entry, const T* x, const int32_t* positions, T* out, int32_
   const int64_t fit = std::min<int64_t>(per_lane * kWave / items, rotary > 0 ? kMaxPairs / (rotary / 2) : kMaxPairs);
   const int64_t per_wave = std::max<int64_t>(1, std::min<int64_t>(fit, tokens));
   const int64_t blocks = ceil_div(tokens, per_wave) * runs;
-  if (chunked && blocks <= kOneWaveBlocks) {
+  if (chunked && blocks <= kOneWaveBlocks && items * slots < (int64_t)1 << 32) {
     const dim3 grid((unsigned)blocks), block(kWave);
     const uint32_t slots_inverse = slots == 1 ? 0 : (uint32_t)ceil_div((int64_t)1 << 32, slots);
     const bool stream = x == out && (!neox || rotary / 2 * sizeof(T) % 128 == 0);
