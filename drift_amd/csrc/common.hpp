@@ -75,6 +75,9 @@ struct Chunk<float> {
     const u32x4 q = {__float_as_uint(v[0]), __float_as_uint(v[1]), __float_as_uint(v[2]), __float_as_uint(v[3])};
     __builtin_nontemporal_store(q, reinterpret_cast<u32x4*>(p));
   }
+  __device__ __forceinline__ static void store_cached(float* p, const float (&v)[4]) {
+    *reinterpret_cast<float4*>(p) = make_float4(v[0], v[1], v[2], v[3]);
+  }
 };
 
 template <>
@@ -96,6 +99,10 @@ struct Chunk<uint16_t> {
   __device__ __forceinline__ static void store(uint16_t* p, const float (&v)[8]) {
     const u32x4 q = {pack_bf16(v[0], v[1]), pack_bf16(v[2], v[3]), pack_bf16(v[4], v[5]), pack_bf16(v[6], v[7])};
     __builtin_nontemporal_store(q, reinterpret_cast<u32x4*>(p));
+  }
+  __device__ __forceinline__ static void store_cached(uint16_t* p, const float (&v)[8]) {
+    *reinterpret_cast<uint4*>(p) =
+        make_uint4(pack_bf16(v[0], v[1]), pack_bf16(v[2], v[3]), pack_bf16(v[4], v[5]), pack_bf16(v[6], v[7]));
   }
 };
 

@@ -55,8 +55,10 @@ __device__ __forceinline__ void load_floats(const float* p, float (&v)[N]) {
   }
 }
 
-// One chunk's operands, loaded: x, y (gated ops), and the F32 factors.
-template <typename T, int OP>
+// One chunk's operands, loaded: x, y (gated ops), and the F32 factors. KEEP: x
+// moves through the caches as usual, both ways (gatedAdd's residual stream,
+// which the norm after it reads again).
+template <typename T, int OP, bool KEEP>
 struct Operands {
   static constexpr int N = Chunk<T>::N;
   typename Chunk<T>::Raw x, y;
@@ -70,7 +72,8 @@ struct Operands {
   // chunk i, which is value c of row r (of sample `sample`, gatedAdd)
   __device__ __forceinline__ void load_at(const T* xs, const T* ys, const float* v, const RowMap& m, int64_t i,
                                           int64_t r, int c, int64_t sample) {
-    x = Chunk<T>::load_raw(xs + i * N);
+    if constexpr (KEEP) x = cached_load(xs + i * N);
+    else x = Chunk<T>::load_raw(xs + i * N);
     if constexpr (OP != MODULATE_CHUNKS) y = Chunk<T>::load_raw(ys + i * N);
     if constexpr (OP == GATED_ADD) {
       load_floats<N, false>(v + sample * m.cols + c, a);
@@ -101,16 +104,17 @@ struct Operands {
 #pragma unroll
       for (int j = 0; j < N; ++j) o[j] = (float)((double)xv[j] + (double)a[j] * (double)yv[j]);
     }
-    Chunk<T>::store(out + i * N, o);
+    if constexpr (KEEP) Chunk<T>::store_cached(out + i * N, o);
+    else Chunk<T>::store(out + i * N, o);
   }
 };
 
-template <typename T, int OP>
+template <typename T, int OP, bool KEEP>
 __global__ void __launch_bounds__(512) row_map_chunks(const T* x, const T* y, const float* v, T* out, RowMap m,
                                                       int64_t total) {
   const int64_t stride = (int64_t)gridDim.x * blockDim.x;
   for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < total; i += stride) {
-    Operands<T, OP> p;
+    Operands<T, OP, KEEP> p;
     p.load(x, y, v, m, i);
     p.apply(out, i);
   }
@@ -120,13 +124,13 @@ __global__ void __launch_bounds__(512) row_map_chunks(const T* x, const T* y, co
 // The row from the grid: blockIdx.x a wave's chunks of the row, blockIdx.y
 // the row within sample blockIdx.z, so no lane divides. For rows of whole
 // waves' chunks and at most 65,535 rows a sample.
-template <typename T, int OP>
+template <typename T, int OP, bool KEEP>
 __global__ void __launch_bounds__(64) row_map_by_row(const T* x, const T* y, const float* v, T* out, RowMap m) {
   constexpr int N = Chunk<T>::N;
   const int64_t r = (int64_t)blockIdx.z * gridDim.y + blockIdx.y;
   const int c = (int)blockIdx.x * 64 + (int)threadIdx.x;
   const int64_t i = r * m.row_chunks + c;
-  Operands<T, OP> p;
+  Operands<T, OP, KEEP> p;
   p.load_at(x, y, v, m, i, r, c * N, blockIdx.z);
   p.apply(out, i);
 }
@@ -184,14 +188,29 @@ int row_map(const char* entry, const T* x, const T* y, const float* v, T* out, R
     // measured even (gatedAddChunk) or slower (modulateChunks, 422 against
     // 406 us) that way, and rowGatedAdd's rows do not fit
     const int64_t samples = m.rows / m.per;
+    // gatedAdd's x stays in the caches where most of it fits the 256 MB MALL
+    // until the norm after it reads it again. A block's convert, AdaLN,
+    // gatedAdd, AdaLN, GELU-tanh in graph replays, non-temporal / kept: F32
+    // [7800, 3072] 167.4 / 160.7 us, [16380, 5120] (x 320 MiB) 601.5 / 572.5,
+    // bf16 [8000, 5120] 181.4 / 171.5, [24570, 3072] 289.2 / 279.2, [1000,
+    // 2048] 18.4 / 18.0; at bf16 [65520, 3072] (384 MiB) 751.7 / 749.0, and
+    // gatedAdd alone there 184.8 / 189.2. The other ops' x kept: even or slower
+    // (modulateChunks, gatedAddChunk and rowGatedAdd of [1000, 1536] 12.7 / 14.8).
+    const bool keep = OP == GATED_ADD && values * (int64_t)sizeof(T) <= (int64_t)352 << 20;
     if (OP == GATED_ADD && m.row_chunks % 64 == 0 && m.row_chunks / 64 <= INT32_MAX && m.per <= 65535 &&
         samples <= 65535 && samples * m.per == m.rows) {
-      hipLaunchKernelGGL((row_map_by_row<T, OP>), dim3((unsigned)(m.row_chunks / 64), (unsigned)m.per,
-                         (unsigned)samples), dim3(64), 0, s, x, y, v, out, m);
+      const dim3 grid((unsigned)(m.row_chunks / 64), (unsigned)m.per, (unsigned)samples);
+      if (keep)
+        hipLaunchKernelGGL((row_map_by_row<T, OP, OP == GATED_ADD>), grid, dim3(64), 0, s, x, y, v, out, m);
+      else
+        hipLaunchKernelGGL((row_map_by_row<T, OP, false>), grid, dim3(64), 0, s, x, y, v, out, m);
       return launched(entry);
     }
-    hipLaunchKernelGGL((row_map_chunks<T, OP>), dim3(grid_for(total, kBlock, kOneShotBlocks)), dim3(kBlock), 0, s, x,
-                       y, v, out, m, total);
+    const dim3 grid(grid_for(total, kBlock, kOneShotBlocks));
+    if (keep)
+      hipLaunchKernelGGL((row_map_chunks<T, OP, OP == GATED_ADD>), grid, dim3(kBlock), 0, s, x, y, v, out, m, total);
+    else
+      hipLaunchKernelGGL((row_map_chunks<T, OP, false>), grid, dim3(kBlock), 0, s, x, y, v, out, m, total);
   } else {
     hipLaunchKernelGGL((row_map_values<T, OP>), dim3(grid_for(values, 256, 8192)), dim3(256), 0, s, x, y, v, out, m,
                        values, 1.0 / (double)m.cols);
