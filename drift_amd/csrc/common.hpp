@@ -310,6 +310,10 @@ constexpr int64_t kOneShotBlocks = (int64_t)1 << 30;
 // number below 2^32.
 constexpr int64_t kOneWaveBlocks = ((int64_t)1 << 26) - 1;
 
+// Outputs that the call after reads again are stored through the caches up to
+// the MALL's size, and non-temporally past it.
+constexpr int64_t kKeptBytes = (int64_t)256 << 20;
+
 // Workgroups for a grid-stride launch: enough to fill the chip many times
 // over, never more than the grid allows.
 inline unsigned grid_for(int64_t items, int per_block, int64_t cap = 1 << 20) {

@@ -254,7 +254,14 @@ __global__ void __launch_bounds__(256) convert_kernel(const void* x, void* out, 
 // it: [65520, 3072] to BF16 (1.2 GB) 217.8 -> 177.6 us (6.8 TB/s), [7800,
 // 3072] to F32 29.0 -> 23.6, against 8 values a lane in a resident grid; that
 // in one pass took 192.3 and 30.0, in one-wave blocks 193.3 and 27.6.
-template <bool TO_BF16>
+//
+// KEEP: the output is stored through the caches, for the call that reads it
+// next. Alone that is slower (cvt to BF16 of [16380, 3072] 44.8 -> 47.9, to
+// F32 of [7800, 3072] 21.9 -> 25.8), but a block's convert, AdaLN, gatedAdd,
+// AdaLN, GELU-tanh takes 160.1 -> 155.2 at F32 [7800, 3072], 170.1 -> 160.6 at
+// bf16 [8000, 5120], 278.2 -> 270.6 at [24570, 3072]; 753.4 -> 763.0 at
+// [65520, 3072], whose output is past the MALL.
+template <bool TO_BF16, bool KEEP>
 __global__ void __launch_bounds__(kWave) convert_bf16_waves(const void* x, void* out, int64_t chunks) {
   const int lane = threadIdx.x;
   const int64_t first = (int64_t)blockIdx.x * kWave;
@@ -288,7 +295,8 @@ __global__ void __launch_bounds__(kWave) convert_bf16_waves(const void* x, void*
     const uint32_t r0 = (uint32_t)dpp_move32<0xb1>((int)(odd ? a0 : b0));
     const uint32_t r1 = (uint32_t)dpp_move32<0xb1>((int)(odd ? a1 : b1));
     const u32x4 q = odd ? u32x4{r0, r1, b0, b1} : u32x4{a0, a1, r0, r1};
-    __builtin_nontemporal_store(q, reinterpret_cast<u32x4*>(ob + chunk * 8));
+    if constexpr (KEEP) *reinterpret_cast<u32x4*>(ob + chunk * 8) = q;
+    else __builtin_nontemporal_store(q, reinterpret_cast<u32x4*>(ob + chunk * 8));
   } else {
     const uint4 q = cached_load(xb + chunk * 8);  // 23.6 us non-temporally, 21.8 so ([7800, 3072])
     const uint32_t r0 = (uint32_t)dpp_move32<0xb1>((int)(odd ? q.x : q.z));
@@ -296,8 +304,13 @@ __global__ void __launch_bounds__(kWave) convert_bf16_waves(const void* x, void*
     const uint32_t a0 = odd ? r0 : q.x, a1 = odd ? r1 : q.y, b0 = odd ? q.z : r0, b1 = odd ? q.w : r1;
     const float lo[4] = {bf16_lo(a0), bf16_hi(a0), bf16_lo(a1), bf16_hi(a1)};
     const float hi[4] = {bf16_lo(b0), bf16_hi(b0), bf16_lo(b1), bf16_hi(b1)};
-    Chunk<float>::store(of + lane * 4, lo);
-    Chunk<float>::store(of + 4 * kWave + lane * 4, hi);
+    if constexpr (KEEP) {
+      Chunk<float>::store_cached(of + lane * 4, lo);
+      Chunk<float>::store_cached(of + 4 * kWave + lane * 4, hi);
+    } else {
+      Chunk<float>::store(of + lane * 4, lo);
+      Chunk<float>::store(of + 4 * kWave + lane * 4, hi);
+    }
   }
 }
 
@@ -406,10 +419,16 @@ extern "C" int drift_convert(const void* x, void* out, int64_t n, int32_t kind, 
   const bool bf16 = kind == DRIFT_F32_TO_BF16 || kind == DRIFT_BF16_TO_F32;
   if (bf16 && n % 8 == 0 && aligned16(x) && aligned16(out) && ceil_div(n / 8, kWave) <= kOneWaveBlocks) {
     const dim3 grid((unsigned)ceil_div(n / 8, kWave)), block(kWave);
-    if (kind == DRIFT_F32_TO_BF16)
-      hipLaunchKernelGGL(convert_bf16_waves<true>, grid, block, 0, s, x, out, n / 8);
+    const bool to_bf16 = kind == DRIFT_F32_TO_BF16;
+    const bool keep = n * (to_bf16 ? 2 : 4) <= kKeptBytes;
+    if (to_bf16 && keep)
+      hipLaunchKernelGGL((convert_bf16_waves<true, true>), grid, block, 0, s, x, out, n / 8);
+    else if (to_bf16)
+      hipLaunchKernelGGL((convert_bf16_waves<true, false>), grid, block, 0, s, x, out, n / 8);
+    else if (keep)
+      hipLaunchKernelGGL((convert_bf16_waves<false, true>), grid, block, 0, s, x, out, n / 8);
     else
-      hipLaunchKernelGGL(convert_bf16_waves<false>, grid, block, 0, s, x, out, n / 8);
+      hipLaunchKernelGGL((convert_bf16_waves<false, false>), grid, block, 0, s, x, out, n / 8);
   } else {
     hipLaunchKernelGGL(convert_kernel, dim3(grid_for(n, 256, 8192)), dim3(256), 0, s, x, out, n, kind);
   }

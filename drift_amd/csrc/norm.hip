@@ -163,7 +163,14 @@ __global__ void __launch_bounds__(256) rms_norm_rows(T* x, const T* y, const flo
 //   with the residual 5.0 / 6.1 / 6.0
 // Alone, two waves a SIMD in the resident grid were 1 to 4% slower on the
 // larger of these, three and four up to 15%.
-template <typename T, int K, bool ADD, bool RESIDENT>
+//
+// KEEP: the output is stored through the caches, for the rope that reads it
+// next. RMSNorm and ropeTable (or rope3d) of queries and keys, bf16 [14040,
+// 3072] 122.0 -> 116.2 (125.5 -> 114.4), [12470, 3072] 109.9 -> 104.6; in a
+// dense layer, whose next kernels do not read it, 119.6 -> 131.0 for 4,093
+// tokens of 4096: rows past the resident line, beyond a prompt's chunk, keep
+// it.
+template <typename T, int K, bool ADD, bool RESIDENT, bool KEEP>
 __global__ void __launch_bounds__(kWave) rms_norm_waves(T* x, const T* y, const float* weight, T* out, int64_t rows,
                                                         int cols, float eps, float offset) {
   constexpr int N = Chunk<T>::N;
@@ -230,7 +237,8 @@ __global__ void __launch_bounds__(kWave) rms_norm_waves(T* x, const T* y, const 
         }
 #pragma unroll
         for (int j = 0; j < N; ++j) o[j] = (float)((double)v[j] * factor * ((double)wk[j] + (double)offset));
-        Chunk<T>::store(out + row * cols + c * N, o);
+        if constexpr (KEEP) Chunk<T>::store_cached(out + row * cols + c * N, o);
+        else Chunk<T>::store(out + row * cols + c * N, o);
       }
     }
     if constexpr (!RESIDENT) return;
@@ -256,7 +264,11 @@ __global__ void __launch_bounds__(kWave) rms_norm_waves(T* x, const T* y, const 
 //   bf16 [100000, 128] 38.2 / 10.8 / 10.8 / 10.8 / 11.5
 //   F32 [70000, 72] 21.8 / 10.8 / 9.4 / 9.7 / 10.2
 //   bf16 [4192, 256] 3.5 / 2.5 / - / 3.1 / -; F32 [32, 128] 1.95 / 1.75 / - / 2.2 / -
-template <typename T, int G, int U>
+//
+// KEEP: the output is stored through the caches, for the rope that reads it
+// next (F32: norms, ropes and the cache write of 2,039 tokens of 32 + 8 heads
+// 42.6 -> 40.1, of 5,000 87.4 -> 83.3; BF16 moved 2% either way by shape).
+template <typename T, int G, int U, bool KEEP>
 __global__ void __launch_bounds__(kWave) rms_norm_groups(const T* x, const float* weight, T* out, int64_t rows,
                                                          int cols, float eps, float offset) {
   constexpr int N = Chunk<T>::N;
@@ -280,7 +292,10 @@ __global__ void __launch_bounds__(kWave) rms_norm_groups(const T* x, const float
     const int64_t row = first + u * kRows;
 #pragma unroll
     for (int j = 0; j < N; ++j) o[j] = (float)((double)v[j] * factor * ((double)w[j] + (double)offset));
-    if (inside && row < rows) Chunk<T>::store(out + row * cols + c, o);
+    if (inside && row < rows) {
+      if constexpr (KEEP) Chunk<T>::store_cached(out + row * cols + c, o);
+      else Chunk<T>::store(out + row * cols + c, o);
+    }
   }
 }
 
@@ -976,17 +991,23 @@ bool rms_waves_launch(T* x, const T* y, const float* weight, T* out, int64_t row
   // against 130.3 at one a SIMD; F32 and the residual 1% faster at one)
   const int64_t waves = sizeof(T) == 2 && !y ? 2 * kSimds : kSimds;
   const dim3 grid((unsigned)(resident ? std::min(rows, waves) : rows)), block(kWave);
+  const bool keep = !y && rows >= 7 * kSimds && rows * cols * (int64_t)sizeof(T) <= kKeptBytes;
 #define DRIFT_RMS_WAVES(K, ADD)                                                                                     \
   if (per_lane <= K) {                                                                                              \
     if constexpr (sizeof(T) == 2 || !ADD) { /* F32 with the residual is never resident */                           \
+      if (keep) {                                                                                                   \
+        hipLaunchKernelGGL((rms_norm_waves<T, K, ADD, true, !ADD>), grid, block, 0, s, x, y, weight, out, rows,     \
+                           cols, eps, offset);                                                                      \
+        return true;                                                                                                \
+      }                                                                                                             \
       if (resident) {                                                                                               \
-        hipLaunchKernelGGL((rms_norm_waves<T, K, ADD, true>), grid, block, 0, s, x, y, weight, out, rows, cols,     \
-                           eps, offset);                                                                            \
+        hipLaunchKernelGGL((rms_norm_waves<T, K, ADD, true, false>), grid, block, 0, s, x, y, weight, out, rows,    \
+                           cols, eps, offset);                                                                      \
         return true;                                                                                                \
       }                                                                                                             \
     }                                                                                                               \
-    hipLaunchKernelGGL((rms_norm_waves<T, K, ADD, false>), grid, block, 0, s, x, y, weight, out, rows, cols, eps,   \
-                       offset);                                                                                     \
+    hipLaunchKernelGGL((rms_norm_waves<T, K, ADD, false, false>), grid, block, 0, s, x, y, weight, out, rows, cols, \
+                       eps, offset);                                                                                \
     return true;                                                                                                    \
   }
   if (y) {
@@ -1014,12 +1035,19 @@ void rms_groups_launch(const T* x, const float* weight, T* out, int64_t rows, in
                        hipStream_t s) {
   constexpr int kRows = kWave / G;
   const int64_t waves = ceil_div(rows, kRows);
-  if (waves <= 4 * kSimds)
-    hipLaunchKernelGGL((rms_norm_groups<T, G, 1>), dim3((unsigned)waves), dim3(kWave), 0, s, x, weight, out, rows,
-                       cols, eps, offset);
+  const bool keep = sizeof(T) == 4 && rows * cols * (int64_t)sizeof(T) <= kKeptBytes;
+  const bool one = waves <= 4 * kSimds;
+  const dim3 grid((unsigned)(one ? waves : ceil_div(waves, 2))), block(kWave);
+  if (one && keep)
+    hipLaunchKernelGGL((rms_norm_groups<T, G, 1, sizeof(T) == 4>), grid, block, 0, s, x, weight, out, rows, cols, eps,
+                       offset);
+  else if (one)
+    hipLaunchKernelGGL((rms_norm_groups<T, G, 1, false>), grid, block, 0, s, x, weight, out, rows, cols, eps, offset);
+  else if (keep)
+    hipLaunchKernelGGL((rms_norm_groups<T, G, 2, sizeof(T) == 4>), grid, block, 0, s, x, weight, out, rows, cols, eps,
+                       offset);
   else
-    hipLaunchKernelGGL((rms_norm_groups<T, G, 2>), dim3((unsigned)ceil_div(waves, 2)), dim3(kWave), 0, s, x, weight,
-                       out, rows, cols, eps, offset);
+    hipLaunchKernelGGL((rms_norm_groups<T, G, 2, false>), grid, block, 0, s, x, weight, out, rows, cols, eps, offset);
 }
 
 template <typename T>
