@@ -155,6 +155,18 @@ def test_convert_waves(hip, n):
     assert bool((back[n:] == -3).all()), "nothing past the end"
 
 
+@pytest.mark.parametrize("to", [torch.bfloat16, torch.float32])
+def test_convert_past_the_kept_size(hip, to):
+    # an output past 256 MiB, stored non-temporally; a last wave part full
+    n = (1 << 28) // (2 if to == torch.bfloat16 else 4) + 264
+    step(f"convert {n} values to {to}")
+    x = torch.randn(n, device=DEV)
+    x = x if to == torch.bfloat16 else x.to(torch.bfloat16)
+    out = torch.empty(n, dtype=to, device=DEV)
+    hip.convert(x, out)
+    assert torch.equal(out, x.to(to)), "round to nearest even, as torch converts"
+
+
 def test_convert_fp8_e4m3_to_f32(hip):
     # the reference's conversion code 4 (ops/HipBase.scala:268-274): every
     # E4M3 "fn" byte, as uint8 or torch's float8_e4m3fn, against the

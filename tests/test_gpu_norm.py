@@ -153,6 +153,21 @@ def test_rms_norm_row_splits(hip, rows, cols, dtype, add):
     (assert_f32 if dtype == "f32" else assert_bf16)(want, host(out), what=f"rmsNorm [{rows}, {cols}]")
 
 
+@pytest.mark.parametrize("rows,cols,dtype", [(530001, 128, torch.float32), (33001, 8192, torch.bfloat16),
+                                             (16500, 4096, torch.float32)])
+def test_rms_norm_past_the_kept_size(hip, rows, cols, dtype):
+    # outputs past 256 MiB, stored non-temporally: rows as they norm alone
+    step(f"rmsNorm {dtype} [{rows}, {cols}]")
+    x = torch.randn((rows, cols), device=DEV).to(dtype)
+    w = torch.randn(cols, device=DEV)
+    out = torch.empty_like(x)
+    hip.rmsNorm(x, w, 1e-6, 0.0, out)
+    for first in (0, rows // 2, rows - 7):
+        few = torch.empty((7, cols), dtype=dtype, device=DEV)
+        hip.rmsNorm(x[first:first + 7], w, 1e-6, 0.0, few)
+        assert torch.equal(few, out[first:first + 7]), f"rows from {first}"
+
+
 # (rows, groups, width) of the group norm, one case for each way the library
 # splits a row: a thread per narrow row (<= 32 values), the scalar path
 # (widths not whole 16-byte chunks), a wave or a 4-wave group per row in a
