@@ -236,18 +236,22 @@ struct RocmFp4 {  // RocmFp4.scala:45-62: Codebook(q) * halfScale, a scale per h
   }
 };
 
-// Dense rows: 8 values from 16 or 32 bytes (16-byte aligned rows).
+// Dense rows: 8 values from 16 or 32 bytes (16-byte aligned rows). A row may
+// be a whole table (decode_launch) of up to INT32_MAX values, so a chunk's
+// byte offset takes 64 bits.
 template <int FORMAT>
 struct Dense {
   static constexpr int kValues = 1, kBytes = FORMAT == DRIFT_F32 ? 4 : 2, kAlign = 16;
   static constexpr int kLut = 0;
+  static constexpr __host__ __device__ int64_t chunk_at(int c) { return (int64_t)c * (8 * kBytes); }
   template <int A = kAlign>
   __device__ static void decode(const uint8_t* b, int c, float (&v)[8], const float* lut) {
     if constexpr (FORMAT == DRIFT_F32) {
-      float4 a = *reinterpret_cast<const float4*>(b + 32 * c), z = *reinterpret_cast<const float4*>(b + 32 * c + 16);
+      const float4* p = reinterpret_cast<const float4*>(b + chunk_at(c));
+      const float4 a = p[0], z = p[1];
       v[0] = a.x, v[1] = a.y, v[2] = a.z, v[3] = a.w, v[4] = z.x, v[5] = z.y, v[6] = z.z, v[7] = z.w;
     } else {
-      const uint4 q = *reinterpret_cast<const uint4*>(b + 16 * c);
+      const uint4 q = *reinterpret_cast<const uint4*>(b + chunk_at(c));
       const uint32_t words[4] = {q.x, q.y, q.z, q.w};
 #pragma unroll
       for (int k = 0; k < 8; ++k) {
@@ -257,6 +261,11 @@ struct Dense {
     }
   }
 };
+
+// the last chunk of the largest whole table (a 32-bit product would wrap, and
+// fail here as no constant)
+static_assert(Dense<DRIFT_F32>::chunk_at(INT32_MAX / 8) / 32 == INT32_MAX / 8 &&
+              Dense<DRIFT_F16>::chunk_at(INT32_MAX / 8) / 16 == INT32_MAX / 8);
 
 // ---------------------------------------------------------------- kernels
 

@@ -4,7 +4,10 @@ BF16 a tensor), so the offsets of the last rows need 64 bits. The rows
 before, across and after value 2^31, and the first and last, are checked
 against the oracle at the bars of the small cases: 1 bf16 ulp for the
 activation, the norms and the rotations, exact for gatedAdd (one rounding of
-the F32 result, as the reference's convert)."""
+the F32 result, as the reference's convert).
+
+And whole tables decoded at the sizes where an offset outgrows 32 bits: a
+dense table's bytes pass 2^31 long before its values do."""
 
 import numpy as np
 import pytest
@@ -134,3 +137,31 @@ def test_query_key_norm_rope_in_place(hip):
     want_q, want_k = o.qk_norm_rope_bf16(qb, kb, qw, kw, positions[check], 1e-6, 0.0, 1e6, dim)
     assert_bf16(want_q, rows_of(q, check), what="queries past 2^31")
     assert_bf16(want_k, rows_of(k, check), what="keys")
+
+
+# dequantize takes a whole table of up to 2^31 - 1 values as one row. Dense
+# tables past 2^31 bytes and past 2^32 (F32 from 2^29 values on, F16 and BF16
+# from 2^30), and one just under 2^31 values; a format decoded by chunks and
+# one by runs just under 2^31 values; and over the line, where rows decode by
+# themselves.
+@pytest.mark.parametrize("name,rows,cols", [
+    ("F32", (1 << 29) // 4096 + 3, 4096), ("F32", (1 << 30) // 5120 + 3, 5120), ("F32", LIMIT // 4096 - 1, 4096),
+    ("F16", (1 << 30) // 8192 + 3, 8192), ("BF16", (1 << 30) // 5120 + 3, 5120), ("BF16", LIMIT // 4096 - 1, 4096),
+    ("Q4_0", LIMIT // 4096 - 1, 4096), ("Q8_0", LIMIT // 5120, 5120), ("Q4_K", LIMIT // 4096 - 1, 4096),
+    ("F16", LIMIT // 4096 + 1, 4096), ("Q4_0", LIMIT // 4096 + 1, 4096), ("Q4_K", LIMIT // 4096 + 1, 4096),
+])
+def test_whole_table(hip, name, rows, cols):
+    step(f"dequantize {name} [{rows}, {cols}] to bf16")
+    period = 61  # the table repeats this many rows
+    raw = o.quant_table(name, period, cols, np.random.default_rng(513))
+    want = o.to_bf16(o.embedding(name, raw, period, cols, np.arange(period, dtype=np.int32)))
+    data = torch.from_numpy(np.ascontiguousarray(raw)).to(DEV).repeat(rows // period + 1, 1)[:rows].contiguous()
+    out = torch.full((rows, cols), -3, dtype=torch.bfloat16, device=DEV)
+    hip.dequantize(d.StoredTable(data, d.STORAGE_TYPES[name], cols), out)
+    del data
+    tile = torch.from_numpy(want.view(np.int16)).to(DEV)
+    bits = out.view(torch.int16)
+    whole = rows // period
+    wrong = (bits[:whole * period].view(whole, period, cols) != tile).any(2).view(-1)
+    wrong = torch.cat((wrong, (bits[whole * period:] != tile[:rows - whole * period]).any(1)))
+    assert not bool(wrong.any()), f"{int(wrong.sum())} of {rows} rows differ, first {int(wrong.nonzero()[0])}"
