@@ -523,22 +523,44 @@ __global__ void __launch_bounds__(256) layer_norm_rows(const T* x, const float* 
 // 8.4, [4830, 1280] 14.9 / 12.7 / 9.8, [9000, 1024] 19.1 / 18.1 / 15.5; group / this
 // [2000, 2048] 9.2 / 7.9, [1100, 4096] 11.6 / 11.1; but [1100, 1024] 4.0 / 4.7
 // and [600, 1152] 4.2 / 4.5: up to 1,024 rows or 2^19 chunks keep the group.
-template <int K>
-__global__ void __launch_bounds__(kWave) layer_norm_waves(const float* x, const float* weight, const float* bias,
-                                                          float* out, int64_t rows, int cols, float eps) {
-  constexpr int N = 4;
-  const int lane = threadIdx.x;
+//
+// MODULATE (as layer_norm_rows): AdaLN rows of 4,097 to 5,120 values, past
+// adaln_launch's, a sample's rows by blockIdx.y, in 256-thread blocks. Us a
+// launch, events around it, its input in HBM behind a matrix product / just
+// written, four-wave group against one-wave blocks and these: bf16 [16380,
+// 5120] 105.3 / 88.2, 80.9 / 67.4, 80.7 / 66.2; bf16 [4000, 5120] 30.7 / 26.0,
+// 23.1 / 23.0, 22.2 / 22.0; F32 [16380, 5120] 183.8 / 155.9, 130.8 / 129.1,
+// 131.1 / 130.5; F32 [1700, 5120] 24.7 / 20.5, 18.8 / 18.8, 18.8 / 18.5. At
+// 1,500 rows bf16 15.3 / 14.0 in the group, 14.4 / 14.1 here, and with the
+// input in HBM behind reads 15.7 and 17.0 (F32 21.3 and 24.7): up to 1,536
+// rows (one and a half a SIMD) keep the group.
+template <bool MODULATE>
+constexpr int kNormBlock = MODULATE ? 256 : kWave;
+
+template <typename T, int K, bool MODULATE>
+__global__ void __launch_bounds__(kNormBlock<MODULATE>) layer_norm_waves(const T* x, const float* weight,
+                                                                       const float* bias, T* out, int64_t rows,
+                                                                       int cols, int64_t rows_per_sample, float eps) {
+  constexpr int N = Chunk<T>::N;
+  const int lane = threadIdx.x & 63;
   const int chunks = cols / N;
-  const int64_t row = blockIdx.x;
-  uint4 raw[K];
+  int64_t row = (int64_t)blockIdx.x * (kNormBlock<MODULATE> / kWave) + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  if constexpr (MODULATE) {
+    if (row >= rows_per_sample) return;
+    row += (int64_t)blockIdx.y * rows_per_sample;
+    if (row >= rows) return;
+    weight += (int64_t)blockIdx.y * cols;
+    bias += (int64_t)blockIdx.y * cols;
+  }
+  typename Chunk<T>::Raw raw[K];
 #pragma unroll
-  for (int k = 0; k < K; ++k) raw[k] = stream_load(x + row * cols + min(k * kWave + lane, chunks - 1) * N);
+  for (int k = 0; k < K; ++k) raw[k] = Chunk<T>::load_raw(x + row * cols + min(k * kWave + lane, chunks - 1) * N);
   constexpr int kSums = K < 4 ? K : 4;
   double sums[4] = {0.0, 0.0, 0.0, 0.0};
 #pragma unroll
   for (int k = 0; k < K; ++k) {
     float v[N];
-    Chunk<float>::unpack(raw[k], v);
+    Chunk<T>::unpack(raw[k], v);
     if (k * kWave + lane < chunks) {
 #pragma unroll
       for (int j = 0; j < N; ++j) sums[k % 4] += (double)v[j];
@@ -553,7 +575,7 @@ __global__ void __launch_bounds__(kWave) layer_norm_waves(const float* x, const 
   for (int k = 0; k < K; ++k) {
     opaque(raw[k]);
     float v[N];
-    Chunk<float>::unpack(raw[k], v);
+    Chunk<T>::unpack(raw[k], v);
     if (k * kWave + lane < chunks) {
 #pragma unroll
       for (int j = 0; j < N; ++j) {
@@ -571,15 +593,20 @@ __global__ void __launch_bounds__(kWave) layer_norm_waves(const float* x, const 
     if (c < chunks) {
       opaque(raw[k]);
       float v[N], w[N], b[N], o[N];
-      Chunk<float>::unpack(raw[k], v);
-      if (weight) load_f32<N>(weight + c * N, w);
-      if (bias) load_f32<N>(bias + c * N, b);
+      Chunk<T>::unpack(raw[k], v);
+      if (MODULATE || weight) load_f32<N>(weight + c * N, w);
+      if (MODULATE || bias) load_f32<N>(bias + c * N, b);
 #pragma unroll
       for (int j = 0; j < N; ++j) {
-        const double normal = ((double)v[j] - mean) * factor;
-        o[j] = (float)(normal * (weight ? (double)w[j] : 1.0) + (bias ? (double)b[j] : 0.0));
+        if constexpr (MODULATE) {
+          const float n = (float)fma((double)v[j] - mean, factor, 0.0);
+          o[j] = (float)fma((double)n, 1.0 + (double)w[j], (double)b[j]);
+        } else {
+          const double normal = ((double)v[j] - mean) * factor;
+          o[j] = (float)(normal * (weight ? (double)w[j] : 1.0) + (bias ? (double)b[j] : 0.0));
+        }
       }
-      Chunk<float>::store(out + row * cols + c * N, o);
+      Chunk<T>::store(out + row * cols + c * N, o);
     }
   }
 }
@@ -621,15 +648,11 @@ __global__ void __launch_bounds__(256) layer_norm_rows_scalar(const T* x, const 
   }
 }
 
-// AdaLN, one wave per row, B / 64 rows of one sample per block (grid.y =
-// sample), the grid covering the rows in one pass: F32 rows, in one-wave
-// blocks, and BF16 rows past adaln_resident's registers, in 256-thread blocks
-// ([16380, 5120] 73.7 us, one-wave blocks 77.4, layer_norm_rows 99.2). F32, us
-// a launch in graph replays, 256-thread / one-wave blocks: [1500, 3840] 14.4 /
-// 9.5, [7800, 3072] 36.9 / 37.6, [8190, 1536] 19.2 / 18.6; [4000, 5120] 44.0
-// in layer_norm_rows, 28.1. Each lane reads its
-// chunks' scale and shift from the sample's rows (cached: every row of the
-// sample reads them).
+// F32 AdaLN, one wave per row, B / 64 rows of one sample per block (grid.y =
+// sample), the grid covering the rows in one pass. Each lane reads its chunks' scale and shift
+// from the sample's rows (cached: every row of the sample reads them). Us a
+// launch in graph replays, in 256-thread blocks / in one-wave blocks: [1500,
+// 3840] 14.4 / 9.5, [7800, 3072] 36.9 / 37.6, [8190, 1536] 19.2 / 18.6.
 //
 // The mean and variance come from one pass over the row about its first
 // value x0 (sums of d = x - x0 and d^2): the same as the reference's two
@@ -637,13 +660,13 @@ __global__ void __launch_bounds__(256) layer_norm_rows_scalar(const T* x, const 
 // most. The arithmetic is the reference's, in double: n = float((x - mean) *
 // factor) is layerNorm's F32 result, out = n * (1 + scale) + shift rounded
 // once, as modulate.
-constexpr int kAdalnMaxCols = 5120;
+constexpr int kAdalnMaxCols = 4096;
 
-template <typename T, int K, bool FULL, int B>
-__global__ void __launch_bounds__(B) adaln_waves(const T* x, const float* scale, const float* shift, T* out,
-                                                    int64_t rows, int cols, int64_t rows_per_sample, float eps) {
-  constexpr int N = Chunk<T>::N;
-  using Raw = typename Chunk<T>::Raw;
+template <int K, bool FULL, int B>
+__global__ void __launch_bounds__(B) adaln_waves(const float* x, const float* scale, const float* shift, float* out,
+                                                 int64_t rows, int cols, int64_t rows_per_sample, float eps) {
+  constexpr int N = 4;
+  using Raw = uint4;
   const int chunks = FULL ? K * kWave : cols / N;
   const int64_t sample = blockIdx.y;
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -653,17 +676,17 @@ __global__ void __launch_bounds__(B) adaln_waves(const T* x, const float* scale,
 #pragma unroll
   for (int k = 0; k < K; ++k) {
     const int c = k * kWave + lane;
-    if (FULL || c < chunks) raw[k] = Chunk<T>::load_raw(x + row * cols + c * N);
+    if (FULL || c < chunks) raw[k] = Chunk<float>::load_raw(x + row * cols + c * N);
   }
   float first_value[N];
-  Chunk<T>::unpack(raw[0], first_value);
+  Chunk<float>::unpack(raw[0], first_value);
   const double x0 = (double)__shfl(first_value[0], 0);
   double s1 = 0.0, s2 = 0.0;
 #pragma unroll
   for (int k = 0; k < K; ++k) {
     if (FULL || k * kWave + lane < chunks) {
       float v[N];
-      Chunk<T>::unpack(raw[k], v);
+      Chunk<float>::unpack(raw[k], v);
 #pragma unroll
       for (int j = 0; j < N; ++j) {
         const double d = (double)v[j] - x0;
@@ -688,7 +711,7 @@ __global__ void __launch_bounds__(B) adaln_waves(const T* x, const float* scale,
     if (FULL || c < chunks) {
       opaque(raw[k]);
       float v[N], o[N], a[N], b[N];
-      Chunk<T>::unpack(raw[k], v);
+      Chunk<float>::unpack(raw[k], v);
       load_f32<N>(sc + c * N, a);
       load_f32<N>(sh + c * N, b);
 #pragma unroll
@@ -696,7 +719,7 @@ __global__ void __launch_bounds__(B) adaln_waves(const T* x, const float* scale,
         const float n = (float)fma((double)v[j], factor, offset);
         o[j] = (float)fma((double)n, 1.0 + (double)a[j], (double)b[j]);
       }
-      Chunk<T>::store(out + row * cols + c * N, o);
+      Chunk<float>::store(out + row * cols + c * N, o);
     }
   }
 }
@@ -1161,11 +1184,10 @@ void adaln_resident_launch(const uint16_t* x, const float* scale, const float* s
                      rows_per_sample, eps, per_sample);
 }
 
-// AdaLN of rows of whole 16-byte chunks, at most 5120 values: BF16 through
-// adaln_resident up to 4096 values and adaln_waves beyond, for more than 1,024
-// rows (fewer are faster four waves a row: [552, 5120] 6.1 us against 6.4);
-// F32 through adaln_resident_f32 or adaln_waves (their comments' figures).
-// Returns -1 when the shape does not qualify.
+// AdaLN of rows of whole 16-byte chunks, at most 4096 values: BF16 through
+// adaln_resident, F32 through adaln_resident_f32 or adaln_waves (their
+// comments' figures), which take a row's sums alike. Returns -1 when the shape
+// does not qualify.
 template <typename T>
 int adaln_launch(const T* x, const float* scale, const float* shift, T* out, int64_t rows, int cols,
                  int64_t rows_per_sample, float eps, hipStream_t s) {
@@ -1174,7 +1196,6 @@ int adaln_launch(const T* x, const float* scale, const float* shift, T* out, int
   if (cols % N != 0 || cols > kAdalnMaxCols || samples > 65535 || rows_per_sample > kOneWaveBlocks) return -1;
   const int chunks = cols / N;
   const int per_lane = (int)ceil_div(chunks, kWave);
-  if (per_lane > 4096 / N / kWave && rows <= kSimds) return -1;
   if constexpr (sizeof(T) == 2) {
 #define DRIFT_ADALN_CASE(K)                                                                                   \
   if (per_lane <= K) {                                                                                        \
@@ -1191,10 +1212,6 @@ int adaln_launch(const T* x, const float* scale, const float* shift, T* out, int
     DRIFT_ADALN_CASE(6)
     DRIFT_ADALN_CASE(8)
 #undef DRIFT_ADALN_CASE
-    const dim3 grid((unsigned)ceil_div(rows_per_sample, 4), (unsigned)samples);
-    hipLaunchKernelGGL((adaln_waves<T, 10, false, 256>), grid, dim3(256), 0, s, x, scale, shift, out, rows, cols,
-                       rows_per_sample, eps);
-    return 0;
   } else {
     if (per_lane <= 12 && (rows <= kSimds || rows >= 7 * kSimds)) {
       // rows shared out as evenly as they go
@@ -1221,10 +1238,10 @@ int adaln_launch(const T* x, const float* scale, const float* shift, T* out, int
 #define DRIFT_ADALN_CASE(K)                                                                                      \
   if (per_lane <= K) {                                                                                           \
     if (chunks == K * kWave)                                                                                     \
-      hipLaunchKernelGGL((adaln_waves<T, K, true, kWave>), grid, block, 0, s, x, scale, shift, out, rows, cols,  \
+      hipLaunchKernelGGL((adaln_waves<K, true, kWave>), grid, block, 0, s, x, scale, shift, out, rows, cols,  \
                          rows_per_sample, eps);                                                                  \
     else                                                                                                         \
-      hipLaunchKernelGGL((adaln_waves<T, K, false, kWave>), grid, block, 0, s, x, scale, shift, out, rows, cols, \
+      hipLaunchKernelGGL((adaln_waves<K, false, kWave>), grid, block, 0, s, x, scale, shift, out, rows, cols, \
                          rows_per_sample, eps);                                                                  \
     return 0;                                                                                                    \
   }
@@ -1236,7 +1253,6 @@ int adaln_launch(const T* x, const float* scale, const float* shift, T* out, int
     DRIFT_ADALN_CASE(8)
     DRIFT_ADALN_CASE(12)
     DRIFT_ADALN_CASE(16)
-    DRIFT_ADALN_CASE(20)
 #undef DRIFT_ADALN_CASE
   }
   return -1;
@@ -1263,15 +1279,25 @@ int layer_norm(const char* entry, const T* x, const float* weight, const float* 
                        bias, out, rows, (int)cols, rows_per_sample, eps);
     return launched(entry);
   }
-  if constexpr (!MODULATE) {
-    const int per_lane = (int)ceil_div(cols / 4, kWave);
+  const int per_lane = (int)ceil_div(cols / Chunk<T>::N, kWave);
+  if constexpr (MODULATE) {
+    const int64_t samples = ceil_div(rows, rows_per_sample);
+    if (plan.waves == 4 && cols <= 5120 && rows > 3 * kSimds / 2 && samples <= 65535 &&
+        rows_per_sample <= kOneWaveBlocks) {
+      const dim3 grid((unsigned)ceil_div(rows_per_sample, 4), (unsigned)samples);
+      hipLaunchKernelGGL((layer_norm_waves<T, 5120 / Chunk<T>::N / kWave, true>), grid, dim3(kNormBlock<true>), 0, s, x,
+                         weight, bias, out, rows, cols, rows_per_sample, eps);
+      return launched(entry);
+    }
+  } else {
     if (plan.waves == 4 && rows > kSimds && rows * (cols / 4) >= (1 << 19) && rows <= kOneWaveBlocks &&
         per_lane <= 20) {
       const dim3 one((unsigned)rows), block(kWave);
-#define DRIFT_LN_WAVES(K)                                                                                \
-  if (per_lane <= K) {                                                                                   \
-    hipLaunchKernelGGL(layer_norm_waves<K>, one, block, 0, s, x, weight, bias, out, rows, cols, eps);           \
-    return launched(entry);                                                                                     \
+#define DRIFT_LN_WAVES(K)                                                                                     \
+  if (per_lane <= K) {                                                                                        \
+    hipLaunchKernelGGL((layer_norm_waves<T, K, false>), one, block, 0, s, x, weight, bias, out, rows, cols,    \
+                       rows_per_sample, eps);                                                                 \
+    return launched(entry);                                                                                   \
   }
       DRIFT_LN_WAVES(4)
       DRIFT_LN_WAVES(5)

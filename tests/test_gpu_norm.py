@@ -290,9 +290,36 @@ def test_layer_norm_modulate(hip, rows, cols, samples, dtype):
     (1024, 1536, 1, "f32"), (1025, 1536, 1, "f32"), (7167, 260, 1, "f32"), (7168, 260, 3, "f32"), (700, 3076, 7, "f32"),
     (9000, 772, 2, "f32"), (1030, 3840, 1, "f32"), (1026, 4100, 2, "f32"), (1100, 5120, 1, "f32"), (30, 5116, 2, "f32"),
     (1025, 5120, 3, "bf16"), (1030, 4104, 1, "bf16"), (1024, 5120, 2, "bf16"), (1200, 5128, 1, "bf16"),
+    (1536, 4100, 1, "f32"), (1537, 4100, 2, "f32"), (1601, 5116, 5, "f32"), (1537, 5120, 1, "bf16"),
+    (1603, 4104, 3, "bf16"), (1540, 5128, 1, "bf16"),
 ])
 def test_layer_norm_modulate_row_splits(hip, rows, cols, samples, dtype):
     test_layer_norm_modulate(hip, rows, cols, samples, dtype)
+
+
+@pytest.mark.parametrize("dtype", ["f32", "bf16"])
+@pytest.mark.parametrize("cols", [768, 1028, 3072, 4096, 4104, 5120, 5128])
+def test_layer_norm_modulate_does_not_depend_on_the_batch(hip, dtype, cols):
+    # the same rows alone, and in batches either side of every line between a
+    # row's splits. Each row's first value stands far out, so that two orders
+    # or methods of its sums (1e-13 of the variance apart) round some of its
+    # values apart
+    step(f"layerNormModulate {dtype} rows of {cols}, alone and in batches")
+    x = gaussian(17, (7200, cols))
+    x[:, 0] = 1 << 20
+    to, host = (dev_f32, host_f32) if dtype == "f32" else (lambda a: dev_bf16(bf16_input(a)), host_bits)
+    xd = to(x)
+    s, sh = dev_f32(0.1 * gaussian(18, (1, cols))), dev_f32(0.1 * gaussian(19, (1, cols)))
+    results = {}
+    for rows in (900, 1026, 1540, 7200):
+        out = torch.empty_like(xd[:rows])
+        hip.layerNormModulate(xd[:rows], s, sh, 1e-6, out, rows)
+        results[rows] = host(out[:900])
+    alone = torch.empty_like(xd[:7])
+    hip.layerNormModulate(xd[893:900], s, sh, 1e-6, alone, 7)
+    for rows, got in results.items():
+        assert np.array_equal(results[900].view(np.uint8), got.view(np.uint8)), f"900 rows, alone and of {rows}"
+    assert np.array_equal(results[900][893:].view(np.uint8), host(alone).view(np.uint8)), "seven rows alone"
 
 
 @pytest.mark.parametrize("shape", [(1024, 2052), (2045, 1028), (1300, 2308), (1100, 3072), (1030, 5120), (1050, 5124),
