@@ -72,6 +72,14 @@ __device__ __forceinline__ double row_factor(double squares, int cols, float eps
   return eps > 0.0f ? inverse_sqrt<true>(mean) : inverse_sqrt(mean);
 }
 
+// The variance from a row's moments about one of its values. Rounding may take
+// it below zero; a NaN (of a row with an infinity or a NaN in it) stays one, as
+// two passes give and the reference writes.
+__device__ __forceinline__ double moment_variance(double s2, double m1, double inverse_cols) {
+  const double v = fma(s2, inverse_cols, -(m1 * m1));
+  return v < 0.0 ? 0.0 : v;
+}
+
 // With q.xq, out is quantized too as it is written (quantize_chunk; cols a
 // multiple of 32, so a row holds whole blocks).
 template <typename T, int K, int W>
@@ -700,7 +708,7 @@ __global__ void __launch_bounds__(B) adaln_waves(const float* x, const float* sc
   const double inverse_cols = 1.0 / (double)cols;
   const double m1 = s1 * inverse_cols;  // mean - x0
   const double mean = x0 + m1;
-  const double variance = fmax(fma(s2, inverse_cols, -(m1 * m1)), 0.0);
+  const double variance = moment_variance(s2, m1, inverse_cols);
   const double factor = eps > 0.0f ? inverse_sqrt<true>(variance + (double)eps) : inverse_sqrt(variance + (double)eps);
   const double offset = -mean * factor;
   const float* sc = scale + sample * cols;
@@ -783,7 +791,7 @@ __global__ void __launch_bounds__(kWave) adaln_resident_f32(const float* x, cons
     s2 = group_sum<64>(s2);
     const double m1 = s1 * inverse_cols;
     const double mean = x0 + m1;
-    const double variance = fmax(fma(s2, inverse_cols, -(m1 * m1)), 0.0);
+    const double variance = moment_variance(s2, m1, inverse_cols);
     const double var_eps = variance + (double)eps;
     const double factor = eps > 0.0f ? inverse_sqrt<true>(var_eps) : inverse_sqrt(var_eps);
     const double offset = -mean * factor;
@@ -883,7 +891,7 @@ __global__ void __launch_bounds__(256) adaln_resident(const uint16_t* x, const f
     // division (each within a double ulp or two)
     const double m1 = s1 * inverse_cols;  // mean - x0
     const double mean = (double)x0 + m1;
-    const double variance = fmax(fma(s2, inverse_cols, -(m1 * m1)), 0.0);
+    const double variance = moment_variance(s2, m1, inverse_cols);
     const double var_eps = variance + (double)eps;
     const double factor = eps > 0.0f ? inverse_sqrt<true>(var_eps) : inverse_sqrt(var_eps);
     const double offset = -mean * factor;

@@ -322,6 +322,35 @@ def test_layer_norm_modulate_does_not_depend_on_the_batch(hip, dtype, cols):
     assert np.array_equal(results[900][893:].view(np.uint8), host(alone).view(np.uint8)), "seven rows alone"
 
 
+# rows with an infinity or a NaN are NaN throughout (the mean is no number),
+# and their neighbours as without them: every way AdaLN splits a row, the value
+# first in its row, inside and last
+@pytest.mark.parametrize("dtype", ["f32", "bf16"])
+@pytest.mark.parametrize("rows,cols,samples", [(40, 3072, 2), (1030, 1536, 1), (7200, 768, 2), (30, 4104, 1),
+                                               (1600, 5120, 2), (30, 6144, 1), (20, 77, 2)])
+def test_layer_norm_modulate_of_rows_that_are_not_finite(hip, rows, cols, samples, dtype):
+    step(f"layerNormModulate {dtype} [{rows}, {cols}] with rows that are not finite")
+    per = -(-rows // samples)
+    x = gaussian(20, (rows, cols))
+    at = {3: (0, np.inf), 5: (cols // 2, np.inf), 6: (cols - 1, -np.inf), 8: (1, np.nan), rows - 1: (cols // 3, -np.inf)}
+    for row, (col, value) in at.items():
+        x[row, col] = value
+    x[10, [2, cols - 2]] = [np.inf, -np.inf]
+    s, sh = (0.1 * gaussian(21, (samples, cols))).astype(np.float32), (0.1 * gaussian(22, (samples, cols))).astype(np.float32)
+    if dtype == "f32":
+        out = torch.empty((rows, cols), dtype=torch.float32, device=DEV)
+        hip.layerNormModulate(dev_f32(x), dev_f32(s), dev_f32(sh), 1e-6, out, per)
+        got = host_f32(out)
+        assert_f32(o.layer_norm_modulate(x, s, sh, per, 1e-6), got, what="AdaLN f32")
+    else:
+        xb = bf16_input(x)
+        out = torch.empty((rows, cols), dtype=torch.bfloat16, device=DEV)
+        hip.layerNormModulate(dev_bf16(xb), dev_f32(s), dev_f32(sh), 1e-6, out, per)
+        got = o.from_bf16(host_bits(out))
+        assert_bf16(o.layer_norm_modulate_bf16(xb, s, sh, per, 1e-6), host_bits(out), what="AdaLN bf16")
+    assert np.isnan(got[sorted([*at, 10])]).all()
+
+
 @pytest.mark.parametrize("shape", [(1024, 2052), (2045, 1028), (1300, 2308), (1100, 3072), (1030, 5120), (1050, 5124),
                                    (1025, 2048), (4100, 1024), (2030, 1028)])
 @pytest.mark.parametrize("affine", [(False, False), (True, False), (False, True), (True, True)])
