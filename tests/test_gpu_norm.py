@@ -322,6 +322,25 @@ def test_layer_norm_modulate_does_not_depend_on_the_batch(hip, dtype, cols):
     assert np.array_equal(results[900][893:].view(np.uint8), host(alone).view(np.uint8)), "seven rows alone"
 
 
+@pytest.mark.parametrize("dtype", ["f32", "bf16"])
+@pytest.mark.parametrize("rows,cols", [(9, 64), (1100, 3072), (1600, 5120), (3, 77)])
+def test_layer_norm_modulate_samples_of_more_rows_than_there_are(hip, dtype, rows, cols):
+    # up to the largest count the entry point takes, more than a grid holds:
+    # the result is a sample's of exactly the rows, to the last bit (first
+    # values far out, as above, show another split's sums)
+    step(f"layerNormModulate {dtype} [{rows}, {cols}], samples of up to 2^63 - 1 rows")
+    x = dev_f32(gaussian(24, (rows, cols)))
+    x[:, 0] = 1 << 20
+    x = x if dtype == "f32" else x.to(torch.bfloat16)
+    s, sh = dev_f32(gaussian(25, (1, cols))), dev_f32(gaussian(26, (1, cols)))
+    want = torch.empty_like(x)
+    hip.layerNormModulate(x, s, sh, 1e-6, want, rows)
+    for per in (rows + 1, 1 << 27, 1 << 40, (1 << 63) - 1):
+        out = torch.full_like(x, 7.0)
+        hip.layerNormModulate(x, s, sh, 1e-6, out, per)
+        assert torch.equal(want, out), f"{per} rows a sample"
+
+
 # rows with an infinity or a NaN are NaN throughout (the mean is no number),
 # and their neighbours as without them: every way AdaLN splits a row, the value
 # first in its row, inside and last
