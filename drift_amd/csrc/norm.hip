@@ -656,11 +656,14 @@ __global__ void __launch_bounds__(256) layer_norm_rows_scalar(const T* x, const 
   }
 }
 
-// F32 AdaLN, one wave per row, B / 64 rows of one sample per block (grid.y =
-// sample), the grid covering the rows in one pass. Each lane reads its chunks' scale and shift
-// from the sample's rows (cached: every row of the sample reads them). Us a
-// launch in graph replays, in 256-thread blocks / in one-wave blocks: [1500,
-// 3840] 14.4 / 9.5, [7800, 3072] 36.9 / 37.6, [8190, 1536] 19.2 / 18.6.
+// F32 AdaLN, one wave per row, four rows of one sample per block (grid.y =
+// sample), the grid covering the rows in one pass. Each lane reads its
+// chunks' scale and shift from the sample's rows (cached: every row of the
+// sample reads them). One-wave blocks spread a sample of few rows over every
+// XCD, each of which fetches its table: us a launch behind a matrix product,
+// one-wave blocks / these: [2000, 3072] of 256 samples 18.5 / 14.0, [4000,
+// 1536] of 1,000 17.9 / 13.4, [7000, 3840] of 1,000 64.0 / 48.0, of one 46.0 /
+// 44.9; [1500, 3840] of one 14.4 / 14.5.
 //
 // The mean and variance come from one pass over the row about its first
 // value x0 (sums of d = x - x0 and d^2): the same as the reference's two
@@ -670,15 +673,15 @@ __global__ void __launch_bounds__(256) layer_norm_rows_scalar(const T* x, const 
 // once, as modulate.
 constexpr int kAdalnMaxCols = 4096;
 
-template <int K, bool FULL, int B>
-__global__ void __launch_bounds__(B) adaln_waves(const float* x, const float* scale, const float* shift, float* out,
-                                                 int64_t rows, int cols, int64_t rows_per_sample, float eps) {
+template <int K, bool FULL>
+__global__ void __launch_bounds__(256) adaln_waves(const float* x, const float* scale, const float* shift, float* out,
+                                                   int64_t rows, int cols, int64_t rows_per_sample, float eps) {
   constexpr int N = 4;
   using Raw = uint4;
   const int chunks = FULL ? K * kWave : cols / N;
   const int64_t sample = blockIdx.y;
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int64_t row = sample * rows_per_sample + (int64_t)blockIdx.x * (B / kWave) + wave;
+  const int64_t row = sample * rows_per_sample + (int64_t)blockIdx.x * 4 + wave;
   if (row >= min(rows, (sample + 1) * rows_per_sample)) return;
   Raw raw[K];
 #pragma unroll
@@ -738,7 +741,11 @@ __global__ void __launch_bounds__(B) adaln_waves(const float* x, const float* sc
 // kept as float: as doubles they would not fit). Measured against adaln_waves
 // in 256-thread blocks, us a launch in graph replays: [300, 3072] 5.0 -> 4.1,
 // [7800, 3072] (192 MB) 36.9 -> 34.9, [16000, 3072] of two samples 70.8 ->
-// 69.5, [8190, 1536] 19.2 -> 18.1; but [1500, 3840] 11.2 against 9.5.
+// 69.5, [8190, 1536] 19.2 -> 18.1; but [1500, 3840] 11.2 against 9.5. In many
+// samples it is slower alone ([8192, 3072] of 64, behind a matrix product 41.8
+// against 45.2, just written 34.9 against 42.3), but a block's convert, AdaLN,
+// gatedAdd, AdaLN, GELU-tanh of those rows is faster with it, 201.9 -> 183.6
+// (of one sample 177.9 -> 171.5).
 template <int K, bool FULL>
 __global__ void __launch_bounds__(kWave) adaln_resident_f32(const float* x, const float* scale, const float* shift,
                                                       float* out, int64_t rows, int cols, int64_t rows_per_sample,
@@ -1242,16 +1249,16 @@ int adaln_launch(const T* x, const float* scale, const float* shift, T* out, int
       DRIFT_ADALN_CASE(12)
 #undef DRIFT_ADALN_CASE
     }
-    const dim3 grid((unsigned)rows_per_sample, (unsigned)samples), block(kWave);
-#define DRIFT_ADALN_CASE(K)                                                                                      \
-  if (per_lane <= K) {                                                                                           \
-    if (chunks == K * kWave)                                                                                     \
-      hipLaunchKernelGGL((adaln_waves<K, true, kWave>), grid, block, 0, s, x, scale, shift, out, rows, cols,  \
-                         rows_per_sample, eps);                                                                  \
-    else                                                                                                         \
-      hipLaunchKernelGGL((adaln_waves<K, false, kWave>), grid, block, 0, s, x, scale, shift, out, rows, cols, \
-                         rows_per_sample, eps);                                                                  \
-    return 0;                                                                                                    \
+    const dim3 grid((unsigned)ceil_div(rows_per_sample, 4), (unsigned)samples);
+#define DRIFT_ADALN_CASE(K)                                                                               \
+  if (per_lane <= K) {                                                                                    \
+    if (chunks == K * kWave)                                                                              \
+      hipLaunchKernelGGL((adaln_waves<K, true>), grid, dim3(256), 0, s, x, scale, shift, out, rows, cols,  \
+                         rows_per_sample, eps);                                                           \
+    else                                                                                                  \
+      hipLaunchKernelGGL((adaln_waves<K, false>), grid, dim3(256), 0, s, x, scale, shift, out, rows, cols, \
+                         rows_per_sample, eps);                                                           \
+    return 0;                                                                                             \
   }
     DRIFT_ADALN_CASE(1)
     DRIFT_ADALN_CASE(2)

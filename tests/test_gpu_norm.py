@@ -291,7 +291,8 @@ def test_layer_norm_modulate(hip, rows, cols, samples, dtype):
     (9000, 772, 2, "f32"), (1030, 3840, 1, "f32"), (1026, 4100, 2, "f32"), (1100, 5120, 1, "f32"), (30, 5116, 2, "f32"),
     (1025, 5120, 3, "bf16"), (1030, 4104, 1, "bf16"), (1024, 5120, 2, "bf16"), (1200, 5128, 1, "bf16"),
     (1536, 4100, 1, "f32"), (1537, 4100, 2, "f32"), (1601, 5116, 5, "f32"), (1537, 5120, 1, "bf16"),
-    (1603, 4104, 3, "bf16"), (1540, 5128, 1, "bf16"),
+    (1603, 4104, 3, "bf16"), (1540, 5128, 1, "bf16"), (1503, 3076, 167, "f32"), (2002, 64, 1001, "f32"),
+    (1101, 1536, 3, "f32"),
 ])
 def test_layer_norm_modulate_row_splits(hip, rows, cols, samples, dtype):
     test_layer_norm_modulate(hip, rows, cols, samples, dtype)
