@@ -528,9 +528,15 @@ __global__ void __launch_bounds__(256) layer_norm_rows(const T* x, const float* 
 // weights and biases are read after the sums: read first, their registers (as
 // doubles) held half as many waves. Measured, us a launch in graph replays,
 // four-wave group / weights first / this: [4087, 1152] (38 MB) 12.6 / 8.9 /
-// 8.4, [4830, 1280] 14.9 / 12.7 / 9.8, [9000, 1024] 19.1 / 18.1 / 15.5; group / this
-// [2000, 2048] 9.2 / 7.9, [1100, 4096] 11.6 / 11.1; but [1100, 1024] 4.0 / 4.7
-// and [600, 1152] 4.2 / 4.5: up to 1,024 rows or 2^19 chunks keep the group.
+// 8.4, [4830, 1280] 14.9 / 12.7 / 9.8, [9000, 1024] 19.1 / 18.1 / 15.5. Up to
+// 2,048 rows or 2^19 chunks the group stays: at two rows a SIMD a row's own
+// chain counts, which replays of one buffer hide. With events around the
+// launch, its input in HBM behind reads / behind a matrix product / just
+// written, group against this: [1100, 3072] 11.0 / 11.0 / 10.5 against 17.6 /
+// 14.0 / 14.5, [1700, 3072] 15.4 / 15.0 / 13.8 against 19.0 / 14.8 / 15.8,
+// [2000, 2560] 15.1 / 15.2 / 14.1 against 17.3 / 14.3 / 14.1, [2300, 2560]
+// 16.8 / 17.6 / 15.3 against 18.1 / 15.0 / 14.6, [3000, 3072] 22.2 / 22.4 /
+// 19.0 against 21.9 / 18.9 / 18.2.
 //
 // MODULATE (as layer_norm_rows): AdaLN rows of 4,097 to 5,120 values, past
 // adaln_launch's, a sample's rows by blockIdx.y, in 256-thread blocks. Us a
@@ -1309,7 +1315,7 @@ int layer_norm(const char* entry, const T* x, const float* weight, const float* 
       return launched(entry);
     }
   } else {
-    if (plan.waves == 4 && rows > kSimds && rows * (cols / 4) >= (1 << 19) && rows <= kOneWaveBlocks &&
+    if (plan.waves == 4 && rows > 2 * kSimds && rows * (cols / 4) >= (1 << 19) && rows <= kOneWaveBlocks &&
         per_lane <= 20) {
       const dim3 one((unsigned)rows), block(kWave);
 #define DRIFT_LN_WAVES(K)                                                                                     \

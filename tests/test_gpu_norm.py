@@ -372,7 +372,8 @@ def test_layer_norm_modulate_of_rows_that_are_not_finite(hip, rows, cols, sample
 
 
 @pytest.mark.parametrize("shape", [(1024, 2052), (2045, 1028), (1300, 2308), (1100, 3072), (1030, 5120), (1050, 5124),
-                                   (1025, 2048), (4100, 1024), (2030, 1028)])
+                                   (1025, 2048), (4100, 1024), (2030, 1028), (2048, 1028), (2049, 1028),
+                                   (2050, 2308), (2049, 5120), (2049, 5124)])
 @pytest.mark.parametrize("affine", [(False, False), (True, False), (False, True), (True, True)])
 def test_layer_norm_row_splits(hip, shape, affine):
     test_layer_norm_f32(hip, shape, affine)
