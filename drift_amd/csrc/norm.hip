@@ -1015,12 +1015,23 @@ int wide_waves(int64_t rows, int cols, const RowPlan& plan) {
 }
 
 // rms_norm_waves for rows of four waves' chunks, where it measured faster than
-// the four-wave group (its comment's figures): alone, from 384 rows (BF16 of
-// more than 8 chunks a lane, from 1025: [600, 6144] 5.5 us in the group, 5.9
-// so); with the residual, from 1025 to 4096 rows of at most 12 chunks a lane,
-// and BF16 rows of at most 10 past the resident line ([9000, 6144] 77.9 in the
-// group, 80.2 so). RESIDENT up to a row a wave (1024 waves: one a SIMD) and
-// from 7 on. Returns false for the others.
+// the four-wave group (its comment's figures): alone, from 384 to 1024 rows
+// (BF16 of at most 8 chunks a lane: [600, 6144] 5.5 us in the group, 5.9 so)
+// and from 1537; with the residual, from 1537 to 4096 rows of at most 12
+// chunks a lane, and BF16 rows of at most 10 past the resident line ([9000,
+// 6144] 77.9 in the group, 80.2 so). RESIDENT up to a row a wave (1024 waves:
+// one a SIMD) and from 7 on. Returns false for the others.
+//
+// From one to one and a half rows a SIMD the second row's chain counts, which
+// replays of one buffer hide. With events around the launch, its input in HBM
+// behind reads / behind a matrix product / just written, group against waves:
+// bf16 [1100, 5120] 10.5 / 10.7 / 10.0 against 13.8 / 11.3 / 11.2, [1500, 5120]
+// 11.3 / 12.2 / 10.8 against 14.6 / 11.9 / 12.3, [1700, 5120] 14.6 / 14.3 /
+// 12.6 against 15.3 / 12.4 / 11.9, [1700, 2560] 10.7 / 10.7 / 9.9 against 9.9 /
+// 8.7 / 8.5; F32 [1100, 2560] 10.7 / 10.8 / 9.4 against 12.7 / 10.7 / 10.3,
+// [1700, 2560] 14.4 / 15.3 / 11.9 against 13.9 / 11.2 / 11.0; bf16 with the
+// residual [1500, 4096] 14.6 / 14.6 / 12.2 against 16.9 / 13.2 / 12.9, [1700,
+// 4096] 18.0 / 18.0 / 13.9 against 17.2 / 13.8 / 13.4.
 template <typename T>
 bool rms_waves_launch(T* x, const T* y, const float* weight, T* out, int64_t rows, int cols, float eps, float offset,
                       hipStream_t s) {
@@ -1028,7 +1039,8 @@ bool rms_waves_launch(T* x, const T* y, const float* weight, T* out, int64_t row
   const bool resident = rows <= kSimds || rows >= 7 * kSimds;
   if (rows < 384 || rows > kOneWaveBlocks || per_lane > (sizeof(T) == 4 ? 20 : 16)) return false;
   if (sizeof(T) == 2 && per_lane > 8 && rows <= kSimds) return false;
-  if (y && (per_lane > 12 || rows <= kSimds)) return false;
+  if (rows <= 3 * kSimds / 2 && (y || !resident)) return false;
+  if (y && per_lane > 12) return false;
   if (y && rows > 4 * kSimds && !(sizeof(T) == 2 && resident && per_lane <= 10)) return false;
   // waves of the resident grid: two a SIMD for BF16 alone, whose output a rope
   // reads next (with ropeTable over [14040, 24, 128] queries and keys 122.7 us

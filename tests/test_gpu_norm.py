@@ -120,7 +120,7 @@ def test_rms_norm_does_not_depend_on_the_batch(hip, dtype, cols):
     assert np.array_equal(host(few).view(np.uint8), host(batch)[100:107].view(np.uint8)), "rows 100-106"
 
 
-# rows on both sides of each line between a row's splits (384, 1,024, 4,096
+# rows on both sides of each line between a row's splits (384, 1,024, 1,536, 4,096
 # and 7,168 rows of four waves' chunks; a last wave's rows part full), lanes
 # past the row's chunks, the most chunks a lane, and rows of at most 64 chunks
 # of one, two and many passes
@@ -129,6 +129,8 @@ def test_rms_norm_does_not_depend_on_the_batch(hip, dtype, cols):
     (1500, 3076, "f32", True), (4097, 1024, "f32", True), (7169, 1024, "f32", False), (400, 5124, "f32", False),
     (1024, 2056, "bf16", False), (1025, 4104, "bf16", False), (4096, 2048, "bf16", True), (4097, 2048, "bf16", True),
     (7168, 2056, "bf16", True), (8193, 2048, "bf16", False), (1100, 10240, "bf16", False),
+    (1536, 2560, "f32", False), (1537, 2564, "f32", False), (1536, 4096, "bf16", True), (1537, 4104, "bf16", True),
+    (1601, 10240, "bf16", False), (1537, 3076, "f32", True),
     (1, 36, "f32", False), (1001, 72, "f32", False), (9001, 256, "f32", False), (70001, 40, "bf16", False),
     (20003, 128, "bf16", False), (9999, 264, "bf16", False), (8193, 512, "bf16", False),
 ])
