@@ -85,7 +85,10 @@ def test_rope_tables_follow_the_configuration(hip):
 
 
 @pytest.mark.parametrize("shape,rotary,layout", [((5, 2, 6), 2, 0), ((4, 3, 10), 6, 1), ((3, 2, 7), 4, 0),
-                                                 ((6, 5, 96), 48, 0), ((2, 1, 512), 512, 1)])
+                                                 ((6, 5, 96), 48, 0), ((2, 1, 512), 512, 1),
+                                                 # more slots than a block's threads, fewer than a head's
+                                                 ((7, 37, 100), 60, 0), ((3, 300, 2), 2, 0), ((2, 5, 511), 510, 1),
+                                                 ((2, 3, 509), 8, 0)])
 def test_rope_odd_shapes_and_in_place(hip, shape, rotary, layout):
     step(f"rope f32 {shape} rotary {rotary} layout {layout}, in place")
     x = gaussian(2, shape, 3.0)
