@@ -467,7 +467,13 @@ constexpr int run_field_align() {
 // 3.6 / 2.9, 7.5 / 7.9, 18.1 / 18.2, 22.1 / 23.1; IQ4_XS 3.2 / 3.0, 8.1 / 7.8,
 // 18.4 / 18.5, 22.7 / 23.6; IQ4_NL 3.4 / 2.8, 7.5 / 7.6, 18.1 / 17.7, 22.2 /
 // 22.4. At [14336, 4096] Q4_0 22.6 / 21.5, Q5_0 29.1 / 23.7, Q5_1 24.6 / 22.8,
-// Q8_0 26.7 / 25.6.
+// Q8_0 26.7 / 25.6. Replays hold the table in the caches; a program's weights
+// lie in HBM, where the lines are drawn: one launch behind a matrix product,
+// runs / by row, Q4_K [1024, 2048] 6.7 / 6.7, [1500, 2048] 6.8 / 7.0, [2001,
+// 2048] 6.9 / 7.8; Q5_K [2001, 2048] 7.2 / 8.1; IQ4_NL [2001, 2048] 7.2 / 7.2,
+// [3000, 2048] 8.4 / 8.7, [2048, 4096] 9.2 / 10.0, [4096, 4096] 12.5 / 14.6,
+// [14336, 4096] 28.9 / 37.5; ROCmFP4 [3000, 2048] 8.4 / 8.7 (just written 8.0 /
+// 7.4), [2048, 4096] 9.2 / 10.3.
 template <typename F>
 struct TakesRuns {
   static constexpr bool kGather = false;
@@ -476,7 +482,7 @@ struct TakesRuns {
 template <bool FIVE>
 struct TakesRuns<QK45<FIVE>> {
   static constexpr bool kGather = true;
-  static constexpr int64_t kWholeFrom = 2048;
+  static constexpr int64_t kWholeFrom = 1024;
 };
 template <>
 struct TakesRuns<Q6_K> {
@@ -491,12 +497,12 @@ struct TakesRuns<IQ4_XS> {
 template <>
 struct TakesRuns<IQ4_NL> {
   static constexpr bool kGather = true;
-  static constexpr int64_t kWholeFrom = INT64_MAX;
+  static constexpr int64_t kWholeFrom = 4096;
 };
 template <>
 struct TakesRuns<RocmFp4<false>> {
   static constexpr bool kGather = true;
-  static constexpr int64_t kWholeFrom = 8192;
+  static constexpr int64_t kWholeFrom = 4096;
 };
 
 template <typename T, typename F>

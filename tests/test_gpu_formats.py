@@ -111,11 +111,14 @@ def test_rows_of_whole_runs(hip, name, cols):
 
 # whole tables decode as one row: rows that fill no block of 256 chunks or run
 # of 2,048 values, a last run part full, enough runs for the run decoder where
-# the format takes it (2,048 for Q4_K and Q5_K, 8,192 for Q6_K and ROCmFP4,
-# 20,480 for IQ4_XS) and one too few, fewer than one
+# the format takes it (1,024 for Q4_K and Q5_K, 4,096 for IQ4_NL and ROCmFP4,
+# 8,192 for Q6_K, 20,480 for IQ4_XS) and one too few, fewer than one
 @pytest.mark.parametrize("name,rows,cols", [(n, 3, 256) for n in NAMES] + [(n, 131, 1280) for n in NAMES] + [
     ("Q5_K", 6555, 1280), ("Q4_K", 13109, 2560), ("IQ4_NL", 6555, 1312), ("Q5_K", 2048, 2048), ("Q4_K", 2047, 2048),
-    ("Q6_K", 13121, 1280), ("Q4_0_ROCMFP4", 13121, 1280), ("IQ4_XS", 32801, 1280), ("Q6_K", 8191, 2048)])
+    ("Q6_K", 13121, 1280), ("Q4_0_ROCMFP4", 13121, 1280), ("IQ4_XS", 32801, 1280), ("Q6_K", 8191, 2048),
+    ("Q4_K", 1024, 2048), ("Q4_K", 1023, 2048), ("Q5_K", 1639, 1280), ("IQ4_NL", 4096, 2048), ("IQ4_NL", 4095, 2048),
+    ("IQ4_NL", 6561, 1312), ("IQ4_NL", 8201, 1024), ("Q4_0_ROCMFP4", 4096, 2048), ("Q4_0_ROCMFP4", 4095, 2048),
+    ("Q4_0_ROCMFP4", 6557, 1280)])
 def test_whole_tables_as_one_row(hip, name, rows, cols):
     raw, table = table_of(name, rows, cols, 101)
     step(f"dequantize {name} -> bf16 [{rows}, {cols}]")
