@@ -543,7 +543,7 @@ __global__ void __launch_bounds__(kWave) qk_norm_rope_wave(const T* q, const T* 
   // keys go last (QK 16.05-16.15 -> 15.72-15.80 us; keys first 16.48-16.54);
   // with it a key wave also places and writes the cache, and goes first
   // (19.45-19.61 against 19.78-19.90 token by token). Blocks number fewer
-  // than 2^31 (the launcher checks): 32-bit division.
+  // than 2^26 (the launcher's rule): 32-bit division.
   const uint32_t tokens = (uint32_t)p.tokens, qw = (uint32_t)query_waves;
   const uint32_t kw = (uint32_t)waves_per_token - qw;  // 0: token by token (qw is every wave)
   const uint32_t first_run = tokens * (keys_first ? kw : qw), first_waves = keys_first ? kw : qw;
@@ -701,13 +701,12 @@ int qk_launch(const char* entry, const T* q, const T* k, T* q_out, T* k_out, con
   const int64_t blocks = (int64_t)p.tokens * waves_per_token + ex.tiles;
   const bool whole = p.rotary > 0 && p.rotary % (p.layout == DRIFT_ROPE_NEOX ? 2 * N : N) == 0 && dim % (2 * N) == 0 &&
                      (lanes_per_head & (lanes_per_head - 1)) == 0 && lanes_per_head <= kWave / 2 && aligned;
-  // the general kernel takes any number of tokens
-  if (!whole || (mixed && blocks > kOneWaveBlocks)) {
+  // the general kernel takes any number of tokens, a launch 2^32 threads
+  if (!whole || blocks > kOneWaveBlocks) {
     hipLaunchKernelGGL((qk_norm_rope_kernel<T, EXTRAS>), dim3(grid_for(p.tokens, 1, 1 << 16)), dim3(256), 0, st, q,
                        k, q_out, k_out, q_weight, k_weight, positions, a, e);
     return launched(entry);
   }
-  if (blocks > INT32_MAX) return refuse("%s: %d tokens of %d heads", entry, p.tokens, a.q_heads + a.kv_heads);
   // a one-wave block per (token, group of 64 / G heads); with the cache,
   // blocks before those write the values by tiles of 16 positions. With the
   // fast body a wave's heads are all queries or all keys, and the grid runs

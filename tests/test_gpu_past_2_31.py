@@ -139,6 +139,30 @@ def test_query_key_norm_rope_in_place(hip):
     assert_bf16(want_k, rows_of(k, check), what="keys")
 
 
+@pytest.mark.parametrize("sections", [d.RopeSections.Single(), d.RopeSections.Axes((4, 4))])
+def test_query_key_norm_rope_past_one_wave_blocks(hip, sections):
+    # a wave a token: more tokens than one-wave blocks fit a launch's 2^32
+    # threads
+    dim, tokens = 16, (1 << 26) + 5
+    check = np.array([0, 1, (1 << 26) - 2, (1 << 26) - 1, 1 << 26, tokens - 1])
+    step(f"queryKeyNormRope bf16 in place over {tokens} tokens of 1 + 1 heads of {dim}, {sections}")
+    q, k = bf16_normal((tokens, 1, dim), 514), bf16_normal((tokens, 1, dim), 515)
+    rng = np.random.default_rng(516)
+    qw = (1 + 0.1 * rng.standard_normal(dim)).astype(np.float32)
+    kw = (1 + 0.1 * rng.standard_normal(dim)).astype(np.float32)
+    norms = d.QueryKeyNorms(dev_f32(qw), dev_f32(kw), 1e-6, 0.0, d.Rope(1e4, dim, d.RopeLayout.Neox, sections))
+    positions = torch.arange(tokens, dtype=torch.int32, device=DEV) % 4099
+    if sections.positionsPerToken > 1:
+        positions = torch.stack((positions, positions // 7)).contiguous()
+    qb, kb = rows_of(q, check), rows_of(k, check)
+    hip.queryKeyNormRope(q, k, norms, positions, q, k)
+    at = positions[..., torch.from_numpy(check).to(DEV)].cpu().numpy()
+    want_q, want_k = o.qk_norm_rope_bf16(qb, kb, qw, kw, at, 1e-6, 0.0, 1e4, dim, sections=sections.code,
+                                         sizes=sections.sizes)
+    assert_bf16(want_q, rows_of(q, check), what="queries")
+    assert_bf16(want_k, rows_of(k, check), what="keys")
+
+
 # dequantize takes a whole table of up to 2^31 - 1 values as one row. Dense
 # tables past 2^31 bytes and past 2^32 (F32 from 2^29 values on, F16 and BF16
 # from 2^30), and one just under 2^31 values; a format decoded by chunks and
