@@ -695,7 +695,7 @@ int qk_launch(const char* entry, const T* q, const T* k, T* q_out, T* k_out, con
   const int waves_per_token = (int)ceil_div(a.q_heads + a.kv_heads, heads_per_wave * passes);
   Extras<T> ex = e;
   const int tile_heads = kTileHeads(kTileWidth(dim));
-  ex.tiles = EXTRAS && e.keys ? ((int64_t)(e.start + p.tokens - 1) / 16 - e.start / 16 + 1) *
+  ex.tiles = EXTRAS && e.keys ? (((int64_t)e.start + p.tokens - 1) / 16 - e.start / 16 + 1) *
                                     ceil_div((int64_t)a.kv_heads * (dim / kTileWidth(dim)), tile_heads)
                               : 0;
   const int64_t blocks = (int64_t)p.tokens * waves_per_token + ex.tiles;

@@ -285,3 +285,32 @@ def test_attention_inputs_partial_rotary_and_sections(hip, dtype, heads, kv, dim
     table = np.random.default_rng(heads).permutation(pages).astype(np.int32)
     rope = d.Rope(1e6, rotary, d.RopeLayout(layout), sections)
     run_attention_inputs(hip, dtype, t, heads, kv, dim, rope, start, table, pages, gated, 200 + heads, offset=1.0)
+
+
+@pytest.mark.parametrize("rotary", [128, 64])
+def test_attention_inputs_across_position_2_31(hip, rotary):
+    # the last cache positions an int32 start can reach, and past them: a page
+    # table of 2^27 entries of which the call reads the last three
+    t, heads, kv, dim, start = 30, 32, 2, 128, (1 << 31) - 21
+    step(f"attentionInputs bf16, positions {start} to {start + t - 1}, rotary {rotary}")
+    first = start // PAGE
+    tail = np.array([2, 0, 1], np.int32)
+    table = torch.full((first + tail.size,), -1, dtype=torch.int32, device=DEV)
+    table[first:] = dev_i32(tail)
+    rng = np.random.default_rng(230)
+    q, k, v = (bf16_input(rng.standard_normal((t, h, dim)).astype(np.float32)) for h in (heads, kv, kv))
+    w = (1 + 0.1 * rng.standard_normal(dim)).astype(np.float32)
+    rope = d.Rope(1e6, rotary, d.RopeLayout.Neox, d.RopeSections.Single())
+    c, keys0, values0 = cache(3, kv, dim, 9)
+    bad = torch.zeros(1, dtype=torch.int32, device=DEV)
+    rq = torch.empty((t, heads, dim), dtype=torch.bfloat16, device=DEV)
+    positions = np.arange(t, dtype=np.int32)
+    hip.queryKeyNormRopeCache(dev_bf16(q), dev_bf16(k), dev_bf16(v), d.QueryKeyNorms(dev_f32(w), dev_f32(w), 1e-6, 0.0, rope),
+                              dev_i32(positions), c, table, start, rq, bad)
+    want_q, want_k = o.qk_norm_rope(o.from_bf16(q), o.from_bf16(k), w, w, positions, 1e-6, 0.0, 1e6, rotary)
+    assert_bf16(o.to_bf16(want_q), host_bits(rq), what="queries")
+    # the same places by positions counted from the first page's start
+    want_keys, want_values = o.cache_write(want_k, o.from_bf16(v), keys0, values0, tail, PAGE, start % PAGE)
+    assert f16_ulps(want_keys, host_bits(c.keys)).max() <= 1, "cached keys"
+    assert_bits(want_values, host_bits(c.values), what="cached values")
+    assert int(bad.item()) == 0
