@@ -53,7 +53,9 @@ def cache(pages, kv, dim, fill_seed):
                                                     # past the line to the value tiles: runs that fill no whole
                                                     # tile, first and last pages cut, one run a token
                                                     (431, 3, 136, 7), (700, 8, 128, 16), (1200, 1, 152, 33),
-                                                    (20501, 1, 8, 3), (650, 5, 56, 15)])
+                                                    (20501, 1, 8, 3), (650, 5, 56, 15),
+                                                    # first and last tiles of 7 and 8 positions, and of 15 and 1
+                                                    (696, 8, 128, 9), (680, 8, 128, 8), (672, 8, 128, 1)])
 def test_cache_write(hip, dtype, tokens, kv, dim, start):
     step(f"cacheWrite {dtype} {tokens} tokens, {kv} heads of {dim}, start {start}")
     pages = -(-(start + tokens) // PAGE) + 1
@@ -314,3 +316,15 @@ def test_attention_inputs_across_position_2_31(hip, rotary):
     assert f16_ulps(want_keys, host_bits(c.keys)).max() <= 1, "cached keys"
     assert_bits(want_values, host_bits(c.values), what="cached values")
     assert int(bad.item()) == 0
+
+
+@pytest.mark.parametrize("dtype", ["f32", "bf16"])
+@pytest.mark.parametrize("t,start", [(1, 15), (7, 5), (8, 5), (7, 9), (8, 8), (15, 0), (15, 1), (23, 9), (31, 1)])
+def test_attention_inputs_cut_tiles(hip, dtype, t, start):
+    # value tiles the tokens cover in part: from one position to 15, at the
+    # tile's start, inside and at its end, heads of one tile and of two
+    step(f"attentionInputs {dtype}, {t} tokens from {start}")
+    table = np.random.default_rng(t).permutation(4).astype(np.int32)
+    for heads, kv, dim in ((32, 3, 128), (16, 2, 256)):
+        rope = d.Rope(1e6, dim, d.RopeLayout.Neox, d.RopeSections.Single())
+        run_attention_inputs(hip, dtype, t, heads, kv, dim, rope, start, table, 4, False, 240 + t)
