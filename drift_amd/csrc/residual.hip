@@ -188,15 +188,23 @@ int row_map(const char* entry, const T* x, const T* y, const float* v, T* out, R
     // measured even (gatedAddChunk) or slower (modulateChunks, 422 against
     // 406 us) that way, and rowGatedAdd's rows do not fit
     const int64_t samples = m.rows / m.per;
-    // gatedAdd's x stays in the caches where most of it fits the 256 MB MALL
-    // until the norm after it reads it again. A block's convert, AdaLN,
-    // gatedAdd, AdaLN, GELU-tanh in graph replays, non-temporal / kept: F32
-    // [7800, 3072] 167.4 / 160.7 us, [16380, 5120] (x 320 MiB) 601.5 / 572.5,
-    // bf16 [8000, 5120] 181.4 / 171.5, [24570, 3072] 289.2 / 279.2, [1000,
-    // 2048] 18.4 / 18.0; at bf16 [65520, 3072] (384 MiB) 751.7 / 749.0, and
-    // gatedAdd alone there 184.8 / 189.2. The other ops' x kept: even or slower
-    // (modulateChunks, gatedAddChunk and rowGatedAdd of [1000, 1536] 12.7 / 14.8).
-    const bool keep = OP == GATED_ADD && values * (int64_t)sizeof(T) <= (int64_t)352 << 20;
+    // gatedAdd's x stays in the caches, from where they gain by it to where
+    // most of it still fits the 256 MB MALL until the norm after it reads it
+    // again. A block's convert, AdaLN, gatedAdd, AdaLN, GELU-tanh behind a
+    // matrix product, non-temporal / kept: F32 [1000, 2048] (8 MiB) 29.6 / 31.4
+    // us, bf16 [2000, 3072] (11) 40.4 / 43.4, [4000, 3072] (23) 63.9 / 62.6, F32
+    // [2000, 3072] (23) 62.7 / 62.4, bf16 [7800, 3072] (45) 106.9 / 105.5, [10500,
+    // 3072] 136.3 / 134.8, F32 [7800, 3072] (91) 170.0 / 163.0, [10500, 3072]
+    // 227.2 / 217.4; in graph replays F32 [16380, 5120] (320) 601.5 / 572.5,
+    // bf16 [65520, 3072] (384) 751.7 / 749.0. Of that gatedAdd and its norm
+    // alone take 94.5 / 88.8 at F32 [9000, 3072]; gatedAdd by itself is even or
+    // up to 8% slower (bf16 [7800, 3072] 26.9 / 29.1, F32 47.1 / 48.0, C5 184.8 /
+    // 189.2). With x loaded non-temporally and only stored through the caches
+    // the pair gained less (bf16 [24570, 3072] 125.3 / 119.3, so 126.1). The
+    // other ops' x kept: even or slower (modulateChunks, gatedAddChunk and
+    // rowGatedAdd of [1000, 1536] 12.7 / 14.8).
+    const int64_t bytes = values * (int64_t)sizeof(T);
+    const bool keep = OP == GATED_ADD && bytes >= (int64_t)20 << 20 && bytes <= (int64_t)352 << 20;
     if (OP == GATED_ADD && m.row_chunks % 64 == 0 && m.row_chunks / 64 <= INT32_MAX && m.per <= 65535 &&
         samples <= 65535 && samples * m.per == m.rows) {
       const dim3 grid((unsigned)(m.row_chunks / 64), (unsigned)m.per, (unsigned)samples);

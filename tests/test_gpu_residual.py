@@ -62,6 +62,14 @@ def test_gated_add(hip, dtype, shape, offset):
     check(dtype, o.gated_add(seen(dtype, x), seen(dtype, y), gate), xd, f"gatedAdd {dtype} {shape}")
 
 
+# either side of the 20 MiB from which x moves through the caches: rows of whole
+# waves' chunks (a row from the grid), and of others
+@pytest.mark.parametrize("dtype,shape", [("f32", (1706, 3072)), ("f32", (1707, 3072)), ("bf16", (3413, 3072)),
+                                         ("bf16", (3414, 3072)), ("f32", (1703, 3080)), ("bf16", (3405, 3080))])
+def test_gated_add_from_the_kept_size(hip, dtype, shape):
+    test_gated_add(hip, dtype, shape, False)
+
+
 @pytest.mark.parametrize("dtype", ["f32", "bf16"])
 @pytest.mark.parametrize("rows,per", [(10, 4), (64, 32), (7, 7)])
 def test_gated_add_per_sample(hip, dtype, rows, per):
