@@ -27,7 +27,10 @@ C-ABI calls those checks produced. The same launches made one by one from
 Python are timed too (`us_eager`), and `host_us_per_call` is the C++ host
 cost of one call of each entry point (drift_amd/host/launch_cost).
 
-Printed: one JSON line. `value` is the step's algorithmic bytes (the reads
+Printed: one JSON line, without the report's long parts (each probe's own
+figures, the kernels' configurations and other times, the CPU baseline's
+samples), so that a reader which keeps a few KB of output has it whole;
+`--report FILE` writes the whole report to FILE. `value` is the step's algorithmic bytes (the reads
 and writes of the tensors each op names) over the step's wall time;
 `kernels` has each kernel's HIP-event times: `us_step`, its K-launch
 replay's span over K in the timed step; `us_replay`, the median over five
@@ -881,6 +884,23 @@ def host_call_cost() -> Optional[dict]:
 
 # ------------------------------------------------------------------ main
 
+BRIEF_KERNEL = ("us", "GB_s", "frac_hbm_peak", "frac_of_ceiling", "frac_of_probe_matched", "rows_per_s")
+
+
+def brief(report: dict) -> dict:
+    """The report's line to print: a few KB."""
+    line = {k: v for k, v in report.items() if k not in ("ceilings", "formats")}
+    line["kernels"] = {name: {k: row[k] for k in BRIEF_KERNEL if k in row} for name, row in report["kernels"].items()}
+    line["graph_start_us"] = report["graph_start_us"]["us"]
+    if "cpu_baseline" in report:
+        line["cpu_baseline"] = dict(report["cpu_baseline"],
+                                    sample=report["cpu_baseline"]["sample"].split(": ")[0])
+    if report["formats"]:
+        line["formats"] = {name: {k: v for k, v in row.items() if isinstance(v, float)}
+                           for name, row in report["formats"].items()}
+    return line
+
+
 def main():
     faulthandler.enable()  # a crash in native code prints the Python stack
     ap = argparse.ArgumentParser(description=__doc__.splitlines()[0])
@@ -896,6 +916,7 @@ def main():
                     help="no long graph: the graph start is not measured, per-kernel us is the K-launch replay's span "
                          "over K (for counter passes: rocprofv3 --pmc has ended in a segmentation fault of its own "
                          "thread in an 80-launch graph)")
+    ap.add_argument("--report", default="", metavar="FILE", help="write the whole report to FILE as JSON")
     ap.add_argument("--no-host", action="store_true",
                     help="skip the host cost per call (a child process that launches kernels of its own: profilers "
                          "tracing this process would trace it too)")
@@ -1113,7 +1134,10 @@ def main():
                             "step_seconds": round(one_core_s, 2)},
             "host": f"{host_cpu()}, {os.cpu_count()} CPUs visible, {host_threads()} used",
         }
-    print(json.dumps(line), flush=True)
+    if args.report:
+        with open(args.report, "w") as f:
+            json.dump(line, f, indent=1)
+    print(json.dumps(brief(line)), flush=True)
 
 
 if __name__ == "__main__":
