@@ -97,7 +97,8 @@ __device__ __forceinline__ void load_codes(const uint8_t* p, uint32_t (&w)[Bytes
 
 // A wave's int8 codes when its 16 groups lie back to back (no ids): 4 KiB
 // from base in four loads of 1 KiB, lane j the j-th 16 bytes of each (plain
-// ones: [13824, 5120] 36.1 us non-temporally, 32.4 so), then through the
+// ones: [13824, 5120] replayed 36.1 us non-temporally, 32.4 so; cached_load has
+// it behind other work), then through the
 // wave's LDS into each lane's own 64 bytes. Every load instruction reads whole 128-byte lines, where a lane
 // loading its own run reads a sixteenth of 32 lines (3.5-4% faster on a
 // [13824, 5120] weight; the 4-bit codes, 2 KiB a wave, measured 2-12%

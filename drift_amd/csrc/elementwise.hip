@@ -256,11 +256,14 @@ __global__ void __launch_bounds__(256) convert_kernel(const void* x, void* out, 
 // in one pass took 192.3 and 30.0, in one-wave blocks 193.3 and 27.6.
 //
 // KEEP: the output is stored through the caches, for the call that reads it
-// next. Alone that is slower (cvt to BF16 of [16380, 3072] 44.8 -> 47.9, to
-// F32 of [7800, 3072] 21.9 -> 25.8), but a block's convert, AdaLN, gatedAdd,
+// next. Replayed alone that is slower (to BF16 of [16380, 3072] 44.8 -> 47.9,
+// to F32 of [7800, 3072] 21.9 -> 25.8), but a block's convert, AdaLN, gatedAdd,
 // AdaLN, GELU-tanh takes 160.1 -> 155.2 at F32 [7800, 3072], 170.1 -> 160.6 at
 // bf16 [8000, 5120], 278.2 -> 270.6 at [24570, 3072]; 753.4 -> 763.0 at
-// [65520, 3072], whose output is past the MALL.
+// [65520, 3072], whose output is past the MALL. Behind a matrix product a
+// convert by itself is even or faster with it (to BF16 of [16380, 5120] 79.3 ->
+// 76.4, of [7800, 3072] 26.2 -> 26.5), and with its AdaLN faster (138.7 -> 131.8,
+// 46.2 -> 44.9).
 template <bool TO_BF16, bool KEEP>
 __global__ void __launch_bounds__(kWave) convert_bf16_waves(const void* x, void* out, int64_t chunks) {
   const int lane = threadIdx.x;

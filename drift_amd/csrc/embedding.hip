@@ -171,8 +171,8 @@ __global__ void __launch_bounds__(256) q8_0_gather(const uint8_t* table, const i
 // one aligned: 19.1-19.3 us against 19.6-19.7 at 8192 random rows of
 // [151936, 4096] (a block per id copying its row to LDS behind a barrier took
 // 20.2-20.3). The loads are plain: a slice's first and last lines are its
-// neighbours' too (4,093 rows of 4096 to bf16 10.8 us non-temporally, 9.0 so;
-// 2,000 of 2560 to F32 7.4, 7.0).
+// neighbours' too (4,093 rows of 4096 to bf16 replayed 10.8 us non-temporally,
+// 9.0 so; 2,000 of 2560 to F32 7.4, 7.0; cached_load has other states).
 template <typename T, int CPL>
 __global__ void __launch_bounds__(256) q8_0_gather_slices(const uint8_t* table, const int32_t* ids, T* out,
                                                           int64_t count, int64_t vocab, int cols, int32_t* bad_id,

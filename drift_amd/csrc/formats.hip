@@ -431,8 +431,8 @@ __global__ void __launch_bounds__(256) decode_staged(const uint8_t* table, const
 // for rows of whole runs on 16-byte boundaries: a one-wave block copies the
 // run's bytes (1,088 to 1,680 for the formats that take it, a multiple of 16)
 // into LDS with 16-byte loads, all in flight together and plain (a run's first
-// and last lines are its neighbours' too: Q4_K [14336, 4096] 26.3 us
-// non-temporally, 23.1 so), then each lane decodes
+// and last lines are its neighbours' too: Q4_K [14336, 4096] replayed 26.3 us
+// non-temporally, 23.1 so; cached_load has other states), then each lane decodes
 // 4 chunks (chunk k * 64 + lane of the run's 256) from there, so each store
 // instruction writes 64 consecutive 16-byte pieces and a block's scales are
 // read from LDS by the lanes that share them.

@@ -178,8 +178,11 @@ __global__ void __launch_bounds__(256) rms_norm_rows(T* x, const T* y, const flo
 // next. RMSNorm and ropeTable (or rope3d) of queries and keys, bf16 [14040,
 // 3072] 122.0 -> 116.2 (125.5 -> 114.4), [12470, 3072] 109.9 -> 104.6; in a
 // dense layer, whose next kernels do not read it, 119.6 -> 131.0 for 4,093
-// tokens of 4096: rows past the resident line, beyond a prompt's chunk, keep
-// it.
+// tokens of 4096. Rows past the resident line keep it, where such a layer is
+// even: behind a matrix product 7,168 tokens of 4096 223.0 -> 221.5, 8,192 249.1
+// -> 250.7, 16,384 480.3 -> 478.8, F32 8,192 of 2560 340.9 -> 344.9 (behind reads
+// 343.0 -> 339.2), and the norm by itself bf16 [8192, 4096] 28.6 -> 26.8, F32
+// 50.7 -> 46.4, bf16 [16384, 4096] 50.7 -> 46.5.
 template <typename T, int K, bool ADD, bool RESIDENT, bool KEEP>
 __global__ void __launch_bounds__(kWave) rms_norm_waves(T* x, const T* y, const float* weight, T* out, int64_t rows,
                                                         int cols, float eps, float offset) {
@@ -961,7 +964,9 @@ __global__ void __launch_bounds__(256) modulate_chunks(const T* x, const float* 
 
 // ------------------------------------------------------------------ launch layer
 
-constexpr int64_t kSimds = 1024;  // 256 CUs of 4
+// MI355X's 256 CUs of 4, which the lines between the splits were measured on
+// (adaln_resident's grid follows its registers and asks the device).
+constexpr int64_t kSimds = 1024;
 
 // How a row is split: W waves per row, K chunks per lane; K = 0 means the
 // scalar path.
@@ -976,10 +981,12 @@ RowPlan plan_rows(int64_t rows, int cols, bool vector_ok) {
   RowPlan plan;
   if (!vector_ok || cols % N != 0) return plan;
   const int chunks = cols / N;
-  // long rows: a 4-wave group per row shortens each lane's chain. The split
-  // depends on the row's width only, never on how many rows come with it, so
-  // a row's sum is taken in the same order (and is the same to the last bit)
-  // whether it is normed alone, as a decode step's token, or in a batch
+  // long rows: a 4-wave group per row shortens each lane's chain. The order
+  // of a row's sums depends on its width only, never on how many rows come
+  // with it (rms_norm_wide, rms_norm_groups, rms_norm_waves and
+  // layer_norm_waves keep this split's order), so a row is the same to the
+  // last bit whether it is normed alone, as a decode step's token, or in a
+  // batch
   plan.waves = chunks >= 4 * kWave ? 4 : 1;
   (void)rows;
   const int per_lane = (int)ceil_div(chunks, kWave * plan.waves);

@@ -79,9 +79,9 @@ RUN_FORMATS = [n for n in NAMES if d.STORAGE_TYPES[n].values > 1]
 @pytest.mark.parametrize("cols", [2048, 6144])
 def test_rows_of_whole_runs(hip, name, cols):
     # rows of whole runs of 2048 values (8 blocks of 256 or 64 of 32), the
-    # table on a 16-byte boundary: the run decoder where the format takes it,
-    # for the gather (with ids outside the table: zero rows and the flag) and
-    # the whole-table decode
+    # table on a 16-byte boundary: the gather's run decoder where the format
+    # takes it (with ids outside the table: zero rows and the flag), and the
+    # whole-table decode of fewer runs than its own takes
     vocab = 19
     raw, table = table_of(name, vocab, cols, 41 + cols)
     assert table.data.data_ptr() % 16 == 0

@@ -285,9 +285,10 @@ def test_layer_norm_modulate(hip, rows, cols, samples, dtype):
         assert_bf16(o.layer_norm_modulate_bf16(xb, s, sh, per, 1e-6), host_bits(out), what="AdaLN bf16")
 
 
-# both sides of the lines between a row's splits (1,024 and 7,168 rows, 4,096
-# and 5,120 values, 12 chunks a lane), rows that fill no whole wave's chunks,
-# samples that share the resident waves unevenly
+# both sides of the lines between a row's splits (1,024 and 7,168 rows, 1,536 of
+# more than 4,096 values, 4,096 and 5,120 values, 12 chunks a lane), rows that
+# fill no whole wave's chunks, samples that share the resident waves unevenly,
+# samples of fewer rows than a block takes
 @pytest.mark.parametrize("rows,cols,samples,dtype", [
     (1024, 1536, 1, "f32"), (1025, 1536, 1, "f32"), (7167, 260, 1, "f32"), (7168, 260, 3, "f32"), (700, 3076, 7, "f32"),
     (9000, 772, 2, "f32"), (1030, 3840, 1, "f32"), (1026, 4100, 2, "f32"), (1100, 5120, 1, "f32"), (30, 5116, 2, "f32"),
