@@ -533,15 +533,17 @@ __global__ void __launch_bounds__(256) layer_norm_rows(const T* x, const float* 
 // weights and biases are read after the sums: read first, their registers (as
 // doubles) held half as many waves. Measured, us a launch in graph replays,
 // four-wave group / weights first / this: [4087, 1152] (38 MB) 12.6 / 8.9 /
-// 8.4, [4830, 1280] 14.9 / 12.7 / 9.8, [9000, 1024] 19.1 / 18.1 / 15.5. Up to
-// 2,048 rows or 2^19 chunks the group stays: at two rows a SIMD a row's own
-// chain counts, which replays of one buffer hide. With events around the
-// launch, its input in HBM behind reads / behind a matrix product / just
-// written, group against this: [1100, 3072] 11.0 / 11.0 / 10.5 against 17.6 /
-// 14.0 / 14.5, [1700, 3072] 15.4 / 15.0 / 13.8 against 19.0 / 14.8 / 15.8,
-// [2000, 2560] 15.1 / 15.2 / 14.1 against 17.3 / 14.3 / 14.1, [2300, 2560]
-// 16.8 / 17.6 / 15.3 against 18.1 / 15.0 / 14.6, [3000, 3072] 22.2 / 22.4 /
-// 19.0 against 21.9 / 18.9 / 18.2.
+// 8.4, [4830, 1280] 14.9 / 12.7 / 9.8, [9000, 1024] 19.1 / 18.1 / 15.5. The
+// group stays up to 2^19 chunks, and up to 1,792 rows of at most 6 chunks a
+// lane and 2,048 of longer ones: at two rows a SIMD a row's own chain counts,
+// which replays of one buffer hide. With events around the launch, its input
+// left by earlier work in the MALL / just written / in HBM, group against this:
+// [1700, 1536] 10.2 against 10.5, even, 14% slower, [1800, 1536] 12.4 against
+// 10.6, 5% and 4% faster; [1100, 3072] 11.0 / 10.5 / 11.0 against 14.0 / 14.5 /
+// 17.6, [1700, 3072] 15.0 / 13.8 / 15.4 against 14.8 / 15.8 / 19.0, [2000, 2560]
+// 15.2 / 14.1 / 15.1 against 14.3 / 14.1 / 17.3, [2300, 2560] 17.6 / 15.3 / 16.8
+// against 15.0 / 14.6 / 18.1, [3000, 3072] 22.4 / 19.0 / 22.2 against 18.9 / 18.2
+// / 21.9.
 //
 // MODULATE (as layer_norm_rows): AdaLN rows of 4,097 to 5,120 values, past
 // adaln_launch's, a sample's rows by blockIdx.y, in 256-thread blocks. Us a
@@ -1024,23 +1026,28 @@ int wide_waves(int64_t rows, int cols, const RowPlan& plan) {
 }
 
 // rms_norm_waves for rows of four waves' chunks, where it measured faster than
-// the four-wave group (its comment's figures): alone, from 384 to 1024 rows
-// (BF16 of at most 8 chunks a lane: [600, 6144] 5.5 us in the group, 5.9 so)
-// and from 1537; with the residual, from 1537 to 4096 rows of at most 12
-// chunks a lane, and BF16 rows of at most 10 past the resident line ([9000,
-// 6144] 77.9 in the group, 80.2 so). RESIDENT up to a row a wave (1024 waves:
-// one a SIMD) and from 7 on. Returns false for the others.
+// the four-wave group (its comment's figures). Alone from 384 to 1024 rows
+// (BF16 of at most 8 chunks a lane: [600, 6144] 5.5 us in the group, 5.9 so),
+// RESIDENT, a row a wave (1024 waves: one a SIMD). Above, from 1281 rows on, or
+// from 1537 if a row is long (BF16 of more than 8 chunks a lane, F32 alone of
+// 11 or 12), or at once (F32 alone of more): RESIDENT from 7 rows a wave. With
+// the residual the same lines, to 4096 rows of at most 12 chunks a lane, and
+// BF16 rows of at most 10 past the resident line ([9000, 6144] 77.9 in the
+// group, 80.2 so). Returns false for the others.
 //
-// From one to one and a half rows a SIMD the second row's chain counts, which
-// replays of one buffer hide. With events around the launch, its input in HBM
-// behind reads / behind a matrix product / just written, group against waves:
-// bf16 [1100, 5120] 10.5 / 10.7 / 10.0 against 13.8 / 11.3 / 11.2, [1500, 5120]
-// 11.3 / 12.2 / 10.8 against 14.6 / 11.9 / 12.3, [1700, 5120] 14.6 / 14.3 /
-// 12.6 against 15.3 / 12.4 / 11.9, [1700, 2560] 10.7 / 10.7 / 9.9 against 9.9 /
-// 8.7 / 8.5; F32 [1100, 2560] 10.7 / 10.8 / 9.4 against 12.7 / 10.7 / 10.3,
-// [1700, 2560] 14.4 / 15.3 / 11.9 against 13.9 / 11.2 / 11.0; bf16 with the
-// residual [1500, 4096] 14.6 / 14.6 / 12.2 against 16.9 / 13.2 / 12.9, [1700,
-// 4096] 18.0 / 18.0 / 13.9 against 17.2 / 13.8 / 13.4.
+// Just past a row a SIMD the second row's chain counts, which replays of one
+// buffer hide. With events around the launch, its input left by earlier work
+// in the MALL / just written / in HBM, group against waves: bf16 [1100, 4096]
+// 10.2 / 8.9 / 10.1 against 9.9 / 9.3 / 11.7, [1350, 4096] 11.1 against 10.3, 3%
+// slower, 12%; [1100, 5120] 10.8 / 10.0 / 10.5 against 11.7 / 11.2 / 13.8,
+// [1536, 5120] 12.5 against 12.4, 5% slower, 31%, [1700, 5120] 14.3 / 12.6 / 14.6
+// against 12.4 / 11.9 / 15.3; with the residual [1200, 4096] 12.6 against 12.3,
+// 10% slower, 25%, [1450, 4096] 14.3 against 12.9, 4%, 16%; F32 [1100, 2560]
+// 11.1 / 9.4 / 10.7 against 10.7 / 10.3 / 12.7, [1350, 2560] 11.8 against 10.8,
+// 6%, 14%, [1281, 3072] 11.7 against 11.9, 12%, 25%, [1100, 4096] 15.2 / 13.0 /
+// 15.4 against 13.4 / 13.0 / 17.9, with the residual [1350, 2560] 14.7 against
+// 13.5, 2% faster, 17% slower. A layer's calls with F32 [1300, 4096] take 87.8
+// us in the group, 86.0 so, [1500, 2560] 69.4 and 67.4.
 template <typename T>
 bool rms_waves_launch(T* x, const T* y, const float* weight, T* out, int64_t rows, int cols, float eps, float offset,
                       hipStream_t s) {
@@ -1048,7 +1055,9 @@ bool rms_waves_launch(T* x, const T* y, const float* weight, T* out, int64_t row
   const bool resident = rows <= kSimds || rows >= 7 * kSimds;
   if (rows < 384 || rows > kOneWaveBlocks || per_lane > (sizeof(T) == 4 ? 20 : 16)) return false;
   if (sizeof(T) == 2 && per_lane > 8 && rows <= kSimds) return false;
-  if (rows <= 3 * kSimds / 2 && (y || !resident)) return false;
+  const bool longer = sizeof(T) == 2 ? per_lane > 8 : !y && per_lane > 10;
+  const int64_t from = sizeof(T) == 4 && per_lane > 12 ? kSimds : longer ? 3 * kSimds / 2 : 5 * kSimds / 4;
+  if (rows <= from && (y || !resident)) return false;
   if (y && per_lane > 12) return false;
   if (y && rows > 4 * kSimds && !(sizeof(T) == 2 && resident && per_lane <= 10)) return false;
   // waves of the resident grid: two a SIMD for BF16 alone, whose output a rope
@@ -1336,7 +1345,8 @@ int layer_norm(const char* entry, const T* x, const float* weight, const float* 
       return launched(entry);
     }
   } else {
-    if (plan.waves == 4 && rows > 2 * kSimds && rows * (cols / 4) >= (1 << 19) && rows <= kOneWaveBlocks &&
+    if (plan.waves == 4 && rows > (per_lane <= 6 ? 7 * kSimds / 4 : 2 * kSimds) &&
+        rows * (cols / 4) >= (1 << 19) && rows <= kOneWaveBlocks &&
         per_lane <= 20) {
       const dim3 one((unsigned)rows), block(kWave);
 #define DRIFT_LN_WAVES(K)                                                                                     \

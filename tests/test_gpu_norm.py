@@ -120,7 +120,7 @@ def test_rms_norm_does_not_depend_on_the_batch(hip, dtype, cols):
     assert np.array_equal(host(few).view(np.uint8), host(batch)[100:107].view(np.uint8)), "rows 100-106"
 
 
-# rows on both sides of each line between a row's splits (384, 1,024, 1,536, 4,096
+# rows on both sides of each line between a row's splits (384, 1,024, 1,280, 1,536, 4,096
 # and 7,168 rows of four waves' chunks; a last wave's rows part full), lanes
 # past the row's chunks, the most chunks a lane, and rows of at most 64 chunks
 # of one, two and many passes
@@ -130,7 +130,9 @@ def test_rms_norm_does_not_depend_on_the_batch(hip, dtype, cols):
     (1024, 2056, "bf16", False), (1025, 4104, "bf16", False), (4096, 2048, "bf16", True), (4097, 2048, "bf16", True),
     (7168, 2056, "bf16", True), (8193, 2048, "bf16", False), (1100, 10240, "bf16", False),
     (1536, 2560, "f32", False), (1537, 2564, "f32", False), (1536, 4096, "bf16", True), (1537, 4104, "bf16", True),
-    (1601, 10240, "bf16", False), (1537, 3076, "f32", True),
+    (1601, 10240, "bf16", False), (1537, 3076, "f32", True), (1280, 2052, "f32", False), (1281, 2052, "f32", False),
+    (1536, 2820, "f32", False), (1537, 2820, "f32", False), (1025, 4100, "f32", False), (1280, 4096, "bf16", False),
+    (1281, 4096, "bf16", False), (1281, 3076, "f32", True), (1281, 2056, "bf16", True),
     (1, 36, "f32", False), (1001, 72, "f32", False), (9001, 256, "f32", False), (70001, 40, "bf16", False),
     (20003, 128, "bf16", False), (9999, 264, "bf16", False), (8193, 512, "bf16", False),
 ])
@@ -376,7 +378,8 @@ def test_layer_norm_modulate_of_rows_that_are_not_finite(hip, rows, cols, sample
 
 @pytest.mark.parametrize("shape", [(1024, 2052), (2045, 1028), (1300, 2308), (1100, 3072), (1030, 5120), (1050, 5124),
                                    (1025, 2048), (4100, 1024), (2030, 1028), (2048, 1028), (2049, 1028),
-                                   (2050, 2308), (2049, 5120), (2049, 5124)])
+                                   (2050, 2308), (2049, 5120), (2049, 5124), (1792, 1536), (1793, 1536),
+                                   (1801, 1284), (1793, 1540)])
 @pytest.mark.parametrize("affine", [(False, False), (True, False), (False, True), (True, True)])
 def test_layer_norm_row_splits(hip, shape, affine):
     test_layer_norm_f32(hip, shape, affine)
